@@ -73,6 +73,24 @@ GPS_HD float det_sqrt_normal(float x) {
     return det_sqrt(x);
 #endif
 }
+// det_sqrt for 0 <= x < 2^64 (either zero gives a zero): the hardware
+// reciprocal root with one residual correction, g = x * y and
+// g + (x - g * g) * (y / 2), is the IEEE-rounded root there.  6 instructions
+// (24 cycles of a SIMD per wave) against det_sqrt_normal's 11 (48): a compare
+// with its select costs as much as four multiplications on gfx950.  Compared
+// with det_sqrt on the GPU for every float in [1, 4) (scaling by 4 commutes)
+// and for every value the sampling radius takes.  The host takes det_sqrt.
+GPS_HD float det_sqrt_radius(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // x = 0: the infinite reciprocal root is cut off, so that g = 0
+    const float y = __builtin_fminf(__builtin_amdgcn_rsqf(__builtin_fabsf(x)), 0x1.0p+100f);
+    const float g = x * y;
+    const float d = __builtin_fmaf(-g, g, x);
+    return __builtin_fmaf(d, 0.5f * y, g);
+#else
+    return det_sqrt(x);
+#endif
+}
 GPS_HD float det_floor(float x) { return __builtin_floorf(x); }
 GPS_HD float det_ceil(float x) { return __builtin_ceilf(x); }
 GPS_HD float det_rint(float x) { return __builtin_rintf(x); }
@@ -103,6 +121,17 @@ GPS_HD int32_t det_f2i_rz(float x) {
     const float c = (x != x) ? 0.0f : glm_min(glm_max(x, -2147483648.0f), 2147483520.0f);
     const int32_t r = (int32_t)c;  // 2147483520 = the largest float below 2^31
     return (x >= 2147483648.0f) ? 2147483647 : r;
+}
+// det_f2i_rz in one instruction on the device: v_cvt_i32_f32 truncates,
+// saturates out-of-range values and converts NaN to 0.
+GPS_HD int32_t det_f2i_sat(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    int32_t r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+#else
+    return det_f2i_rz(x);
+#endif
 }
 GPS_HD int32_t det_f2i_rn(float x) { return det_f2i_rz(det_rint(x)); }
 // det_f2i_rz(v) where only its order against lo and hi matters (the caller
@@ -212,6 +241,28 @@ GPS_HD float det_logf_normal(float x, int32_t e = 0) {
     return det_fma(fe, 0x1.62e400p-1f, det_fma(fe, 0x1.7f7d1cp-20f, logm));
 }
 
+// -2 * det_logf_normal(x), the same bits: the factor is exact in every
+// product and sum that it is carried through, and the exponent's multiple of
+// 2^23 takes 2^-23 into its two constants.  Adding to the bit pattern instead
+// of comparing the mantissa with sqrt(2) gives the same split.
+GPS_HD float det_neg2_logf_normal(float x) {
+    const uint32_t ix = f2u_bits(x);
+    const uint32_t eb = (ix - 0x3F3504F4u) & 0xFF800000u;     // exponent of x / sqrt(2), rounded up to above 1/2
+    const float f = u2f_bits(ix - eb) - 1.0f;                 // m - 1, m in (sqrt(2)/2, sqrt(2)]
+    const float s = det_log_quotient(f);
+    const float z = s * s;
+    float p = 0x1.745d18p-4f;
+    p = det_fma(p, z, 0x1.c71c72p-4f);
+    p = det_fma(p, z, 0x1.24924ap-3f);
+    p = det_fma(p, z, 0x1.99999ap-3f);
+    p = det_fma(p, z, 0x1.555556p-2f);
+    p = p * z;
+    const float t = -4.0f * s;
+    const float l = det_fma(t, p, t);
+    const float fe = (float)(int32_t)eb;                      // e * 2^23, exact
+    return det_fma(fe, -0x1.62e400p-23f, det_fma(fe, -0x1.7f7d1cp-42f, l));
+}
+
 GPS_HD float det_logf(float x) {
     if (x != x) return x;
     if (x < 0.0f) return u2f_bits(0x7FC00000u);
@@ -248,6 +299,38 @@ GPS_HD void det_sincosf_inrange(float x, float* sp, float* cp) {
     const float c = odd ? sr : cr;
     *sp = (q & 2u) ? -s : s;
     *cp = ((q + 1u) & 2u) ? -c : c;
+}
+
+// det_sincosf_inrange(2 pi * (v * 2^-32)) for v a uint32 rounded to float,
+// the same bits (checked for every such v): the scale goes into the
+// constants, the quadrant comes from a rounding addition (v * 2^-30 is exact,
+// and rint of it is the rint that det_sincosf_inrange takes), and selects and
+// sign changes are bit operations, which cost half of a compare or select.
+GPS_HD void det_sincosf_u32(float v, float* sp, float* cp) {
+    const float x = v * 0x1.921fb6p-30f;
+    const float w = det_fma(v, 0x1.0p-30f, 12582912.0f);     // 1.5 * 2^23 + quadrant
+    const float k = w - 12582912.0f;
+    float r = det_fma(-k, 0x1.921fb6p+0f, x);
+    r = det_fma(-k, -0x1.777a5cp-25f, r);
+    r = det_fma(-k, -0x1.000000p-49f, r);
+    const float z = r * r;
+    float ps = 0x1.71de3ap-19f;
+    ps = det_fma(ps, z, -0x1.a01a02p-13f);
+    ps = det_fma(ps, z, 0x1.111112p-7f);
+    ps = det_fma(ps, z, -0x1.555556p-3f);
+    const float sr = det_fma(r * z, ps, r);
+    float pc = -0x1.27e4fcp-22f;
+    pc = det_fma(pc, z, 0x1.a01a02p-16f);
+    pc = det_fma(pc, z, -0x1.6c16c2p-10f);
+    pc = det_fma(pc, z, 0x1.555556p-5f);
+    pc = det_fma(pc, z, -0x1.000000p-1f);
+    const float cr = det_fma(pc, z, 1.0f);
+    const uint32_t q = f2u_bits(w);                           // quadrant in the low two bits
+    const uint32_t odd = (uint32_t)((int32_t)(q << 31) >> 31);
+    const uint32_t swap = (f2u_bits(sr) ^ f2u_bits(cr)) & odd;
+    const uint32_t neg = q << 30;                             // bit 31: quadrants 2 and 3
+    *sp = u2f_bits(f2u_bits(sr) ^ swap ^ (neg & 0x80000000u));
+    *cp = u2f_bits(f2u_bits(cr) ^ swap ^ ((neg ^ odd) & 0x80000000u));
 }
 
 GPS_HD void det_sincosf(float x, float* sp, float* cp) {

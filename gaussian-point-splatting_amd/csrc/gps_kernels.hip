@@ -1204,6 +1204,61 @@ __device__ __forceinline__ uint32_t add_color_sample(unsigned long long* __restr
     return 1u;
 }
 
+// Screen rectangle [x0, x0 + w) x [y0, y0 + h) that a Gaussian's samples may
+// land in.
+struct SampleRect {
+    int x0, y0;
+    uint32_t w, h;
+};
+__device__ __forceinline__ SampleRect record_rect(const SplatRecord& rec) {
+    const int x0 = (int)(rec.bmin & 0xFFFFu), y0 = (int)(rec.bmin >> 16);
+    return SampleRect{x0, y0, (rec.bmax & 0xFFFFu) - (uint32_t)x0, (rec.bmax >> 16) - (uint32_t)y0};
+}
+// One sample of the unbiased splat from an RNG state (splatGaussianPoint,
+// gaussian_point_splatting.cu:67-128): whether it lands in the rectangle and
+// passes the alpha test, and its pixel relative to the rectangle's corner.
+// The pixel conversion saturates and reads NaN as 0, so one unsigned compare
+// per axis is the reference's bounds test; the tests are combined before the
+// one branch, since nearly every sample passes them.
+__device__ __forceinline__ bool sample_pixel(const SplatRecord& rec, u32x2 state, const SampleRect& r, uint32_t& ux,
+                                             uint32_t& uy) {
+    const f32x2 xy = corrected_box_muller_v((float)state.x, (float)state.y, rec.inv_alpha, rec.dilog_alpha);
+    const float fx = det_floor(rec.pmx + rec.c0 * xy.x);
+    const float fy = det_floor((rec.pmy + rec.c1 * xy.x) + rec.c2 * xy.y);
+    ux = (uint32_t)det_f2i_sat(fx) - (uint32_t)r.x0;
+    uy = (uint32_t)det_f2i_sat(fy) - (uint32_t)r.y0;
+    const float dx = rec.pmx - fx, dy = rec.pmy - fy;
+    const float sigma = -0.5f * (rec.conx * dx * dx + rec.conz * dy * dy) - rec.cony * dx * dy;
+    if ((ux >= r.w) | (uy >= r.h) | (sigma < rec.alpha_t - GPS_ALPHA_BAND)) return false;
+    return alpha_passes(rec, sigma);
+}
+
+// The K * spp samples of point p of the biased splat: sample q = layer * K + k
+// lands in layer q / K, and every sample adds (no repeat skip, no word table).
+// Returns the atomics issued.
+__device__ __forceinline__ uint32_t splat_point_biased(const SplatRecord& rec, uint32_t p, uint32_t frame_seed, int K,
+                                                       int spp, int up_w, unsigned long long* __restrict__ fb) {
+    const int bminx = (int)(rec.bmin & 0xFFFFu), bminy = (int)(rec.bmin >> 16);
+    const int bmaxx = (int)(rec.bmax & 0xFFFFu), bmaxy = (int)(rec.bmax >> 16);
+    const unsigned long long packed = ((unsigned long long)rec.packed_hi << 32) | rec.packed_lo;
+    uint32_t issued = 0;
+    u32x2 seed = make_seed(p, frame_seed);
+    for (int layer = 0; layer < spp; ++layer)
+        for (int k = 0; k < K; ++k) {
+            const f32x2 u = pcg2d(seed);
+            const f32x2 xy = box_muller(u.x, u.y);
+            const float fx = det_floor(rec.pmx + rec.c0 * xy.x);
+            const float fy = det_floor((rec.pmy + rec.c1 * xy.x) + rec.c2 * xy.y);
+            int x, y;  // det_f2i_rz(fx), det_f2i_rz(fy) inside the bounds
+            if (!det_pixel_in(fx, bminx, bmaxx, &x) || !det_pixel_in(fy, bminy, bmaxy, &y)) continue;
+            const float dx = rec.pmx - fx, dy = rec.pmy - fy;
+            const float sigma = -0.5f * (rec.conx * dx * dx + rec.conz * dy * dy) - rec.cony * dx * dy;
+            if (!alpha_passes(rec, sigma)) continue;
+            issued += add_color_sample(fb + fb_index(x, y, layer, spp, up_w), packed);
+        }
+    return issued;
+}
+
 // The K * spp samples of point p (seed stream p of RNG frame `frame_seed`)
 // of one Gaussian (splatGaussianPoint, gaussian_point_splatting.cu:67-141):
 // sample q = layer * K + k lands in layer q / K.  Returns the atomics issued.
@@ -1211,8 +1266,8 @@ __device__ __forceinline__ uint32_t splat_point(const SplatRecord& rec, uint32_t
                                                 int spp, int up_w, int unbiased, unsigned long long* __restrict__ fb,
                                                 int& last, uint32_t* s_key = nullptr,
                                                 unsigned long long* s_val = nullptr, uint32_t key_base = 0u) {
-    const int bminx = (int)(rec.bmin & 0xFFFFu), bminy = (int)(rec.bmin >> 16);
-    const int bmaxx = (int)(rec.bmax & 0xFFFFu), bmaxy = (int)(rec.bmax >> 16);
+    if (!unbiased) return splat_point_biased(rec, p, frame_seed, K, spp, up_w, fb);
+    const SampleRect rect = record_rect(rec);
     const unsigned long long packed = ((unsigned long long)rec.packed_hi << 32) | rec.packed_lo;
     const unsigned long long depth_bits = packed & ~(unsigned long long)GPS_COLOR_MASK;
     const int samples = spp * K;
@@ -1224,22 +1279,10 @@ __device__ __forceinline__ uint32_t splat_point(const SplatRecord& rec, uint32_t
             ++layer;
         }
         ++k;
-        const f32x2 u = pcg2d(seed);
-        const f32x2 xy = unbiased ? corrected_box_muller_pre(u.x, u.y, rec.inv_alpha, rec.dilog_alpha)
-                                  : box_muller(u.x, u.y);
-        const float fx = det_floor(rec.pmx + rec.c0 * xy.x);
-        const float fy = det_floor((rec.pmy + rec.c1 * xy.x) + rec.c2 * xy.y);
-        int x, y;  // det_f2i_rz(fx), det_f2i_rz(fy) inside the bounds
-        if (!det_pixel_in(fx, bminx, bmaxx, &x) || !det_pixel_in(fy, bminy, bmaxy, &y)) continue;
-        const float dx = rec.pmx - fx, dy = rec.pmy - fy;
-        const float sigma = -0.5f * (rec.conx * dx * dx + rec.conz * dy * dy) - rec.cony * dx * dy;
-        if (!alpha_passes(rec, sigma)) continue;
-        const int idx = fb_index(x, y, layer, spp, up_w);
-        if (!unbiased) {
-            // every sample adds: no repeat skip, no word table
-            issued += add_color_sample(fb + idx, packed);
-            continue;
-        }
+        seed = pcg2d_uint(seed);
+        uint32_t ux, uy;
+        if (!sample_pixel(rec, seed, rect, ux, uy)) continue;
+        const int idx = fb_index(rect.x0 + (int)ux, rect.y0 + (int)uy, layer, spp, up_w);
         // The word this thread just read or wrote for the same Gaussian
         // (same packed value): a second atomicMin would change nothing.
         if (idx == last) continue;
@@ -1965,8 +2008,7 @@ struct BinSplat {
 // Samples of point p of one Gaussian that land in the LDS region.
 __device__ __forceinline__ void splat_point_region(const SplatRecord& rec, uint32_t p, const BinSplat& b, int rx0,
                                                    int ry0, unsigned long long* s_fb) {
-    const int bminx = (int)(rec.bmin & 0xFFFFu), bminy = (int)(rec.bmin >> 16);
-    const int bmaxx = (int)(rec.bmax & 0xFFFFu), bmaxy = (int)(rec.bmax >> 16);
+    const SampleRect rect = record_rect(rec);
     const unsigned long long packed = ((unsigned long long)rec.packed_hi << 32) | rec.packed_lo;
     const unsigned long long depth_bits = packed & ~(unsigned long long)GPS_COLOR_MASK;
     const int rw = 1 << b.g.rw_shift, rh = 1 << b.g.rh_shift;
@@ -1978,18 +2020,12 @@ __device__ __forceinline__ void splat_point_region(const SplatRecord& rec, uint3
             ++layer;
         }
         ++k;
-        const f32x2 u = pcg2d(seed);
-        const f32x2 xy = b.unbiased ? corrected_box_muller_pre(u.x, u.y, rec.inv_alpha, rec.dilog_alpha)
-                                    : box_muller(u.x, u.y);
-        const float fx = det_floor(rec.pmx + rec.c0 * xy.x);
-        const float fy = det_floor((rec.pmy + rec.c1 * xy.x) + rec.c2 * xy.y);
-        int x, y;  // det_f2i_rz(fx), det_f2i_rz(fy) inside the bounds
-        if (!det_pixel_in(fx, bminx, bmaxx, &x) || !det_pixel_in(fy, bminy, bmaxy, &y)) continue;
+        seed = pcg2d_uint(seed);
+        uint32_t ux, uy;
+        if (!sample_pixel(rec, seed, rect, ux, uy)) continue;
+        const int x = rect.x0 + (int)ux, y = rect.y0 + (int)uy;
         const int lx = x - rx0, ly = y - ry0;
         if ((unsigned)lx >= (unsigned)rw || (unsigned)ly >= (unsigned)rh) continue;  // another region's sample
-        const float dx = rec.pmx - fx, dy = rec.pmy - fy;
-        const float sigma = -0.5f * (rec.conx * dx * dx + rec.conz * dy * dy) - rec.cony * dx * dy;
-        if (!alpha_passes(rec, sigma)) continue;
         const uint32_t t = (uint32_t)((ly >> GPS_TILE_BITS) * b.g.rtx + (lx >> GPS_TILE_BITS));
         const uint32_t i = (t * GPS_TILE_WORDS + morton_encode((uint32_t)(x & (GPS_TILE_SIZE - 1)),
                                                                 (uint32_t)(y & (GPS_TILE_SIZE - 1)))) *

@@ -136,26 +136,38 @@ GPS_HD float inv_dilog_poly(float t) {
 // Polynomial fit of the inverse of Li2 (random.cuh:110-127).
 GPS_HD float inv_dilog(float x) { return inv_dilog_poly(det_fmin(det_div_li2max(x), 1.0f)); }
 
-// Opacity-corrected radial sampling (random.cuh:132-141).  `inv_alpha` is
-// 1/max(alpha, 1e-37) and `dilog_alpha` is dilog(alpha); both depend only on
-// the Gaussian, so callers may compute them once per Gaussian.
-GPS_HD f32x2 corrected_box_muller_pre(float u1, float u2, float inv_alpha, float dilog_alpha) {
-    // (1 - u1) * dilog(alpha) is finite and >= 0, so det_fmin's NaN cases
-    // cannot arise and a compare-select gives its result; a is finite
-    // (inv_alpha <= 1e37), so the clamp is the hardware median of three
-    const float q = det_div_li2max((1.0f - u1) * dilog_alpha);
-    float a = inv_alpha * inv_dilog_poly(1.0f < q ? 1.0f : q);
+// Opacity-corrected radial sampling (random.cuh:132-141) from the two state
+// words as floats, u = v * 2^-32.  `inv_alpha` is 1/max(alpha, 1e-37) and
+// `dilog_alpha` is dilog(alpha); both depend only on the Gaussian, so callers
+// may compute them once per Gaussian.
+//
+// gfx950 runs a wave's fp32 add / multiply / fma and plain bit operations in 2
+// cycles of its SIMD, compares, selects, min / max, conversions and shifts
+// left in 4, reciprocals and roots in 8; the splats spend most of their time
+// here, so the forms below avoid compares and selects (about 180 cycles per
+// sample; 270 with the general functions).  Every step has the bits of the
+// general form:
+//   1 - u1           one fma (u1 = v * 2^-32 is exact)
+//   / Li2(1)         det_div_li2max without its guard: a quotient below
+//                    2^-99 may differ in its last bits, where the polynomial's
+//                    constant term absorbs it; zero gives zero
+//   min(q, 1)        a clamp to [0, 1] (q >= 0)
+//   sqrt(-2 log a)   a is normal and at most 1, so the logarithm is <= 0
+GPS_HD f32x2 corrected_box_muller_v(float v1, float v2, float inv_alpha, float dilog_alpha) {
+    constexpr float z = 1.0f / GPS_LI2_MAX;
+    const float x = det_fma(v1, -0x1.0p-32f, 1.0f) * dilog_alpha;
+    const float q0 = x * z;
+    const float q = det_fma(det_fma(-q0, GPS_LI2_MAX, x), z, q0);
 #if defined(__HIP_DEVICE_COMPILE__)
-    a = __builtin_amdgcn_fmed3f(a, 1.e-37f, 1.0f);
+    float a = inv_alpha * inv_dilog_poly(__builtin_amdgcn_fmed3f(q, 0.0f, 1.0f));
+    a = __builtin_amdgcn_fmed3f(a, 1.e-37f, 1.0f);  // finite (inv_alpha <= 1e37)
 #else
+    float a = inv_alpha * inv_dilog_poly(1.0f < q ? 1.0f : q);
     a = glm_clamp(a, 1.e-37f, 1.0f);
 #endif
-    // a is normal: det_logf needs no special cases
-    // -2 log a is 0 (a = 1) or at least ~1.2e-7 (a <= 1 - 2^-24), at most ~170
-    const float R = det_sqrt_normal(det_fmax(-2.0f * det_logf_normal(a), 0.0f));
-    const float theta = GPS_TWO_PI_F * u2;  // u2 in [0, 1]: in det_sincosf's range
+    const float R = det_sqrt_radius(det_neg2_logf_normal(a));
     float s, c;
-    det_sincosf_inrange(theta, &s, &c);
+    det_sincosf_u32(v2, &s, &c);
     return f32x2{R * c, R * s};
 }
 GPS_HD float corrected_inv_alpha(float alpha) { return 1.0f / det_fmax(alpha, 1.e-37f); }
@@ -182,7 +194,7 @@ GPS_HD bool alpha_test_banded(float opacity, float t, float sigma, float band = 
     return alpha_test(opacity, sigma);
 }
 GPS_HD f32x2 corrected_box_muller(float u1, float u2, float alpha) {
-    return corrected_box_muller_pre(u1, u2, corrected_inv_alpha(alpha), dilog(alpha));
+    return corrected_box_muller_v(u1 * 0x1.0p+32f, u2 * 0x1.0p+32f, corrected_inv_alpha(alpha), dilog(alpha));
 }
 
 // Giles' QN3 normal-asymptotic Poisson sampler, M.B. Giles, "Algorithm 955",
