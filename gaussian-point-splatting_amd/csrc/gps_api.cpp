@@ -86,16 +86,15 @@ struct gps_pass {
     int32_t count_atomics = 0;
     int32_t count_rejects = 0;
     uint32_t cus = 256;
-    uint2* erect = nullptr;
-    uint32_t* ew = nullptr;
-    uint32_t *reg_cnt = nullptr, *reg_pts = nullptr, *reg_ecnt = nullptr, *reg_ptot = nullptr, *reg_eoff = nullptr,
-             *reg_poff = nullptr, *reg_cursor = nullptr, *reg_jobs = nullptr;
+    uint2* bounds = nullptr;  // the records' bounds, written while the frame may be binned
+    unsigned long long* reg_pts = nullptr;
+    uint32_t *reg_ptot = nullptr, *reg_poff = nullptr, *reg_cursor = nullptr;
     uint32_t *job_reg = nullptr, *job_p0 = nullptr;
-    uint32_t *list = nullptr, *lw = nullptr, *lpre = nullptr;
-    uint32_t *tsum = nullptr, *toff = nullptr;
-    uint32_t* big = nullptr;
-    uint32_t* bin_state = nullptr;
-    uint32_t list_cap = 0, job_cap = 0;
+    uint2* list = nullptr;
+    uint2* first_list = nullptr;  // replaced by a longer one when binning was forced
+    uint2* big = nullptr;
+    const uint32_t* bin_state = nullptr;  // of the last binned pass, in ctr
+    uint32_t list_cap = 0, first_list_cap = 0, job_cap = 0;
     int last_binned = 0;
     uint64_t dbg_indices_cap = 0;
     // framebuffers
@@ -194,6 +193,20 @@ gps_status ensure_fb(gps_pass* p, int ss, uint64_t frame_words) {
     p->fb_ss = ss;
     return GPS_OK;
 }
+
+// Points that the binned splat's list holds: the automatic choice bins at most
+// GPS_BIN_DENSE_SAMPLES samples per framebuffer word, i.e. that many points per
+// output pixel (a binned frame's points carry ss^2 samples per layer), or
+// GPS_BIN_DENSE_LARGE in a large framebuffer, which takes millions of Gaussians.
+// Room for the first twice and for the second 1.25 times (Gaussians straddling
+// regions are replayed in each: 1.15 to 1.3 times).
+uint64_t bin_list_points(const gps_render_settings& st, uint64_t N) {
+    const uint64_t px = (uint64_t)st.width * (uint64_t)st.height;
+    const uint64_t most = std::min<uint64_t>(8 * N, px * GPS_BIN_DENSE_LARGE * 5 / 4);
+    return std::min<uint64_t>(std::max<uint64_t>({2 * GPS_BIN_DENSE_SAMPLES * px, 2 * N, most}), 0xFFFFF000ull);
+}
+// ... and room for the whole point budget, up to 2 GiB, once binning is forced.
+uint32_t bin_forced_points(int64_t budget) { return (uint32_t)std::min<int64_t>(2 * std::max<int64_t>(budget, 1 << 20), 1 << 28); }
 
 constexpr int kOcc = 2;
 inline int ev_index(int slot, int stage, int occ, int which) {
@@ -497,26 +510,20 @@ gps_status gps_pass_create(const gps_render_settings* st, gps_scene* scene, gps_
     chk(dalloc(&p->ord_bucket, (uint64_t)p->budget / GPS_SPLAT_CHUNK + 2, false));
     chk(dalloc(&p->ord_hist, GPS_ORD_BINS, true));
     chk(dalloc(&p->ord_lim, GPS_ORD_PHASES, true));
-    // Binned splat lists: up to 2 regions per valid Gaussian on average
-    // (overflow falls back to the point-parallel splat on the device).
+    // Binned splat: its list holds a pass's points once per region they are
+    // replayed in (overflow falls back to the point-parallel splat on the
+    // device).
     {
-        const uint64_t cap = round_up(std::min<uint64_t>(2 * std::max<uint64_t>(N, 1) + 65536, 0xFFFFF000ull), GPS_TILE);
+        const uint64_t cap = bin_list_points(*st, N);
         p->list_cap = (uint32_t)cap;
-        p->job_cap = GPS_BIN_HIST + p->budget / GPS_BIN_JOB_POINTS + 1;
-        chk(dalloc(&p->erect, std::max<uint64_t>(N, 1), false));
-        chk(dalloc(&p->ew, std::max<uint64_t>(N, 1), false));
-        chk(dalloc(&p->big, std::max<uint64_t>(N, 1), false));
-        for (uint32_t** a : {&p->reg_cnt, &p->reg_pts, &p->reg_ecnt, &p->reg_ptot, &p->reg_eoff, &p->reg_poff,
-                             &p->reg_cursor, &p->reg_jobs})
-            chk(dalloc(a, GPS_BIN_HIST, true));
+        p->job_cap = GPS_BIN_HIST + (uint32_t)(std::max<uint64_t>(cap, bin_forced_points(p->budget)) / GPS_BIN_JOB_POINTS) + 1;
+        chk(dalloc(&p->bounds, std::max<uint64_t>(N, 1), false));
+        chk(dalloc(&p->big, N + (uint64_t)p->budget / GPS_BIG_SLICE + 1, false));
+        chk(dalloc(&p->reg_pts, GPS_BIN_HIST, true));
+        for (uint32_t** a : {&p->reg_ptot, &p->reg_poff, &p->reg_cursor}) chk(dalloc(a, GPS_BIN_HIST, false));
         chk(dalloc(&p->job_reg, p->job_cap, false));
         chk(dalloc(&p->job_p0, p->job_cap, false));
         chk(dalloc(&p->list, cap, false));
-        chk(dalloc(&p->lw, cap, true));
-        chk(dalloc(&p->lpre, cap, false));
-        chk(dalloc(&p->tsum, cap / GPS_TILE + 1, false));
-        chk(dalloc(&p->toff, cap / GPS_TILE + 1, false));
-        chk(dalloc(&p->bin_state, 8, true));
     }
     chk(dalloc(&p->ctr, 1, true));
     // Hi-Z pyramid at output resolution, initialised to +inf (nothing occluded).
@@ -588,8 +595,21 @@ gps_status gps_pass_set_ordered_splat(gps_pass* p, int32_t mode) {
 }
 
 gps_status gps_pass_set_splat_mode(gps_pass* p, int32_t mode) {
-    if (!p || (mode != GPS_SPLAT_AUTO && mode != GPS_SPLAT_POINT_PARALLEL && mode != GPS_SPLAT_BINNED))
-        return GPS_ERR_INVALID_ARG;
+    if (!p || mode < GPS_SPLAT_AUTO || mode > GPS_SPLAT_BINNED) return GPS_ERR_INVALID_ARG;
+    // Forced binning takes denser frames than the automatic choice: a longer
+    // list.  The first one stays (a captured frame may write to it).
+    const uint32_t want = bin_forced_points(p->budget);
+    if (mode == GPS_SPLAT_BINNED && p->list_cap < want) {
+        uint2* list = nullptr;
+        if (dalloc(&list, want, false) == GPS_OK) {
+            p->first_list = p->list;
+            p->first_list_cap = p->list_cap;
+            p->list = list;
+            p->list_cap = want;
+        } else {
+            (void)hipGetLastError();  // the list there is serves, up to its length
+        }
+    }
     p->splat_mode = mode;
     return GPS_OK;
 }
@@ -621,9 +641,9 @@ uint64_t gps_pass_estimate_bytes(const gps_render_settings* st, const gps_scene*
     b += (budget / GPS_SPLAT_CHUNK + 2) * 2 + 4ull * (GPS_ORD_BINS + GPS_ORD_PHASES) +
          fb / (256ull * (uint64_t)st->render_pass_count) * 4;  // ordered splat
     {
-        const uint64_t cap = round_up(std::min<uint64_t>(2 * std::max<uint64_t>(N, 1) + 65536, 0xFFFFF000ull), GPS_TILE);
-        b += std::max<uint64_t>(N, 1) * 16 + 3 * cap * 4 + 2 * (cap / GPS_TILE + 1) * 4 + 8ull * 4 * GPS_BIN_HIST +
-             2ull * 4 * (GPS_BIN_HIST + budget / GPS_BIN_JOB_POINTS + 1) + 32;
+        const uint64_t cap = bin_list_points(*st, N);
+        b += std::max<uint64_t>(N, 1) * 8 + (N + budget / GPS_BIG_SLICE + 1) * 8 + cap * 8 + 20ull * GPS_BIN_HIST +
+             2ull * 4 * (GPS_BIN_HIST + std::max<uint64_t>(cap, bin_forced_points((int64_t)budget)) / GPS_BIN_JOB_POINTS + 1) + 32;
     }
     if (!st->fully_disable_hierarchical_culling) {
         const uint64_t gpb = st->gaussians_per_block > 0 ? (uint64_t)st->gaussians_per_block
@@ -653,8 +673,8 @@ uint64_t gps_pass_device_bytes(const gps_pass* p) {
              p->fb_cap / (256ull * (uint64_t)p->settings.render_pass_count) * 4;
     if (p->gboxes) b += (uint64_t)p->group.count * sizeof(GroupBox) + round_up(p->group.count, 4) + 4;
     if (p->live) b += (uint64_t)p->cull.node_count * 4 + (N + GPS_PRE_THREADS - 1) / GPS_PRE_THREADS;
-    b += std::max<uint64_t>(N, 1) * 16 + 3ull * p->list_cap * 4 + 2ull * (p->list_cap / GPS_TILE + 1) * 4 +
-         8ull * 4 * GPS_BIN_HIST + 2ull * 4 * p->job_cap + 32;
+    b += std::max<uint64_t>(N, 1) * 8 + (N + (uint64_t)p->budget / GPS_BIG_SLICE + 1) * 8 +
+         8ull * ((uint64_t)p->list_cap + p->first_list_cap) + 20ull * GPS_BIN_HIST + 2ull * 4 * p->job_cap + 32;
     return b;
 }
 
@@ -687,13 +707,12 @@ void gps_pass_destroy(gps_pass* p) {
     dfree(p->gocc);
     dfree(p->live);
     dfree(p->wg_live);
-    dfree(p->erect);
-    dfree(p->ew);
+    dfree(p->bounds);
     dfree(p->big);
-    for (uint32_t** a : {&p->reg_cnt, &p->reg_pts, &p->reg_ecnt, &p->reg_ptot, &p->reg_eoff, &p->reg_poff,
-                         &p->reg_cursor, &p->reg_jobs, &p->job_reg, &p->job_p0, &p->list, &p->lw, &p->lpre, &p->tsum,
-                         &p->toff, &p->bin_state})
-        dfree(*a);
+    dfree(p->reg_pts);
+    dfree(p->list);
+    dfree(p->first_list);
+    for (uint32_t** a : {&p->reg_ptot, &p->reg_poff, &p->reg_cursor, &p->job_reg, &p->job_p0}) dfree(*a);
     delete p;
 }
 
@@ -790,10 +809,18 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     } else {
         p->timing_slot = -1;
     }
+    BinGeom bg_geom;
+    // the biased splat adds colours per sample and has only the
+    // point-parallel form
+    const bool binned = f.unbiased && p->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
+                        (p->splat_mode == GPS_SPLAT_BINNED || binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, false)) &&
+                        binned_geometry(f.up_w, f.up_h, f.spp, &bg_geom);
     stage_mark(p, 0, 0, 0, st);
     // The clear also resets the per-frame counters (pass results, culled
     // counts, atomics) and keeps the Hi-Z ticket and the mask iteration.
-    launch_clear(p->cur_fb, p->fb_words, bg, st, reinterpret_cast<uint32_t*>(p->ctr), 10, &p->ctr->atomics,
+    // A binned frame's framebuffer is cleared later, as far as it is needed
+    // (bin_clear).
+    launch_clear(p->cur_fb, binned ? 0 : p->fb_words, bg, st, reinterpret_cast<uint32_t*>(p->ctr), 10, &p->ctr->atomics,
                  (uint32_t)((sizeof(FrameCounters) - offsetof(FrameCounters, atomics)) / 4));
     stage_mark(p, 0, 0, 1, st);
 
@@ -838,12 +865,51 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
         a.cull = p->cull;
         a.hiz = p->hiz;
         a.gocc = group_test ? p->gocc : nullptr;
+        // the automatic choice also tests the pass's density on the device
+        const uint32_t dense_points =
+            p->splat_mode == GPS_SPLAT_BINNED ? 0xFFFFFFFFu : binned_dense_points(f.up_w, f.up_h, f.spp, f.Ki, false);
+        a.bounds = binned && (f.occl || 2ull * p->N <= dense_points) ? p->bounds : nullptr;
         if (live_mode) a.wg_live = p->wg_live;
         a.rejects = p->count_rejects ? &p->ctr->rejects[0][0] : nullptr;
         stage_mark(p, 2, slot, 0, st);
         launch_preprocess(a, st);
         stage_mark(p, 2, slot, 1, st);
+        BinnedArgs ba{};
+        if (binned) {
+            ba.recs = p->recs;
+            ba.cidx = p->cidx;
+            ba.coff = p->coff;
+            ba.ctr = &p->ctr->pass[slot];
+            ba.g = bg_geom;
+            ba.sc.spp = f.spp;
+            ba.sc.K = f.Ki;
+            ba.sc.up_w = f.up_w;
+            ba.sc.unbiased = f.unbiased;
+            ba.sc.frame_seed = frame_seed + 1u;
+            ba.sc.xcds = p->xcds;
+            ba.background = bg;
+            ba.fb = p->cur_fb;
+            ba.bounds = a.bounds;
+            ba.fresh = first ? 1 : 0;
+            ba.clear_words = first ? p->fb_words : 0;
+            ba.reg_pts = p->reg_pts;
+            ba.reg_ptot = p->reg_ptot;
+            ba.reg_poff = p->reg_poff;
+            ba.reg_cursor = p->reg_cursor;
+            ba.job_reg = p->job_reg;
+            ba.job_p0 = p->job_p0;
+            ba.list = p->list;
+            ba.big = p->big;
+            ba.state = p->ctr->bin_state[slot];
+            p->bin_state = ba.state;
+            ba.list_cap = p->list_cap;
+            ba.job_cap = p->job_cap;
+            ba.cus = p->cus;
+            ba.dense_points = dense_points;
+            ba.atomics_count = p->count_atomics ? &p->ctr->atomics : nullptr;
+        }
         DistributeArgs da;
+        da.bin = binned ? &ba : nullptr;
         da.tile_sum = p->tile_sum;
         da.tile_cnt = p->tile_cnt;
         da.ntiles = p->ntiles;
@@ -878,59 +944,13 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
         sa.grid = p->splat_grid;
         sa.xcds = p->xcds;
         stage_mark(p, 4, slot, 0, st);
-        BinGeom bg_geom;
-        // the biased splat adds colours per sample and has only the
-        // point-parallel form
-        const bool binned = f.unbiased && p->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
-                            (p->splat_mode == GPS_SPLAT_BINNED || f.Ki * f.spp >= GPS_BIN_AUTO_SAMPLES) &&
-                            binned_geometry(f.up_w, f.up_h, f.spp, &bg_geom);
         p->last_binned = binned ? 1 : 0;
         if (binned) {
-            BinnedArgs ba{};
-            ba.recs = p->recs;
-            ba.cidx = p->cidx;
-            ba.coff = p->coff;
-            ba.ctr = &p->ctr->pass[slot];
-            ba.g = bg_geom;
-            ba.sc.spp = f.spp;
-            ba.sc.K = f.Ki;
-            ba.sc.up_w = f.up_w;
-            ba.sc.unbiased = f.unbiased;
-            ba.sc.frame_seed = frame_seed + 1u;
-            ba.sc.xcds = p->xcds;
-            ba.background = bg;
-            ba.fb = p->cur_fb;
-            ba.erect = p->erect;
-            ba.ew = p->ew;
-            ba.reg_cnt = p->reg_cnt;
-            ba.reg_pts = p->reg_pts;
-            ba.reg_ecnt = p->reg_ecnt;
-            ba.reg_ptot = p->reg_ptot;
-            ba.reg_eoff = p->reg_eoff;
-            ba.reg_poff = p->reg_poff;
-            ba.reg_cursor = p->reg_cursor;
-            ba.reg_jobs = p->reg_jobs;
-            ba.job_reg = p->job_reg;
-            ba.job_p0 = p->job_p0;
-            ba.list = p->list;
-            ba.lw = p->lw;
-            ba.lpre = p->lpre;
-            ba.tsum = p->tsum;
-            ba.toff = p->toff;
-            ba.big = p->big;
-            ba.state = p->bin_state;
-            ba.list_cap = p->list_cap;
-            ba.job_cap = p->job_cap;
-            ba.job_points = GPS_BIN_JOB_POINTS;
-            ba.cus = p->cus;
-            // the automatic choice also tests the pass's density on the device
-            ba.dense_points =
-                p->splat_mode == GPS_SPLAT_BINNED ? 0xFFFFFFFFu : binned_dense_points(f.up_w, f.up_h, f.Ki);
-            ba.atomics_count = p->count_atomics ? &p->ctr->atomics : nullptr;
             launch_binned_splat(ba, st);
-            sa.only_if = p->bin_state + 3;  // stood down: the point-parallel splat takes the pass
-        } else {
-            sa.only_if = nullptr;
+            // the point-parallel splat takes the big Gaussians, or the whole
+            // pass when the binned one stands down
+            sa.bin_state = ba.state;
+            sa.big = ba.big;
         }
         // Dense passes of many-sample points splat point-parallel nearest
         // first and skip Gaussians behind their tiles (the density is decided

@@ -75,6 +75,7 @@ struct gps_batch {
     bool bin_ready = false, bin_failed = false;
     BatchBinArgs bin{};
     uint32_t bin_regions_cap = 0;
+    std::vector<uint2*> old_lists;  // replaced by larger ones (see ensure_list)
     bool use_graph = false;
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
@@ -96,11 +97,11 @@ template <typename T> gps_status balloc(gps_batch* b, T** p, uint64_t count, boo
 
 void free_binned(gps_batch* b) {
     BatchBinArgs& a = b->bin;
-    for (void* p : {(void*)a.erect, (void*)a.ew, (void*)a.big, (void*)a.reg_cnt, (void*)a.reg_pts, (void*)a.reg_ecnt,
-                    (void*)a.reg_ptot, (void*)a.reg_eoff, (void*)a.reg_poff, (void*)a.reg_cursor, (void*)a.reg_jobs,
-                    (void*)a.job_reg, (void*)a.job_p0, (void*)a.list, (void*)a.lw, (void*)a.lpre, (void*)a.tsum,
-                    (void*)a.toff, (void*)a.state})
+    for (void* p : {(void*)a.bounds, (void*)a.big, (void*)a.reg_pts, (void*)a.reg_ptot, (void*)a.reg_poff,
+                    (void*)a.reg_cursor, (void*)a.job_reg, (void*)a.job_p0, (void*)a.list, (void*)a.state})
         if (p) (void)hipFree(p);
+    for (uint2* p : b->old_lists) (void)hipFree(p);
+    b->old_lists.clear();
     a = BatchBinArgs{};
 }
 
@@ -125,28 +126,17 @@ bool ensure_binned(gps_batch* b) {
     }
     BatchBinArgs& a = b->bin;
     const uint64_t regions = V * max_regions;
-    const uint64_t cap = std::min<uint64_t>(entries + entries / 2 + 65536, 0xFFFFF000ull);
-    const uint64_t list_cap = (cap + GPS_TILE - 1) / GPS_TILE * GPS_TILE;
-    a.list_cap = (uint32_t)list_cap;
     a.job_cap = (uint32_t)(regions + (1ull << 32) / GPS_BIN_JOB_POINTS + 1);
-    a.job_points = GPS_BIN_JOB_POINTS;
     gps_status s = GPS_OK;
     auto chk = [&](gps_status r) {
         if (s == GPS_OK) s = r;
     };
-    chk(balloc(b, &a.erect, entries, false));
-    chk(balloc(b, &a.ew, entries, false));
-    chk(balloc(b, &a.big, entries, false));
-    for (uint32_t** p : {&a.reg_cnt, &a.reg_pts, &a.reg_ecnt, &a.reg_ptot, &a.reg_eoff, &a.reg_poff, &a.reg_cursor,
-                         &a.reg_jobs})
-        chk(balloc(b, p, regions, true));
+    chk(balloc(b, &a.bounds, std::max<uint64_t>(V * b->npad, 1), false));  // per record
+    chk(balloc(b, &a.big, entries + (1ull << 32) / GPS_BIG_SLICE, false));
+    chk(balloc(b, &a.reg_pts, regions, true));
+    for (uint32_t** p : {&a.reg_ptot, &a.reg_poff, &a.reg_cursor}) chk(balloc(b, p, regions, false));
     chk(balloc(b, &a.job_reg, a.job_cap, false));
     chk(balloc(b, &a.job_p0, a.job_cap, false));
-    chk(balloc(b, &a.list, list_cap, false));
-    chk(balloc(b, &a.lw, list_cap, true));
-    chk(balloc(b, &a.lpre, list_cap, false));
-    chk(balloc(b, &a.tsum, list_cap / GPS_TILE + 1, false));
-    chk(balloc(b, &a.toff, list_cap / GPS_TILE + 1, false));
     chk(balloc(b, &a.state, 8, true));
     if (s != GPS_OK) {
         free_binned(b);
@@ -165,6 +155,29 @@ void drop_graph(gps_batch* b) {
     b->exec = nullptr;
     b->graph = nullptr;
     b->layout = Layout{};
+}
+
+// The binned views' point list: room for `points`, replaced by one of at
+// least twice the size when a batch needs more.  The replaced lists stay until
+// the batch goes: batches in flight and graphs that a caller captured write to
+// them.  False when it cannot be had: the batch then renders every view
+// point-parallel.
+bool ensure_list(gps_batch* b, uint64_t points) {
+    BatchBinArgs& a = b->bin;
+    constexpr uint64_t kMost = 0xFFFFF000ull;
+    points = std::min<uint64_t>(std::max<uint64_t>(points, 1ull << 21), kMost);
+    if (points <= a.list_cap) return true;
+    drop_graph(b);
+    uint2* list = nullptr;
+    uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(points, 2ull * a.list_cap), kMost);
+    if (balloc(b, &list, cap, false) != GPS_OK) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (a.list) b->old_lists.push_back(a.list);
+    a.list = list;
+    a.list_cap = (uint32_t)cap;
+    return true;
 }
 
 BatchArgs args(gps_batch* b, int nviews) {
@@ -321,7 +334,11 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
     lay.threads = b->threads;
     lay.ppt = b->ppt;
     lay.pre_views = b->pre_views;
-    uint32_t regions = 0, max_view_regions = 0;
+    uint32_t regions = 0, max_view_regions = 0, bin_views = 0;
+    // Room of the binned views' list: their densest binnable points twice, as
+    // a pass's list; at least 2^24 points a view (128 MB), and two per
+    // Gaussian, where forced binning takes denser views too.
+    uint64_t list_points = 0;
     for (int v = 0; v < nviews; ++v) {
         const gps_frame_params& f = views[v];
         const int spp = f.samples_per_pixel > 0 ? f.samples_per_pixel : b->settings.max_spp;
@@ -347,15 +364,22 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
         // (unbiased frames only: the biased splat adds colours per sample).
         BinGeom g;
         if (bv.f.unbiased && b->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
-            (b->splat_mode == GPS_SPLAT_BINNED || bv.f.Ki * bv.f.spp >= GPS_BIN_AUTO_SAMPLES) &&
+            (b->splat_mode == GPS_SPLAT_BINNED || binned_auto(bv.f.up_w, bv.f.up_h, bv.f.spp, bv.f.Ki, b->N, true)) &&
             binned_geometry(bv.f.up_w, bv.f.up_h, bv.f.spp, &g) && ensure_binned(b) &&
             regions + g.nregions <= b->bin_regions_cap) {
             bv.bg = g;
             bv.rbase = regions;
             bv.dense_points =
-                b->splat_mode == GPS_SPLAT_BINNED ? 0xFFFFFFFFu : binned_dense_points(bv.f.up_w, bv.f.up_h, bv.f.Ki);
+                b->splat_mode == GPS_SPLAT_BINNED ? 0xFFFFFFFFu
+                                                   : binned_dense_points(bv.f.up_w, bv.f.up_h, bv.f.spp, bv.f.Ki, true);
+            bv.write_bounds = 2ull * b->N <= bv.dense_points ? 1 : 0;
             regions += g.nregions;
+            ++bin_views;
             max_view_regions = std::max(max_view_regions, g.nregions);
+            const uint64_t px = (uint64_t)f.width * (uint64_t)f.height;
+            const uint64_t dense = std::max<uint64_t>(2 * GPS_BIN_DENSE_SAMPLES * px,
+                                                      std::min<uint64_t>(8ull * b->N, px * GPS_BIN_DENSE_LARGE * 5 / 4));
+            list_points += b->splat_mode == GPS_SPLAT_BINNED ? std::max<uint64_t>({dense, 2ull * b->N, 1ull << 24}) : dense;
         } else {
             bv.rbase = regions;  // bg.nregions == 0: point-parallel
         }
@@ -364,7 +388,16 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
         lay.outs.push_back(colors[v]);
         lay.outs.push_back(depths[v]);
     }
+    if (regions > 0 && !ensure_list(b, list_points)) {
+        for (int v = 0; v < nviews; ++v) {
+            b->h_views[v].bg = BinGeom{};
+            b->h_views[v].rbase = 0;
+            lay.shape[6 * (size_t)v + 5] = 0;
+        }
+        regions = max_view_regions = 0;
+    }
     b->bin.any = regions > 0 ? 1 : 0;
+    b->bin.views = std::max(bin_views, 1u);
     b->bin.nregions = regions;
     b->bin.max_view_regions = max_view_regions;
     b->bin.cus = b->cus;

@@ -35,6 +35,14 @@ GPS_HD uint32_t morton_spread(uint32_t a) {
 }
 GPS_HD uint32_t morton_encode(uint32_t x, uint32_t y) { return morton_spread(x) | (morton_spread(y) << 1); }
 
+// The even bits of a 12-bit Morton code (the inverse of morton_spread).
+GPS_HD uint32_t morton_compact(uint32_t a) {
+    a &= 0x555u;
+    a = (a | (a >> 1)) & 0x333u;
+    a = (a | (a >> 2)) & 0x30Fu;
+    return (a | (a >> 4)) & 0x3Fu;
+}
+
 GPS_HD int32_t fb_tiles_per_row(int32_t width) { return (width + GPS_TILE_SIZE - 1) >> GPS_TILE_BITS; }
 
 // Word index of sample layer `p` of pixel (x, y) in a framebuffer `width`

@@ -109,8 +109,9 @@ struct FrameCounters {
     uint32_t rejects[2][9];  // per pass: preprocess reject reasons (diagnostic; see RejectReason)
     uint32_t group_violations[2];  // per pass, with the reasons: members of culled groups that survived (must be 0)
     uint32_t ordered_skipped[2];   // per pass, with the reasons: points the ordered splat skipped (diagnostic)
+    uint32_t bin_state[2][8];      // per pass: the binned splat's counters (BinnedArgs::state)
 };
-static_assert(sizeof(FrameCounters) == 156, "counter words zeroed by the clear kernel");
+static_assert(sizeof(FrameCounters) == 220, "counter words zeroed by the clear kernel");
 
 // Region geometry of the binned splat for one framebuffer.
 struct BinGeom {
@@ -134,6 +135,7 @@ struct BatchView {
     BinGeom bg;             // binned splat regions (bg.nregions == 0: point-parallel splat)
     uint32_t rbase;         // first region of the view in the batch's region numbering
     uint32_t dense_points;  // more points than this: the view is splatted point-parallel
+    int32_t write_bounds;   // the preprocess writes the view's bounds for the binned lists
     // written on the device
     uint32_t base;          // first point of the view in the batch's point list
     uint32_t points;        // points splatted (min(total, budget))
@@ -185,31 +187,57 @@ static_assert((1u << GPS_SPLAT_CHUNK_SHIFT) == GPS_SPLAT_CHUNK, "chunk is a powe
 #endif
 static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of two");
 // Binned splat: one 1024-thread workgroup renders a screen region of at most
-// GPS_BIN_WORDS framebuffer words in LDS; GPS_BIN_PPT points per thread per
-// step; Gaussians overlapping more regions than GPS_BIN_MAX_REGIONS take the
-// global-atomic path; at most GPS_BIN_HIST regions per frame.
+// GPS_BIN_WORDS framebuffer words in LDS (GPS_BIN_LDS_WORDS with the rows'
+// padding); Gaussians overlapping more regions than GPS_BIN_MAX_REGIONS take
+// the global-atomic path; at most GPS_BIN_HIST regions per frame.
 #define GPS_TILE_WORDS 4096u
 #define GPS_BIN_THREADS 1024
-#define GPS_BIN_PPT 4
-#define GPS_BIN_CHUNK (GPS_BIN_THREADS * GPS_BIN_PPT)
+// Workgroups that list the points per region: they wait on memory, so the more
+// waves the better, also when only some of a batch's views are binned (us, 10M-
+// Gaussian frame / batch of 16 views: 256 threads x 4 workgroups per CU 145 /
+// 1576, 1024 x 2 136 / 970, 1024 x 4 126 / 658, 512 x 8 124 / 617).
+#define GPS_LIST_THREADS 512
+#define GPS_LIST_WGS_PER_CU 8
+#define GPS_LIST_ENTRIES 4096  // entries of one step
 #define GPS_BIN_WORDS 16384u
+#define GPS_BIN_LDS_WORDS 17408u
 #define GPS_BIN_MAX_REGIONS 4u
 #define GPS_BIN_HIST 8192u
-#define GPS_BIN_JOB_POINTS 16384u
+#define GPS_BIN_JOB_POINTS 2048u       // smallest full job (bin_scan_kernel)
+#define GPS_BIN_JOB_POINTS_MAX 32768u
+#define GPS_BIG_SLICE 1024u  // points of a Gaussian too large to bin that one workgroup takes at a time
 // GPS_SPLAT_AUTO bins a frame when a point has >= GPS_BIN_AUTO_SAMPLES
-// samples (K * spp); with fewer the binning launches and the replays of
-// Gaussians that span several regions cost more than the global atomics
-// they save (over the whole 100M fly-through at 1 sample per point: 2.42 ms
-// binned against 1.40 ms point-parallel per frame).
-#define GPS_BIN_AUTO_SAMPLES 8
-// ... and while the pass has at most GPS_BIN_DENSE_SAMPLES samples per
+// samples (K * spp) and at most GPS_BIN_DENSE_SAMPLES samples land on a
 // framebuffer word (points * K <= 8 * up_w * up_h, tested on the device once
-// the point count is known).  Denser frames reject most samples at the
-// point-parallel splat's pre-read, which the binned form cannot skip:
-// 1920x1080 ss 2, 4 spp, K 4 requests measured 0.5-1.05 ms binned vs
-// 0.6-1.9 ms point-parallel at 2.4-4.8 samples per word, 2.44 vs 2.70 at
-// 7.5, 2.17 vs 1.6 at 15, 14.6 vs 9.1 at 250.
+// the point count is known).  Fewer samples per point do not pay for the lists,
+// and denser frames reject most samples at the point-parallel splat's
+// pre-read, which the binned form cannot skip.  A framebuffer of more than
+// GPS_BIN_LARGE_FB words (32 MB) misses the caches, so there both limits are
+// wider: 4 samples per point (given a Gaussian per 16 words, for the launches),
+// and 6 samples per word for every GPS_BIN_LARGE_FB words, up to
+// GPS_BIN_DENSE_LARGE (above that dense frames are splatted nearest first,
+// GPS_ORD_DENSE_SAMPLES).  Whole frames, us, point-parallel / binned, by samples
+// per word:
+//   16 samples a point  33M words 18.7: 6132 / 3945, 3.0: 1551 / 824;
+//                       6.6M words 12.4: 640 / 706; 0.9M words 4.4: 150 / 128
+//   4 samples a point   8.3M words 2.4: 415 / 324, 18.7: 2149 / 2142;
+//                       1.6M words 12.4: 325 / 402, 4.8: 180 / 192
+// A batch shares the lists' launches among its views and has no ordered form:
+// views of more than GPS_BIN_LARGE_FB_BATCH words take the wide limits (batch of
+// 16 views from 1.2M to 33M words, 4 to 13 samples per word: all point-parallel
+// 25.2 ms, views of up to 8 samples per word binned 14.7, all binned 8.7).
+#define GPS_BIN_AUTO_SAMPLES 8
 #define GPS_BIN_DENSE_SAMPLES 8u
+#define GPS_BIN_LARGE_FB (1ull << 22)
+#define GPS_BIN_LARGE_FB_BATCH (1ull << 20)
+#define GPS_BIN_AUTO_SAMPLES_LARGE 4
+#define GPS_BIN_DENSE_LARGE 32u
+// The preprocess writes the records' bounds once more, 8 bytes each, for the
+// binned lists (which otherwise fetch a 64-byte record line for them: 168
+// against 57 us at 7.7M valid Gaussians).  Not in a scene of more than half as
+// many Gaussians as points can be binned, unless occluded ones are culled: a
+// pass over all of it is too dense to bin and would pay for bounds that
+// nothing reads (3519 against 3430 us on a 25M-Gaussian 720p request).
 
 // Ordered point-parallel splat, for dense passes of points with many samples
 // (K * spp >= GPS_BIN_AUTO_SAMPLES, and more than GPS_ORD_DENSE_SAMPLES

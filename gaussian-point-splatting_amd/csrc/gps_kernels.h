@@ -21,10 +21,13 @@ struct PreprocessArgs {
     // one byte per workgroup, 0 when the block cull culled its block (and
     // zeroed its mask words), or null; needs gaussians_per_block a multiple of 256
     const uint8_t* wg_live = nullptr;
+    uint2* bounds = nullptr;      // the records' bounds again, for the binned splat's lists, or null
     uint32_t* rejects = nullptr;  // 2 x 9 reject-reason counters + 2 group checks (diagnostic), or null
 };
 
+struct BinnedArgs;
 struct DistributeArgs {
+    const BinnedArgs* bin = nullptr;  // the pass may be binned: count its regions' points too
     uint32_t* tile_sum;
     uint32_t* tile_cnt;
     uint32_t ntiles;
@@ -54,7 +57,10 @@ struct SplatArgs {
     uint32_t frame_seed;
     uint32_t grid;   // multiple of xcds
     int32_t xcds;    // accelerator complex dies (workgroups round-robin over them)
-    const uint32_t* only_if;  // when set, the splat runs only if *only_if != 0
+    // a pass that may be binned: when the binned splat did not stand down
+    // (bin_state[3] == 0) only its big slices are splatted
+    const uint32_t* bin_state = nullptr;
+    const uint2* big = nullptr;
 };
 
 // Ordered point-parallel splat (dense passes, GPS_ORD_BINS): the splat
@@ -91,41 +97,45 @@ struct BinnedArgs {
     SplatConsts sc;
     uint64_t background;
     uint64_t* fb;
-    uint2* erect;
-    uint32_t* ew;
-    uint32_t *reg_cnt, *reg_pts, *reg_ecnt, *reg_ptot, *reg_eoff, *reg_poff, *reg_cursor, *reg_jobs;
+    int32_t fresh;        // the frame's first pass: the framebuffer holds only the background
+    uint64_t clear_words; // framebuffer words that the lists' kernel still has to clear (0: cleared)
+    const uint2* bounds;  // (bmin, bmax) per record (PreprocessArgs::bounds)
+    unsigned long long* reg_pts;  // points per region, zero between passes
+    uint32_t *reg_ptot, *reg_poff, *reg_cursor;
     uint32_t *job_reg, *job_p0;
-    uint32_t *list, *lw, *lpre;
-    uint32_t *tsum, *toff;
-    uint32_t* big;
-    uint32_t* state;      // 8 words: list length, jobs, big count, stand-down, job cursor, big cursor
-    uint32_t list_cap, job_cap, job_points;
+    uint2* list;          // (record, point) of every point and region, region by region
+    uint2* big;           // (entry, first point) slices of the Gaussians too large to bin
+    uint32_t* state;      // 8 words: (entry, region) pairs, jobs, big Gaussians, stand-down, job cursor, unused,
+                          // slices, points per job
+    uint32_t list_cap, job_cap;
     uint32_t cus;
     uint32_t dense_points;  // more points than this: the binned kernels stand down (state[3] = 2)
     uint32_t* atomics_count;
 };
 bool binned_geometry(int up_w, int up_h, int spp, BinGeom* g);
-// Points above which a frame of up_w x up_h pixels has more than
-// GPS_BIN_DENSE_SAMPLES samples per framebuffer word (a point writes K * spp
-// samples into up_w * up_h * spp words).
-uint32_t binned_dense_points(int up_w, int up_h, int K);
+// Whether the automatic choice may bin a frame of N Gaussians, and the points
+// above which such a frame is too dense to bin, tested on the device
+// (GPS_BIN_AUTO_SAMPLES, GPS_BIN_DENSE_SAMPLES; a point writes K * spp samples
+// into up_w * up_h * spp words).
+bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool batch);
+uint32_t binned_dense_points(int up_w, int up_h, int spp, int K, bool batch);
 void launch_binned_splat(const BinnedArgs& a, hipStream_t st);
 
 // Binned splat buffers of a batch: entries are the batch's compacted entries,
 // regions those of all binned views (view v owns [rbase, rbase + nregions)).
 struct BatchBinArgs {
     int32_t any;                // at least one view is binned
+    uint32_t views;             // views with binned regions
     uint32_t nregions;          // regions of all binned views
     uint32_t max_view_regions;  // largest view's regions (LDS histogram size)
-    uint2* erect;
-    uint32_t* ew;
-    uint32_t* big;
-    uint32_t *reg_cnt, *reg_pts, *reg_ecnt, *reg_ptot, *reg_eoff, *reg_poff, *reg_cursor, *reg_jobs;
+    uint2* bounds;
+    uint2* big;
+    unsigned long long* reg_pts;
+    uint32_t *reg_ptot, *reg_poff, *reg_cursor;
     uint32_t *job_reg, *job_p0;
-    uint32_t *list, *lw, *lpre;
-    uint32_t *tsum, *toff;
+    uint2* list;                // as BinnedArgs::list
     uint32_t* state;            // as BinnedArgs::state
-    uint32_t list_cap, job_cap, job_points;
+    uint32_t list_cap, job_cap;
     uint32_t cus;
 };
 

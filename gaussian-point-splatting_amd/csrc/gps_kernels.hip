@@ -536,11 +536,12 @@ __global__ __launch_bounds__(256) void group_cull_live_kernel(GroupView gv, Cull
 // One Gaussian under one frame (gaussian_point_splatting.cu:147-307, steps 2-11
 // of its cull order): returns the point count, 0 if the Gaussian is not
 // splatted, and writes its 64-byte splat record when the count is > 0.
-// `mask_prev` is read only when f.only_prev is set; `h` only when f.occl.
+// `mask_prev` is read only when f.only_prev is set; `h` only when f.occl.  The
+// record's bounds also go to bounds_out (or null) for the binned splat's lists.
 template <int FORMAT, int DEG>
 __device__ __forceinline__ uint32_t preprocess_one(const DevScene& s, const FrameConsts& f, uint32_t g,
                                                    const uint32_t* __restrict__ mask_prev, const HiZView& h,
-                                                   SplatRecord* __restrict__ rec_out) {
+                                                   SplatRecord* __restrict__ rec_out, uint2* __restrict__ bounds_out) {
     if (f.only_prev && mask_bit(mask_prev, g)) return 0u;
     u32x2 seed = make_seed(g, f.frame_seed);
     const Geo ge = load_geo<FORMAT>(s, g);
@@ -584,6 +585,9 @@ __device__ __forceinline__ uint32_t preprocess_one(const DevScene& s, const Fram
                       (uint32_t)pr.minx | ((uint32_t)pr.miny << 16));
     r[3] = make_uint4((uint32_t)pr.maxx | ((uint32_t)pr.maxy << 16), (uint32_t)packed, (uint32_t)(packed >> 32),
                       __float_as_uint(alpha_threshold(op)));
+    if (bounds_out)
+        *bounds_out = make_uint2((uint32_t)pr.minx | ((uint32_t)pr.miny << 16),
+                                 (uint32_t)pr.maxx | ((uint32_t)pr.maxy << 16));
     return cnt;
 }
 
@@ -691,7 +695,7 @@ __device__ __forceinline__ void preprocess_wg(const DevScene& s, const FrameCons
                                               SplatRecord* __restrict__ recs, uint32_t* __restrict__ tile_sum,
                                               uint32_t* __restrict__ tile_cnt, const CullView& cv, const HiZView& h,
                                               const uint8_t* __restrict__ gocc_bytes, uint32_t* __restrict__ rejects,
-                                              uint32_t g0, bool live) {
+                                              uint32_t g0, bool live, uint2* __restrict__ bounds) {
     __shared__ PreItem s_item[GPS_PRE_THREADS];
     // 15 KB of LDS per workgroup
     __shared__ uint32_t s_count[GPS_PRE_THREADS];
@@ -850,6 +854,7 @@ __device__ __forceinline__ void preprocess_wg(const DevScene& s, const FrameCons
             const uint64_t packed = ((uint64_t)(uint32_t)depth_quantize(q.view_z, f.near_plane, f.far_plane)
                                      << GPS_DEPTH_SHIFT) | pack_color36(rgb[0], rgb[1], rgb[2]);
             r[3] = make_uint4(q.bmax, (uint32_t)packed, (uint32_t)(packed >> 32), __float_as_uint(alpha_threshold(q.op)));
+            if (bounds) bounds[q.g] = make_uint2(q.bmin, q.bmax);
             s_count[q.g - g0] = cnt;
         }
         weights[q.g] = cnt;
@@ -878,14 +883,15 @@ __global__ __launch_bounds__(GPS_PRE_THREADS) void preprocess_kernel(
     DevScene s, FrameConsts f, uint32_t* __restrict__ maskA, uint32_t* __restrict__ maskB,
     const uint32_t* __restrict__ iteration, uint32_t* __restrict__ weights, SplatRecord* __restrict__ recs,
     uint32_t* __restrict__ tile_sum, uint32_t* __restrict__ tile_cnt, CullView cv, HiZView h,
-    const uint8_t* __restrict__ gocc_bytes, uint32_t* __restrict__ rejects, const uint8_t* __restrict__ wg_live) {
+    const uint8_t* __restrict__ gocc_bytes, uint32_t* __restrict__ rejects, const uint8_t* __restrict__ wg_live,
+    uint2* __restrict__ bounds) {
     if (wg_live && wg_live[blockIdx.x] == 0u) return;
     // workload_distributor.cu:32-40: current = A on even iterations.
     const uint32_t it = *iteration;
     uint32_t* mask_cur = (it & 1u) ? maskB : maskA;
     const uint32_t* mask_prev = (it & 1u) ? maskA : maskB;
     preprocess_wg<FORMAT, DEG, STATS>(s, f, mask_cur, mask_prev, weights, recs, tile_sum, tile_cnt, cv, h, gocc_bytes,
-                                      rejects, blockIdx.x * GPS_PRE_THREADS, wg_live != nullptr);
+                                      rejects, blockIdx.x * GPS_PRE_THREADS, wg_live != nullptr, bounds);
 }
 
 // The same outputs with preprocess_one per lane and no work lists: cheaper
@@ -895,7 +901,8 @@ template <int FORMAT, int DEG>
 __global__ __launch_bounds__(GPS_PRE_THREADS) void preprocess_flat_kernel(
     DevScene s, FrameConsts f, uint32_t* __restrict__ maskA, uint32_t* __restrict__ maskB,
     const uint32_t* __restrict__ iteration, uint32_t* __restrict__ weights, SplatRecord* __restrict__ recs,
-    uint32_t* __restrict__ tile_sum, uint32_t* __restrict__ tile_cnt, CullView cv, HiZView h) {
+    uint32_t* __restrict__ tile_sum, uint32_t* __restrict__ tile_cnt, CullView cv, HiZView h,
+    uint2* __restrict__ bounds) {
     const uint32_t g0 = blockIdx.x * GPS_PRE_THREADS;
     const uint32_t g = g0 + threadIdx.x;
     const uint32_t it = *iteration;
@@ -903,7 +910,7 @@ __global__ __launch_bounds__(GPS_PRE_THREADS) void preprocess_flat_kernel(
     const uint32_t* mask_prev = (it & 1u) ? maskA : maskB;
     uint32_t n = 0;
     if (g < s.N && !(f.hier && block_culled(cv, g))) {
-        n = preprocess_one<FORMAT, DEG>(s, f, g, mask_prev, h, recs + g);
+        n = preprocess_one<FORMAT, DEG>(s, f, g, mask_prev, h, recs + g, bounds ? bounds + g : nullptr);
         weights[g] = n;
     }
     preprocess_epilogue(n, g, g0, s.N, mask_cur, tile_sum, tile_cnt);
@@ -1026,6 +1033,55 @@ __global__ __launch_bounds__(1024) void tile_scan_kernel(const uint32_t* __restr
     }
 }
 
+// The compacted entries of one frame: they end at v_end, their points at
+// t_end, the point budget at p_end; the frame's regions start at rbase.
+struct BinFrame {
+    const uint32_t* cidx;
+    const uint32_t* coff;
+    const uint2* bounds;  // (bmin, bmax) per record, or null: read from the records
+    const SplatRecord* recs;
+    BinGeom g;
+    uint32_t v_end, t_end, p_end, rbase;
+};
+// Points of entry r, clipped to the budget.
+__device__ __forceinline__ uint32_t entry_points(const uint32_t* __restrict__ coff, uint32_t r, uint32_t v_end,
+                                                 uint32_t t_end, uint32_t p_end) {
+    const uint32_t lo = coff[r];
+    const uint32_t hi = min(r + 1 < v_end ? coff[r + 1] : t_end, p_end);
+    return lo < hi ? hi - lo : 0u;
+}
+__device__ __forceinline__ uint2 record_bounds(const BinFrame& f, uint32_t rec) {
+    return f.bounds ? f.bounds[rec] : make_uint2(f.recs[rec].bmin, f.recs[rec].bmax);
+}
+// Region rectangle of an entry with bounds b and w points: n regions (0: no
+// point can land).
+struct BinRect {
+    uint32_t rx0, rx1, ry0, ry1, n;
+};
+__device__ __forceinline__ BinRect bounds_rect(const BinGeom& g, uint2 b, uint32_t w) {
+    BinRect q{0u, 0u, 0u, 0u, 0u};
+    const uint32_t bx0 = b.x & 0xFFFFu, by0 = b.x >> 16, bx1 = b.y & 0xFFFFu, by1 = b.y >> 16;
+    if (!w || bx1 <= bx0 || by1 <= by0) return q;  // empty bounds: every sample would be rejected
+    q.rx0 = bx0 >> g.rw_shift;
+    q.rx1 = (bx1 - 1u) >> g.rw_shift;
+    q.ry0 = by0 >> g.rh_shift;
+    q.ry1 = (by1 - 1u) >> g.rh_shift;
+    q.n = (q.rx1 - q.rx0 + 1u) * (q.ry1 - q.ry0 + 1u);
+    return q;
+}
+
+// Counting for the binned splat, done by the distributor while it holds the
+// counts (a kernel of its own read the compacted lists again: 57 us at 7.7M
+// valid Gaussians).  state[0]: (entry, region) pairs.
+struct BinCount {
+    BinFrame f;                   // single frame: g, bounds, recs
+    uint32_t dense_points;        // single frame
+    const BatchView* views;       // batch: the views' own geometry and limits
+    unsigned long long* reg_pts;  // points per region
+    uint2* big;
+    uint32_t* state;
+};
+
 // Per tile of 4096 Gaussians: local exclusive scan of the masked weights, then
 // the compacted (Gaussian id, point offset) lists and the first compacted
 // entry of every splat chunk.  Equivalent to the reference's scatter +
@@ -1040,6 +1096,11 @@ __global__ __launch_bounds__(1024) void tile_scan_kernel(const uint32_t* __restr
 // v * npad + g, its cull mask at cv.mask + v * mask_stride; `cview`, when not
 // null, receives the view of every compacted entry.  Chunks are
 // 2^chunk_shift points.
+//
+// BIN: also the points per screen region of the binned splat, per tile in LDS
+// and then added to the frame's regions (the Morton-ordered tiles touch few
+// regions), and the slices of the Gaussians too large to bin.
+template <bool BIN>
 __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restrict__ weights,
                                                          const uint32_t* __restrict__ tile_off,
                                                          const uint32_t* __restrict__ tile_voff, uint32_t ntiles,
@@ -1048,7 +1109,9 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
                                                          CullView cv, int hier, uint32_t N, uint32_t tiles_per_view,
                                                          uint32_t npad, uint32_t mask_stride,
                                                          uint8_t* __restrict__ cview, uint32_t chunk_shift,
-                                                         uint32_t* __restrict__ tile_sum, uint32_t* __restrict__ tile_cnt) {
+                                                         uint32_t* __restrict__ tile_sum, uint32_t* __restrict__ tile_cnt,
+                                                         BinCount bc) {
+    extern __shared__ uint32_t s_pts[];  // BIN: the regions of the frame, or of the batch's largest view
     __shared__ uint32_t s_a[4], s_c[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t tile = blockIdx.x;
@@ -1090,6 +1153,22 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
             }
             if (c) live &= ~(1u << k);
         }
+    }
+    bool bin = BIN;
+    if (BIN) {
+        if (bc.views) {
+            const BatchView& bv = bc.views[view];
+            bc.f.g = bv.bg;
+            bc.f.rbase = bv.rbase;
+            bc.f.p_end = bv.base + bv.points;
+            if (!bv.write_bounds) bc.f.bounds = nullptr;
+            bin = bv.bg.nregions != 0u && bv.points <= bv.dense_points;
+        } else {
+            bc.f.p_end = (uint32_t)P;
+            bin = P <= bc.dense_points;  // else too dense to bin: bin_scan_kernel stands the binned kernels down
+        }
+        if (bin)
+            for (uint32_t i = (uint32_t)tid; i < bc.f.g.nregions; i += 256u) s_pts[i] = 0u;
     }
     const uint4* wp = reinterpret_cast<const uint4*>(weights + g0);
     // Groups of 4 without a live element re-read the first live group's
@@ -1133,6 +1212,39 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
     }
     uint32_t off = a0 + wa + ia - sa;
     uint32_t r = v0 + wc + ic - sc;
+    if (BIN && bin) {
+        // before the lists are written: one branch over the thread's Gaussians
+        // with all of their bounds requested together
+        uint2 bnd[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) bnd[k] = w[k] ? record_bounds(bc.f, g0 + (uint32_t)k) : make_uint2(0u, 0u);
+        uint32_t o = off, rr = r, pairs = 0u;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            if (!w[k]) continue;
+            const uint32_t hi = min(o + w[k], bc.f.p_end);
+            const uint32_t pts = o < hi ? hi - o : 0u;
+            const BinRect q = bounds_rect(bc.f.g, bnd[k], pts);
+            if (q.n > GPS_BIN_MAX_REGIONS) {
+                // too large to bin: its points in slices (a few hold hundreds
+                // of thousands), which bin_big_kernel takes one by one
+                atomicAdd(&bc.state[2], 1u);
+                const uint32_t slices = (pts + GPS_BIG_SLICE - 1u) / GPS_BIG_SLICE;
+                const uint32_t at = atomicAdd(&bc.state[6], slices);
+                for (uint32_t j = 0; j < slices; ++j) bc.big[at + j] = make_uint2(rr, j * GPS_BIG_SLICE);
+            } else if (q.n) {
+                pairs += q.n;
+                for (uint32_t ry = q.ry0; ry <= q.ry1; ++ry)
+                    for (uint32_t rx = q.rx0; rx <= q.rx1; ++rx)
+                        atomicAdd(&s_pts[ry * (uint32_t)bc.f.g.nrx + rx], pts);
+            }
+            o += w[k];
+            ++rr;
+        }
+        add_count(&bc.state[0], pairs);  // (its barriers order the histogram too)
+        for (uint32_t i = (uint32_t)tid; i < bc.f.g.nregions; i += 256u)
+            if (s_pts[i]) atomicAdd(&bc.reg_pts[bc.f.rbase + i], (unsigned long long)s_pts[i]);
+    }
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         if (w[k]) {
@@ -1464,6 +1576,31 @@ __device__ __forceinline__ uint32_t splat_chunk(uint32_t c, const SplatRecord* _
     return issued;
 }
 
+// Gaussians too large to bin (the distributor's slices): their points with
+// global atomics, by the kernel that follows the binned splat and would take the
+// whole pass had it stood down.
+struct BigSlices {
+    const uint2* big;
+    const uint32_t* state;  // null: the pass is not binned
+};
+__device__ __forceinline__ uint32_t splat_big(const BigSlices& b, const SplatRecord* __restrict__ recs,
+                                              const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ coff,
+                                              const PassCounters* __restrict__ ctr, const SplatConsts& sc,
+                                              unsigned long long* __restrict__ fb) {
+    const uint32_t n = b.state[6];
+    uint32_t issued = 0;
+    for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
+        const uint2 it = b.big[e];
+        const SplatRecord rec = load_record(recs, cidx[it.x]);
+        const uint32_t p0 = coff[it.x];
+        const uint32_t w = min(entry_points(coff, it.x, ctr->valid, ctr->total, ctr->points), it.y + GPS_BIG_SLICE);
+        int last = -1;  // one Gaussian throughout
+        for (uint32_t k = it.y + threadIdx.x; k < w; k += blockDim.x)
+            issued += splat_point(rec, p0 + k, sc.frame_seed, sc.K, sc.spp, sc.up_w, 1, fb, last);
+    }
+    return issued;
+}
+
 __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_kernel(const SplatRecord* __restrict__ recs,
                                                                   const uint32_t* __restrict__ cidx,
                                                                   const uint32_t* __restrict__ coff,
@@ -1471,7 +1608,7 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_kernel(const SplatRec
                                                                   const PassCounters* __restrict__ ctr,
                                                                   unsigned long long* __restrict__ fb, SplatConsts sc,
                                                                   uint32_t* __restrict__ atomics_count,
-                                                                  const uint32_t* __restrict__ only_if) {
+                                                                  BigSlices big) {
     __shared__ uint32_t s_off[GPS_SPLAT_CHUNK + 1];
 #if GPS_SPLAT_SLOTS
     __shared__ uint32_t s_key[GPS_SPLAT_SLOTS];
@@ -1480,7 +1617,11 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_kernel(const SplatRec
     uint32_t* const s_key = nullptr;
     unsigned long long* const s_val = nullptr;
 #endif
-    if (only_if && *only_if == 0u) return;  // the binned splat covers this pass
+    if (big.state && big.state[3] == 0u) {  // the binned splat covers this pass
+        const uint32_t n = splat_big(big, recs, cidx, coff, ctr, sc, fb);
+        if (atomics_count) add_count(atomics_count, n);
+        return;
+    }
     const uint32_t P = ctr->points;
     const uint32_t V = ctr->valid;
     const uint32_t nchunks = ctr->chunks;
@@ -1625,7 +1766,7 @@ __global__ __launch_bounds__(256) void ord_tile_max_kernel(const unsigned long l
 __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_ordered_kernel(
     const SplatRecord* __restrict__ recs, const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ coff,
     const uint32_t* __restrict__ chunk_start, const PassCounters* __restrict__ ctr, unsigned long long* __restrict__ fb,
-    SplatConsts sc, uint32_t* __restrict__ atomics_count, const uint32_t* __restrict__ only_if,
+    SplatConsts sc, uint32_t* __restrict__ atomics_count, BigSlices big,
     const uint16_t* __restrict__ bucket, const uint32_t* __restrict__ lim, const uint32_t* __restrict__ tmax,
     int tw64, int phase, int test, OrdGate gate, uint32_t* __restrict__ skipped_count) {
     __shared__ uint32_t s_off[GPS_SPLAT_CHUNK + 1];
@@ -1636,7 +1777,12 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_ordered_kernel(
     uint32_t* const s_key = nullptr;
     unsigned long long* const s_val = nullptr;
 #endif
-    if (only_if && *only_if == 0u) return;
+    if (big.state && big.state[3] == 0u) {  // the binned splat covers this pass
+        if (phase > 0) return;
+        const uint32_t n = splat_big(big, recs, cidx, coff, ctr, sc, fb);
+        if (atomics_count) add_count(atomics_count, n);
+        return;
+    }
     const bool active = ord_active(ctr, gate);
     if (!active && phase > 0) return;
     const uint32_t P = ctr->points;
@@ -1679,457 +1825,366 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_ordered_kernel(
 }
 
 // ------------------------------------------------------------------ binned splat
-// Screen regions of at most GPS_BIN_WORDS framebuffer words (128x128 px at
-// 1 spp, 128x64 at 2, 64x64 at 3-4) are rendered by one workgroup in LDS.
-// The valid Gaussians are binned to the regions their bounds overlap; a
-// region job replays the points of its Gaussians with their global point
-// index (hence exactly the samples of the point-parallel splat) and keeps
-// the samples that land inside the region, with LDS atomicMin.  A region
-// rendered by one job starts from the framebuffer and stores the region
-// back; a heavy region split into several jobs merges its changed words with
-// global atomicMin.  Gaussians overlapping more than GPS_BIN_MAX_REGIONS
-// regions are splatted afterwards with global atomics (no replay).  Since
-// min is order-independent the framebuffer is bit-identical to the
-// point-parallel splat.  If the region lists overflow their allocation
+// Screen regions of GPS_BIN_WORDS framebuffer words (128x128 px at 1 spp,
+// 128x64 at 2, 64x64 at 3-4) are rendered by one workgroup in LDS.  The
+// points of the valid Gaussians are listed per region that their Gaussian's
+// bounds overlap (8 bytes each: record index, point index in the frame); a
+// region job replays its points with their global point index (hence exactly
+// the samples of the point-parallel splat) and keeps the samples that land
+// inside the region, with LDS atomicMin.  A region rendered by one job is
+// stored whole; a heavy region split into several jobs merges its changed
+// words with global atomicMin.  Gaussians overlapping more than
+// GPS_BIN_MAX_REGIONS regions are splatted afterwards with global atomics (no
+// replay).  Since min is order-independent the framebuffer is bit-identical
+// to the point-parallel splat.  If the list overflows its allocation
 // (state[3] = 1), or the pass has more points than dense_points (state[3] = 2,
 // the automatic choice's density test), the binned kernels stand down and the
 // point-parallel splat runs instead.
 
-__device__ __forceinline__ uint32_t bin_region_words(const BinGeom& g) {
-    return (uint32_t)(g.rtx * g.rty) * GPS_TILE_WORDS * (uint32_t)g.spp;
-}
-
-// Entries [r0, r1) of one frame whose entries end at v_end, whose points end
-// at t_end and whose point budget ends at p_end: points per entry (clipped to
-// the budget), region rectangle, region histogram in LDS (a workgroup takes
-// one contiguous entry range, so the Morton-ordered entries touch few
-// regions), big entries to their list.  The histogram is added to the
-// frame's regions, which start at rbase.
-__device__ __forceinline__ void bin_count_range(const SplatRecord* __restrict__ recs, const uint32_t* __restrict__ cidx,
-                                                const uint32_t* __restrict__ coff, const BinGeom& g, uint32_t r0,
-                                                uint32_t r1, uint32_t v_end, uint32_t t_end, uint32_t p_end,
-                                                uint32_t rbase, uint2* __restrict__ erect, uint32_t* __restrict__ ew,
-                                                uint32_t* __restrict__ reg_cnt, uint32_t* __restrict__ reg_pts,
-                                                uint32_t* __restrict__ big, uint32_t* __restrict__ state,
-                                                uint32_t* s_cnt, uint32_t* s_pts) {
-    const int tid = threadIdx.x;
-    for (uint32_t i = tid; i < g.nregions; i += 256) {
-        s_cnt[i] = 0u;
-        s_pts[i] = 0u;
-    }
-    __syncthreads();
-    for (uint32_t r = r0 + tid; r < r1; r += 256) {
-        const uint32_t lo = coff[r];
-        const uint32_t hi = min(r + 1 < v_end ? coff[r + 1] : t_end, p_end);
-        uint32_t w = lo < hi ? hi - lo : 0u;
-        uint2 rect = make_uint2(0xFFFFFFFFu, 0u);
-        if (w) {
-            const uint32_t* rp = reinterpret_cast<const uint32_t*>(recs + cidx[r]);
-            const uint32_t bmin = rp[11], bmax = rp[12];
-            const uint32_t bx0 = bmin & 0xFFFFu, by0 = bmin >> 16, bx1 = bmax & 0xFFFFu, by1 = bmax >> 16;
-            if (bx1 > bx0 && by1 > by0) {
-                const uint32_t rx0 = bx0 >> g.rw_shift, rx1 = (bx1 - 1u) >> g.rw_shift;
-                const uint32_t ry0 = by0 >> g.rh_shift, ry1 = (by1 - 1u) >> g.rh_shift;
-                if ((rx1 - rx0 + 1u) * (ry1 - ry0 + 1u) > GPS_BIN_MAX_REGIONS) {
-                    big[atomicAdd(&state[2], 1u)] = r;
-                } else {
-                    rect = make_uint2(rx0 | (rx1 << 16), ry0 | (ry1 << 16));
-                    for (uint32_t ry = ry0; ry <= ry1; ++ry)
-                        for (uint32_t rx = rx0; rx <= rx1; ++rx) {
-                            const uint32_t reg = ry * (uint32_t)g.nrx + rx;
-                            atomicAdd(&s_cnt[reg], 1u);
-                            atomicAdd(&s_pts[reg], w);
-                        }
-                }
-            } else {
-                w = 0u;  // empty bounds: every sample would be rejected
-            }
-        }
-        erect[r] = rect;
-        ew[r] = w;
-    }
-    __syncthreads();
-    for (uint32_t i = tid; i < g.nregions; i += 256)
-        if (s_cnt[i]) {
-            atomicAdd(&reg_cnt[rbase + i], s_cnt[i]);
-            atomicAdd(&reg_pts[rbase + i], s_pts[i]);
-        }
-}
-
-__global__ __launch_bounds__(256) void bin_count_kernel(const SplatRecord* __restrict__ recs,
-                                                        const uint32_t* __restrict__ cidx,
-                                                        const uint32_t* __restrict__ coff,
-                                                        const PassCounters* __restrict__ ctr, BinGeom g,
-                                                        uint2* __restrict__ erect, uint32_t* __restrict__ ew,
-                                                        uint32_t* __restrict__ reg_cnt, uint32_t* __restrict__ reg_pts,
-                                                        uint32_t* __restrict__ big, uint32_t* __restrict__ state,
-                                                        uint32_t dense_points) {
-    extern __shared__ uint32_t s_dyn[];  // 2 * nregions words
-    const uint32_t V = ctr->valid, P = ctr->points, T = ctr->total;
-    if (P > dense_points) return;  // too dense to bin: bin_scan_kernel stands the binned kernels down
-    const uint32_t per = (V + gridDim.x - 1) / gridDim.x;
-    const uint32_t r0 = min(V, blockIdx.x * per), r1 = min(V, r0 + per);
-    bin_count_range(recs, cidx, coff, g, r0, r1, V, T, P, 0u, erect, ew, reg_cnt, reg_pts, big, state, s_dyn,
-                    s_dyn + g.nregions);
-}
-// One workgroup: region offsets, jobs of at most `job_points` points per
-// region, the job table, and the list length (overflow flag).  Clears the
-// region counters for the next pass.
-__global__ __launch_bounds__(1024) void bin_scan_kernel(BinGeom g, uint32_t* __restrict__ reg_cnt,
-                                                        uint32_t* __restrict__ reg_pts,
-                                                        uint32_t* __restrict__ reg_ecnt,
+// One workgroup: the regions' list offsets, and the job table: jobs of at most
+// state[7] points, the largest first (eight size classes), so that the
+// persistent splat does not end on a long one.  Large jobs start and store
+// fewer regions twice, small ones share out evenly: a little more than one a CU
+// between GPS_BIN_JOB_POINTS and 32768 points (splat, us, at 8192 / 16384 /
+// 32768 / 65536: 5M listed points 212 / 193 / 229 / 421, 20M 1120 / 1065 /
+// 1026 / 1039, 44M 2296 / 2201 / 2174 / 2287; whole frame at 0.3M, where 16384
+// leaves three CUs of four idle: 273 against 128 at 2048).  Clears the region
+// counters for the next pass.
+__global__ __launch_bounds__(1024) void bin_scan_kernel(uint32_t nregions, unsigned long long* __restrict__ reg_pts,
                                                         uint32_t* __restrict__ reg_ptot,
-                                                        uint32_t* __restrict__ reg_eoff,
                                                         uint32_t* __restrict__ reg_poff,
                                                         uint32_t* __restrict__ reg_cursor,
-                                                        uint32_t* __restrict__ reg_jobs,
                                                         uint32_t* __restrict__ job_reg, uint32_t* __restrict__ job_p0,
                                                         uint32_t* __restrict__ state, uint32_t list_cap,
-                                                        uint32_t job_points, uint32_t job_cap,
+                                                        uint32_t cus, uint32_t job_cap,
                                                         const PassCounters* __restrict__ ctr, uint32_t dense_points) {
-    __shared__ uint32_t s_a[16], s_b[16], s_c[16];
-    __shared__ uint32_t s_ca, s_cb, s_cc;
-    __shared__ unsigned long long s_wide_e, s_wide_p;  // 64-bit totals: list and point overflow
+    constexpr uint32_t CLASSES = 8;
+    __shared__ unsigned long long s_w[16], s_carry;  // 64-bit: an overflowing list must not wrap
+    __shared__ uint32_t s_cls[CLASSES];
+    __shared__ uint32_t s_jobs;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) {
-        s_ca = 0u;
-        s_cb = 0u;
-        s_cc = 0u;
-        s_wide_e = 0ull;
-        s_wide_p = 0ull;
+    if (tid == 0) s_carry = 0ull;
+    if (tid < (int)CLASSES) s_cls[tid] = 0u;
+    __syncthreads();
+    for (uint32_t base = 0; base < nregions; base += 1024) {
+        const uint32_t i = base + (uint32_t)tid;
+        const unsigned long long pts = i < nregions ? reg_pts[i] : 0ull;
+        unsigned long long incl = pts;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned long long t = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += t;
+        }
+        if (lane == 63) s_w[wave] = incl;
+        __syncthreads();
+        unsigned long long off = s_carry + incl - pts, total = s_carry;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) off += s_w[w];
+            total += s_w[w];
+        }
+        if (i < nregions) {
+            const uint32_t p32 = (uint32_t)min(pts, 0xFFFFFFFFull);
+            reg_ptot[i] = p32;
+            reg_poff[i] = (uint32_t)off;
+            reg_cursor[i] = (uint32_t)off;
+            reg_pts[i] = 0ull;
+        }
+        __syncthreads();
+        if (tid == 0) s_carry = total;
+        __syncthreads();
+    }
+    const uint32_t job_points =
+        (uint32_t)min((unsigned long long)GPS_BIN_JOB_POINTS_MAX,
+                      max((unsigned long long)GPS_BIN_JOB_POINTS, s_carry * 5ull / (6ull * cus)));
+    auto cls_of = [&](uint32_t rest) { return min(CLASSES - 1u, (job_points - rest) * CLASSES / job_points); };
+    for (uint32_t i = (uint32_t)tid; i < nregions; i += 1024) {
+        const uint32_t p32 = reg_ptot[i];  // this thread's own store
+        const uint32_t full = p32 / job_points, rest = p32 - full * job_points;
+        if (full) atomicAdd(&s_cls[0], full);
+        if (rest) atomicAdd(&s_cls[cls_of(rest)], 1u);
     }
     __syncthreads();
-    for (uint32_t base = 0; base < g.nregions; base += 1024) {
-        const uint32_t i = base + tid;
-        const uint32_t cnt = i < g.nregions ? reg_cnt[i] : 0u;
-        const uint32_t pts = i < g.nregions ? reg_pts[i] : 0u;
-        if (cnt) {
-            atomicAdd(&s_wide_e, (unsigned long long)cnt);
-            atomicAdd(&s_wide_p, (unsigned long long)pts);
-        }
-        const uint32_t nj = pts ? (pts + job_points - 1u) / job_points : 0u;
-        const uint32_t ia = wave_scan_incl(cnt), ib = wave_scan_incl(pts), ic = wave_scan_incl(nj);
-        if (lane == 63) {
-            s_a[wave] = ia;
-            s_b[wave] = ib;
-            s_c[wave] = ic;
-        }
-        __syncthreads();
-        uint32_t wa = 0, wb = 0, wc = 0;
-        for (int w = 0; w < wave; ++w) {
-            wa += s_a[w];
-            wb += s_b[w];
-            wc += s_c[w];
-        }
-        const uint32_t ca = s_ca, cb = s_cb, cc = s_cc;
-        if (i < g.nregions) {
-            const uint32_t eoff = ca + wa + ia - cnt, joff = cc + wc + ic - nj;
-            reg_ecnt[i] = cnt;
-            reg_ptot[i] = pts;
-            reg_eoff[i] = eoff;
-            reg_poff[i] = cb + wb + ib - pts;
-            reg_cursor[i] = eoff;
-            reg_jobs[i] = nj;
-            for (uint32_t j = 0; j < nj && joff + j < job_cap; ++j) {
-                job_reg[joff + j] = i;
-                job_p0[joff + j] = j * job_points;
-            }
-            reg_cnt[i] = 0u;
-            reg_pts[i] = 0u;
-        }
-        __syncthreads();
-        if (tid == 1023) {
-            s_ca = ca + wa + ia;
-            s_cb = cb + wb + ib;
-            s_cc = cc + wc + ic;
-        }
-        __syncthreads();
-    }
     if (tid == 0) {
-        state[0] = s_ca;
-        state[1] = min(s_cc, job_cap);
+        uint32_t run = 0;
+        for (uint32_t c = 0; c < CLASSES; ++c) {
+            const uint32_t n = s_cls[c];
+            s_cls[c] = run;
+            run += n;
+        }
+        s_jobs = run;
         const bool dense = ctr && ctr->points > dense_points;
-        state[3] = dense ? 2u : (s_wide_e > list_cap || s_cc > job_cap || s_wide_p > 0xFFFFFFFFull) ? 1u : 0u;
+        state[1] = min(run, job_cap);
+        state[3] = dense ? 2u : (s_carry > list_cap || run > job_cap) ? 1u : 0u;
         state[4] = 0u;
-        state[5] = 0u;
+        state[7] = job_points;
+    }
+    __syncthreads();
+    if (s_jobs > job_cap || s_carry > list_cap) return;
+    for (uint32_t i = (uint32_t)tid; i < nregions; i += 1024) {
+        const uint32_t p32 = reg_ptot[i];
+        const uint32_t full = p32 / job_points, rest = p32 - full * job_points;
+        if (full) {
+            const uint32_t j = atomicAdd(&s_cls[0], full);
+            for (uint32_t k = 0; k < full; ++k) {
+                job_reg[j + k] = i;
+                job_p0[j + k] = k * job_points;
+            }
+        }
+        if (rest) {
+            const uint32_t j = atomicAdd(&s_cls[cls_of(rest)], 1u);
+            job_reg[j] = i;
+            job_p0[j] = full * job_points;
+        }
     }
 }
 
-// Region lists: the entry ranges of bin_count_range; the workgroup counts its
-// entries per region in LDS, reserves one range per region with a single
-// global atomic, and fills it.
-__device__ __forceinline__ void bin_scatter_range(const BinGeom& g, uint32_t r0, uint32_t r1, uint32_t rbase,
-                                                  const uint2* __restrict__ erect, const uint32_t* __restrict__ ew,
-                                                  uint32_t* __restrict__ reg_cursor, uint32_t* __restrict__ list,
-                                                  uint32_t* __restrict__ lw, uint32_t* s_cnt, uint32_t* s_base) {
-    const int tid = threadIdx.x;
-    for (uint32_t i = tid; i < g.nregions; i += 256) s_cnt[i] = 0u;
-    __syncthreads();
-    for (uint32_t r = r0 + tid; r < r1; r += 256) {
-        const uint2 rect = erect[r];
-        if (rect.x == 0xFFFFFFFFu) continue;
-        for (uint32_t ry = rect.y & 0xFFFFu; ry <= (rect.y >> 16); ++ry)
-            for (uint32_t rx = rect.x & 0xFFFFu; rx <= (rect.x >> 16); ++rx)
-                atomicAdd(&s_cnt[ry * (uint32_t)g.nrx + rx], 1u);
+// Point lists of the regions, 4096 entries at a time: the workgroup adds up
+// its entries' points per region in LDS (the Morton-ordered entries touch few
+// regions), reserves one range per region with a single global atomic, and
+// fills it.  The entries stay in registers in between.  A lane writes the
+// points of a small entry by itself (two points on average; sharing them out
+// over the wave's lanes by prefix sums measured 180 us against 145 at 20M
+// points); an entry of more than 16 points is written by its whole wave.
+// `pbias` turns point offsets into the frame's own indices.
+__device__ __forceinline__ void bin_scatter_range(const BinFrame& f, uint32_t r0, uint32_t r1, uint32_t pbias,
+                                                  uint32_t* __restrict__ reg_cursor, uint2* __restrict__ list,
+                                                  uint32_t* s_pos) {
+    constexpr int PER = GPS_LIST_ENTRIES / GPS_LIST_THREADS;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t nrx = (uint32_t)f.g.nrx;
+    for (uint32_t base = r0 + blockIdx.x * GPS_LIST_ENTRIES; base < r1; base += gridDim.x * GPS_LIST_ENTRIES) {
+        for (uint32_t i = tid; i < f.g.nregions; i += GPS_LIST_THREADS) s_pos[i] = 0u;
+        uint32_t rec[PER], p[PER], w[PER];
+        uint2 bnd[PER];
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const uint32_t r = base + (uint32_t)(k * GPS_LIST_THREADS + tid);
+            const uint32_t rc = min(r, r1 - 1u);
+            rec[k] = f.cidx[rc];
+            p[k] = f.coff[rc];
+            const uint32_t next = rc + 1u < f.v_end ? f.coff[rc + 1u] : f.t_end;
+            const uint32_t hi = min(next, f.p_end);
+            w[k] = r < r1 && p[k] < hi ? hi - p[k] : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) bnd[k] = record_bounds(f, rec[k]);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const BinRect q = bounds_rect(f.g, bnd[k], w[k]);
+            if (q.n == 0u || q.n > GPS_BIN_MAX_REGIONS) continue;
+            for (uint32_t ry = q.ry0; ry <= q.ry1; ++ry)
+                for (uint32_t rx = q.rx0; rx <= q.rx1; ++rx) atomicAdd(&s_pos[ry * nrx + rx], w[k]);
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < f.g.nregions; i += GPS_LIST_THREADS)
+            if (s_pos[i]) s_pos[i] = atomicAdd(&reg_cursor[f.rbase + i], s_pos[i]);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            BinRect q = bounds_rect(f.g, bnd[k], w[k]);
+            if (q.n > GPS_BIN_MAX_REGIONS) q.n = 0u;
+            const uint32_t pk = p[k] - pbias, wk = w[k], rk = rec[k];
+            uint32_t rx = q.rx0, ry = q.ry0;
+            for (uint32_t j = 0; __ballot(j < q.n) != 0ull; ++j) {
+                uint32_t slot = 0u;
+                const bool has = j < q.n;
+                if (has) {
+                    slot = atomicAdd(&s_pos[ry * nrx + rx], wk);
+                    if (rx == q.rx1) {
+                        rx = q.rx0;
+                        ++ry;
+                    } else {
+                        ++rx;
+                    }
+                }
+                if (has && wk <= 16u)
+                    for (uint32_t i = 0; i < wk; ++i) list[slot + i] = make_uint2(rk, pk + i);
+                for (uint64_t m = __ballot(has && wk > 16u); m; m &= m - 1ull) {
+                    const int src = __builtin_ctzll(m);
+                    const uint32_t bw = __shfl(wk, src, 64), bs = __shfl(slot, src, 64), br = __shfl(rk, src, 64),
+                                   bp = __shfl(pk, src, 64);
+                    for (uint32_t i = (uint32_t)lane; i < bw; i += 64u) list[bs + i] = make_uint2(br, bp + i);
+                }
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    for (uint32_t i = tid; i < g.nregions; i += 256) {
-        if (s_cnt[i]) s_base[i] = atomicAdd(&reg_cursor[rbase + i], s_cnt[i]);
-        s_cnt[i] = 0u;
+}
+
+// The frame's clear, where the binned splat does not make it needless: with
+// `all` every word, else the words of the regions that no job or several jobs
+// render (a region's one job stores all of it).  Shared by the workgroups of a
+// grid row.
+__device__ __forceinline__ void bin_clear(const BinGeom& g, uint32_t rbase, const uint32_t* __restrict__ reg_ptot,
+                                          uint32_t job_points, bool all, uint64_t fb_words, uint64_t background,
+                                          unsigned long long* __restrict__ fb) {
+    const uint4 v = make_uint4((uint32_t)background, (uint32_t)(background >> 32), (uint32_t)background,
+                               (uint32_t)(background >> 32));
+    uint4* dst = reinterpret_cast<uint4*>(fb);
+    if (all) {
+        for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < fb_words / 2;
+             i += (uint64_t)gridDim.x * blockDim.x)
+            dst[i] = v;
+        return;
     }
-    __syncthreads();
-    for (uint32_t r = r0 + tid; r < r1; r += 256) {
-        const uint2 rect = erect[r];
-        if (rect.x == 0xFFFFFFFFu) continue;
-        const uint32_t w = ew[r];
-        for (uint32_t ry = rect.y & 0xFFFFu; ry <= (rect.y >> 16); ++ry)
-            for (uint32_t rx = rect.x & 0xFFFFu; rx <= (rect.x >> 16); ++rx) {
-                const uint32_t reg = ry * (uint32_t)g.nrx + rx;
-                const uint32_t slot = s_base[reg] + atomicAdd(&s_cnt[reg], 1u);
-                list[slot] = r;
-                lw[slot] = w;
+    const uint32_t half = GPS_TILE_WORDS * (uint32_t)g.spp / 2u;  // 16-byte pieces of a 64x64 tile
+    const int tiles_rows = (g.up_h + GPS_TILE_SIZE - 1) >> GPS_TILE_BITS;
+    for (uint32_t reg = blockIdx.x; reg < g.nregions; reg += gridDim.x) {
+        const uint32_t tot = reg_ptot[rbase + reg];
+        if (tot != 0u && tot <= job_points) continue;
+        const int tx0 = (int)(reg % (uint32_t)g.nrx) * g.rtx, ty0 = (int)(reg / (uint32_t)g.nrx) * g.rty;
+        for (int ty = ty0; ty < min(ty0 + g.rty, tiles_rows); ++ty)
+            for (int tx = tx0; tx < min(tx0 + g.rtx, g.tiles_per_row); ++tx) {
+                uint4* t = dst + (uint64_t)(ty * g.tiles_per_row + tx) * half;
+                for (uint32_t i = threadIdx.x; i < half; i += blockDim.x) t[i] = v;
             }
     }
 }
 
-__global__ __launch_bounds__(256) void bin_scatter_kernel(const PassCounters* __restrict__ ctr, BinGeom g,
-                                                          const uint2* __restrict__ erect,
-                                                          const uint32_t* __restrict__ ew,
-                                                          uint32_t* __restrict__ reg_cursor,
-                                                          uint32_t* __restrict__ list, uint32_t* __restrict__ lw,
-                                                          const uint32_t* __restrict__ state) {
-    extern __shared__ uint32_t s_dyn[];  // 2 * nregions words
+// `clear_words` (or 0): the frame's framebuffer of that many words has not been
+// cleared yet.
+__global__ __launch_bounds__(GPS_LIST_THREADS) void bin_scatter_kernel(BinFrame f, const PassCounters* __restrict__ ctr,
+                                                                       uint32_t* __restrict__ reg_cursor,
+                                                                       uint2* __restrict__ list,
+                                                                       const uint32_t* __restrict__ state,
+                                                                       const uint32_t* __restrict__ reg_ptot,
+                                                                       unsigned long long* __restrict__ fb,
+                                                                       uint64_t clear_words, uint64_t background) {
+    extern __shared__ uint32_t s_dyn[];  // nregions words
+    if (clear_words) bin_clear(f.g, 0u, reg_ptot, state[7], state[3] != 0u, clear_words, background, fb);
     if (state[3]) return;
-    const uint32_t V = ctr->valid;
-    const uint32_t per = (V + gridDim.x - 1) / gridDim.x;
-    const uint32_t r0 = min(V, blockIdx.x * per), r1 = min(V, r0 + per);
-    bin_scatter_range(g, r0, r1, 0u, erect, ew, reg_cursor, list, lw, s_dyn, s_dyn + g.nregions);
-}
-// Exclusive scan of lw over the list (region-major) in tiles of 4096 slots:
-// per-tile sums, a one-workgroup scan of the tile sums, then the local scan.
-// The list length comes from the device (grid-stride over its tiles).
-__global__ __launch_bounds__(256) void bin_tile_sum_kernel(const uint32_t* __restrict__ lw,
-                                                           const uint32_t* __restrict__ state,
-                                                           uint32_t* __restrict__ tsum) {
-    __shared__ uint32_t s[4];
-    const uint32_t L = state[3] ? 0u : state[0];
-    const uint32_t nt = (L + GPS_TILE - 1) / GPS_TILE;
-    for (uint32_t tile = blockIdx.x; tile < nt; tile += gridDim.x) {
-        const uint32_t t0 = tile * GPS_TILE + threadIdx.x * 16u;
-        uint32_t sum = 0;
-        if (t0 < L) {
-            const uint4* p = reinterpret_cast<const uint4*>(lw + t0);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint4 v = p[k];
-                const uint32_t b = t0 + 4u * k;
-                sum += (b < L ? v.x : 0u) + (b + 1 < L ? v.y : 0u) + (b + 2 < L ? v.z : 0u) + (b + 3 < L ? v.w : 0u);
-            }
-        }
-        sum = wave_reduce_add(sum);
-        if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = sum;
-        __syncthreads();
-        if (threadIdx.x == 0) tsum[tile] = (s[0] + s[1]) + (s[2] + s[3]);
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(1024) void bin_tiles_scan_kernel(const uint32_t* __restrict__ tsum,
-                                                              const uint32_t* __restrict__ state,
-                                                              uint32_t* __restrict__ toff) {
-    __shared__ uint32_t s_a[16];
-    __shared__ uint32_t s_carry;
-    const uint32_t L = state[3] ? 0u : state[0];
-    const uint32_t nt = (L + GPS_TILE - 1) / GPS_TILE;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) s_carry = 0u;
-    __syncthreads();
-    for (uint32_t base = 0; base < nt; base += 1024) {
-        const uint32_t i = base + tid;
-        const uint32_t a = i < nt ? tsum[i] : 0u;
-        const uint32_t ia = wave_scan_incl(a);
-        if (lane == 63) s_a[wave] = ia;
-        __syncthreads();
-        uint32_t wa = 0;
-        for (int w = 0; w < wave; ++w) wa += s_a[w];
-        const uint32_t c = s_carry;
-        if (i < nt) toff[i] = c + wa + ia - a;
-        __syncthreads();
-        if (tid == 1023) s_carry = c + wa + ia;
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(256) void bin_local_scan_kernel(const uint32_t* __restrict__ lw,
-                                                             const uint32_t* __restrict__ state,
-                                                             const uint32_t* __restrict__ toff,
-                                                             uint32_t* __restrict__ lpre) {
-    __shared__ uint32_t s_a[4];
-    const uint32_t L = state[3] ? 0u : state[0];
-    const uint32_t nt = (L + GPS_TILE - 1) / GPS_TILE;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (uint32_t tile = blockIdx.x; tile < nt; tile += gridDim.x) {
-        const uint32_t b0 = tile * GPS_TILE + (uint32_t)tid * 16u;
-        uint32_t w[16];
-        const uint4* p = reinterpret_cast<const uint4*>(lw + b0);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint4 v = b0 < L ? p[k] : make_uint4(0u, 0u, 0u, 0u);
-            w[4 * k] = b0 + 4u * k < L ? v.x : 0u;
-            w[4 * k + 1] = b0 + 4u * k + 1u < L ? v.y : 0u;
-            w[4 * k + 2] = b0 + 4u * k + 2u < L ? v.z : 0u;
-            w[4 * k + 3] = b0 + 4u * k + 3u < L ? v.w : 0u;
-        }
-        uint32_t sa = 0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) sa += w[k];
-        const uint32_t ia = wave_scan_incl(sa);
-        if (lane == 63) s_a[wave] = ia;
-        __syncthreads();
-        uint32_t wa = 0;
-        for (int q = 0; q < wave; ++q) wa += s_a[q];
-        uint32_t off = toff[tile] + wa + ia - sa;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            if (b0 + (uint32_t)k < L) lpre[b0 + k] = off;
-            off += w[k];
-        }
-        __syncthreads();
-    }
+    f.v_end = ctr->valid;
+    f.t_end = ctr->total;
+    f.p_end = ctr->points;
+    bin_scatter_range(f, 0u, f.v_end, 0u, reg_cursor, list, s_dyn);
 }
 
 struct BinSplat {
     BinGeom g;
-    int32_t K, unbiased;
+    int32_t K;
     uint32_t frame_seed;
     uint64_t background;
+    int32_t fresh;  // the framebuffer holds only the background: single-job regions need not read it
 };
 
-// Samples of point p of one Gaussian that land in the LDS region.
-__device__ __forceinline__ void splat_point_region(const SplatRecord& rec, uint32_t p, const BinSplat& b, int rx0,
-                                                   int ry0, unsigned long long* s_fb) {
-    const SampleRect rect = record_rect(rec);
-    const unsigned long long packed = ((unsigned long long)rec.packed_hi << 32) | rec.packed_lo;
-    const unsigned long long depth_bits = packed & ~(unsigned long long)GPS_COLOR_MASK;
-    const int rw = 1 << b.g.rw_shift, rh = 1 << b.g.rh_shift;
-    const int K = b.K, spp = b.g.spp, samples = spp * K;
-    u32x2 seed = make_seed(p, b.frame_seed);
-    for (int layer = 0, k = 0, q = 0; q < samples; ++q) {
-        if (k == K) {
-            k = 0;
-            ++layer;
-        }
-        ++k;
-        seed = pcg2d_uint(seed);
-        uint32_t ux, uy;
-        if (!sample_pixel(rec, seed, rect, ux, uy)) continue;
-        const int x = rect.x0 + (int)ux, y = rect.y0 + (int)uy;
-        const int lx = x - rx0, ly = y - ry0;
-        if ((unsigned)lx >= (unsigned)rw || (unsigned)ly >= (unsigned)rh) continue;  // another region's sample
-        const uint32_t t = (uint32_t)((ly >> GPS_TILE_BITS) * b.g.rtx + (lx >> GPS_TILE_BITS));
-        const uint32_t i = (t * GPS_TILE_WORDS + morton_encode((uint32_t)(x & (GPS_TILE_SIZE - 1)),
-                                                                (uint32_t)(y & (GPS_TILE_SIZE - 1)))) *
-                               (uint32_t)spp +
-                           (uint32_t)layer;
-        if (s_fb[i] <= depth_bits) continue;
-        atomicMin(s_fb + i, packed);
+// A region in LDS: one plane per sample layer, rows of the region's pixels at
+// a pitch of 4 more words.  In the framebuffer's own order (Morton, layers
+// innermost) a step of the sample loop, whose lanes write one layer, would use
+// a quarter of the banks at 4 spp, and the index would take 14 more
+// instructions per sample.
+template <int SPP> struct RegionLds {
+    static constexpr int W_SHIFT = SPP <= 2 ? 7 : 6, H_SHIFT = SPP == 1 ? 7 : 6;
+    static constexpr uint32_t PITCH = (1u << W_SHIFT) + 4u;
+    static constexpr uint32_t PLANE = PITCH << H_SHIFT;
+    static constexpr uint32_t WORDS = PLANE * SPP;
+    static_assert(WORDS <= GPS_BIN_LDS_WORDS, "the region fits");
+    // LDS word of the region's framebuffer word w (tiles of 64x64 pixels, row
+    // by row)
+    __device__ __forceinline__ static uint32_t word(uint32_t w) {
+        constexpr uint32_t TILE = GPS_TILE_WORDS * SPP;
+        const uint32_t t = w / TILE, in = w % TILE;
+        const uint32_t m = in / SPP, layer = in % SPP;
+        constexpr uint32_t RTX = 1u << (W_SHIFT - GPS_TILE_BITS);
+        const uint32_t x = morton_compact(m) + (t % RTX) * GPS_TILE_SIZE;
+        const uint32_t y = morton_compact(m >> 1) + (t / RTX) * GPS_TILE_SIZE;
+        return layer * PLANE + y * PITCH + x;
     }
-}
+};
 
-// One region job: the region's words from the framebuffer (a region with one
-// job) or the background (several jobs), the job's points [p_lo, p_hi) of
-// the region's list (e0, ecnt: its slots; pbase: its first point in list
-// order), then the region back to the framebuffer: a plain store, or
-// atomicMin of the changed words when the region has several jobs.  `pbias`
-// turns the entries' point offsets into the frame's own point indices.
-// Returns the global atomics issued.  Called by every thread of the
-// workgroup.
+// One region job: the job's points [p_lo, p_hi) of the region's list, then the
+// region to the framebuffer: a plain store of a single job's region (started
+// from the framebuffer's words, or from the background in a fresh one), or
+// atomicMin of the words below the framebuffer's when the region has several
+// jobs (started from the background; the n-th job of a region to end lowers
+// about one word in n).  Called by every thread of the workgroup; returns the
+// global atomics issued.
+//
+// A thread takes every 1024th point.  Its next list entry and the next point's
+// record are requested a point ahead, so that the loop waits for no memory
+// and holds no barrier: with the entries found by search in an LDS prefix and
+// records loaded at use, the waves spent 53 % of their time waiting.
+template <int SPP>
 __device__ __forceinline__ uint32_t bin_splat_job(const SplatRecord* __restrict__ recs,
-                                                  const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ coff,
-                                                  const uint32_t* __restrict__ list, const uint32_t* __restrict__ lpre,
-                                                  uint32_t e0, uint32_t ecnt, uint32_t pbase, uint32_t p_lo,
-                                                  uint32_t p_hi, bool single, uint32_t lreg, const BinSplat& b,
-                                                  unsigned long long* __restrict__ fb, uint32_t pbias,
-                                                  unsigned long long* s_fb, uint32_t* s_off, uint32_t* s_slot0) {
+                                                  const uint2* __restrict__ list, uint32_t p_lo, uint32_t p_hi,
+                                                  bool single, uint32_t lreg, const BinSplat& b,
+                                                  unsigned long long* __restrict__ fb, unsigned long long* s_fb) {
+    using L = RegionLds<SPP>;
+    constexpr uint32_t words = GPS_TILE_WORDS * SPP << (L::W_SHIFT + L::H_SHIFT - 2 * GPS_TILE_BITS);
+    constexpr uint32_t tile_words = GPS_TILE_WORDS * SPP;
+    constexpr uint32_t RTX = 1u << (L::W_SHIFT - GPS_TILE_BITS);
     const int tid = threadIdx.x;
-    const uint32_t words = bin_region_words(b.g);
-    const uint32_t tile_words = GPS_TILE_WORDS * (uint32_t)b.g.spp;
     const int tiles_rows = (b.g.up_h + GPS_TILE_SIZE - 1) >> GPS_TILE_BITS;
     const int rxi = (int)(lreg % (uint32_t)b.g.nrx), ryi = (int)(lreg / (uint32_t)b.g.nrx);
-    const int rx0 = rxi << b.g.rw_shift, ry0 = ryi << b.g.rh_shift;
+    const int rx0 = rxi << L::W_SHIFT, ry0 = ryi << L::H_SHIFT;
     const int tx0 = rx0 >> GPS_TILE_BITS, ty0 = ry0 >> GPS_TILE_BITS;
+    uint32_t p = p_lo + (uint32_t)tid;
+    uint2 cur = make_uint2(0u, 0u), nxt = make_uint2(0u, 0u);
+    SplatRecord rec{};
+    if (p < p_hi) cur = list[p];
+    if (p < p_hi && p_hi - p > GPS_BIN_THREADS) nxt = list[p + GPS_BIN_THREADS];
+    if (p < p_hi) rec = load_record(recs, cur.x);
+    if (single && !b.fresh) {
+        for (uint32_t w = (uint32_t)tid * 2u; w < words; w += 2u * GPS_BIN_THREADS) {
+            const uint32_t t = w / tile_words, within = w % tile_words;
+            const int tx = tx0 + (int)(t % RTX), ty = ty0 + (int)(t / RTX);
+            if (tx >= b.g.tiles_per_row || ty >= tiles_rows) continue;  // no sample lands there
+            const uint4 v = *reinterpret_cast<const uint4*>(fb + (uint64_t)(ty * b.g.tiles_per_row + tx) * tile_words + within);
+            s_fb[L::word(w)] = ((unsigned long long)v.y << 32) | v.x;
+            s_fb[L::word(w + 1u)] = ((unsigned long long)v.w << 32) | v.z;
+        }
+    } else {
+        for (uint32_t i = (uint32_t)tid; i < L::WORDS; i += GPS_BIN_THREADS) s_fb[i] = b.background;
+    }
+    __syncthreads();
+    while (p < p_hi) {
+        SplatRecord nrec = rec;
+        uint2 nnxt = nxt;
+        const bool more = p_hi - p > GPS_BIN_THREADS;
+        if (more) nrec = load_record(recs, nxt.x);
+        if (p_hi - p > 2u * GPS_BIN_THREADS) nnxt = list[p + 2u * GPS_BIN_THREADS];
+        // the Gaussian's bounds inside the region
+        SampleRect rect = record_rect(rec);
+        const int ox = max(rect.x0 - rx0, 0), oy = max(rect.y0 - ry0, 0);
+        rect.w = (uint32_t)max(min(rect.x0 + (int)rect.w, rx0 + (1 << L::W_SHIFT)) - (rx0 + ox), 0);
+        rect.h = (uint32_t)max(min(rect.y0 + (int)rect.h, ry0 + (1 << L::H_SHIFT)) - (ry0 + oy), 0);
+        rect.x0 = rx0 + ox;
+        rect.y0 = ry0 + oy;
+        const unsigned long long packed = ((unsigned long long)rec.packed_hi << 32) | rec.packed_lo;
+        unsigned long long* dst = s_fb + (uint32_t)oy * L::PITCH + (uint32_t)ox;
+        u32x2 seed = make_seed(cur.y, b.frame_seed);
+        for (int layer = 0; layer < SPP; ++layer, dst += L::PLANE)
+            for (int k = 0; k < b.K; ++k) {
+                seed = pcg2d_uint(seed);
+                uint32_t ux, uy;
+                if (!sample_pixel(rec, seed, rect, ux, uy)) continue;
+                atomicMin(dst + (__umul24(uy, L::PITCH) + ux), packed);
+            }
+        rec = nrec;
+        cur = nxt;
+        nxt = nnxt;
+        if (!more) break;
+        p += GPS_BIN_THREADS;
+    }
+    __syncthreads();
     uint32_t merged = 0;
-    // region words <- framebuffer (single job) or background (merged later)
     for (uint32_t w = (uint32_t)tid * 2u; w < words; w += 2u * GPS_BIN_THREADS) {
-        const uint32_t t = w / tile_words, within = w - t * tile_words;
-        const int tx = tx0 + (int)(t % (uint32_t)b.g.rtx), ty = ty0 + (int)(t / (uint32_t)b.g.rtx);
-        uint4 v = make_uint4((uint32_t)b.background, (uint32_t)(b.background >> 32), (uint32_t)b.background,
-                             (uint32_t)(b.background >> 32));
-        if (single && tx < b.g.tiles_per_row && ty < tiles_rows)
-            v = *reinterpret_cast<const uint4*>(fb + (uint64_t)(ty * b.g.tiles_per_row + tx) * tile_words + within);
-        s_fb[w] = ((unsigned long long)v.y << 32) | v.x;
-        s_fb[w + 1] = ((unsigned long long)v.w << 32) | v.z;
-    }
-    for (uint32_t q0 = p_lo; q0 < p_hi; q0 += GPS_BIN_CHUNK) {
-        // last slot whose region-local prefix is <= q0
-        if (tid == 0) {
-            uint32_t lo = 0, hi = ecnt - 1u;
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi + 1u) >> 1;
-                if (lpre[e0 + mid] - pbase <= q0) lo = mid;
-                else hi = mid - 1u;
-            }
-            *s_slot0 = lo;
-        }
-        __syncthreads();
-        const uint32_t j0 = *s_slot0;
-        for (int j = tid; j <= GPS_BIN_CHUNK; j += GPS_BIN_THREADS)
-            s_off[j] = j0 + (uint32_t)j < ecnt ? lpre[e0 + j0 + (uint32_t)j] - pbase : 0xFFFFFFFFu;
-        __syncthreads();
-        const uint32_t qa = q0 + (uint32_t)tid * GPS_BIN_PPT;
-        if (qa < p_hi) {
-            int lo = 0, hi = GPS_BIN_CHUNK;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (s_off[mid] <= qa) lo = mid;
-                else hi = mid - 1;
-            }
-            int j = lo;
-            uint32_t cur = 0xFFFFFFFFu, pstart = 0;
-            SplatRecord rec;
-            for (int k = 0; k < GPS_BIN_PPT; ++k) {
-                const uint32_t q = qa + (uint32_t)k;
-                if (q >= p_hi) break;
-                while (j < GPS_BIN_CHUNK - 1 && s_off[j + 1] <= q) ++j;
-                const uint32_t slot = j0 + (uint32_t)j;
-                if (slot >= ecnt) break;
-                if (slot != cur) {
-                    cur = slot;
-                    const uint32_t r = list[e0 + slot];
-                    pstart = coff[r] - pbias;
-                    rec = load_record(recs, cidx[r]);
-                }
-                splat_point_region(rec, pstart + (q - s_off[j]), b, rx0, ry0, s_fb);
-            }
-        }
-        __syncthreads();
-    }
-    // region -> framebuffer
-    for (uint32_t w = (uint32_t)tid * 2u; w < words; w += 2u * GPS_BIN_THREADS) {
-        const uint32_t t = w / tile_words, within = w - t * tile_words;
-        const int tx = tx0 + (int)(t % (uint32_t)b.g.rtx), ty = ty0 + (int)(t / (uint32_t)b.g.rtx);
+        const uint32_t t = w / tile_words, within = w % tile_words;
+        const int tx = tx0 + (int)(t % RTX), ty = ty0 + (int)(t / RTX);
         if (tx >= b.g.tiles_per_row || ty >= tiles_rows) continue;
         unsigned long long* dst = fb + (uint64_t)(ty * b.g.tiles_per_row + tx) * tile_words + within;
-        const unsigned long long a0 = s_fb[w], a1 = s_fb[w + 1];
+        const unsigned long long a0 = s_fb[L::word(w)], a1 = s_fb[L::word(w + 1u)];
         if (single) {
             *reinterpret_cast<uint4*>(dst) = make_uint4((uint32_t)a0, (uint32_t)(a0 >> 32), (uint32_t)a1,
                                                         (uint32_t)(a1 >> 32));
         } else {
-            if (a0 != b.background) {
+            // another job's words may be newer than this read; the minimum decides
+            const uint4 v = *reinterpret_cast<const uint4*>(dst);
+            if (a0 < (((unsigned long long)v.y << 32) | v.x)) {
                 atomicMin(dst, a0);
                 ++merged;
             }
-            if (a1 != b.background) {
+            if (a1 < (((unsigned long long)v.w << 32) | v.z)) {
                 atomicMin(dst + 1, a1);
                 ++merged;
             }
@@ -2138,63 +2193,39 @@ __device__ __forceinline__ uint32_t bin_splat_job(const SplatRecord* __restrict_
     __syncthreads();
     return merged;
 }
+__device__ __forceinline__ uint32_t bin_splat_any(const SplatRecord* __restrict__ recs,
+                                                  const uint2* __restrict__ list, uint32_t p_lo, uint32_t p_hi,
+                                                  bool single, uint32_t lreg, const BinSplat& b,
+                                                  unsigned long long* __restrict__ fb, unsigned long long* s_fb) {
+    switch (b.g.spp) {
+        case 1: return bin_splat_job<1>(recs, list, p_lo, p_hi, single, lreg, b, fb, s_fb);
+        case 2: return bin_splat_job<2>(recs, list, p_lo, p_hi, single, lreg, b, fb, s_fb);
+        case 3: return bin_splat_job<3>(recs, list, p_lo, p_hi, single, lreg, b, fb, s_fb);
+        default: return bin_splat_job<4>(recs, list, p_lo, p_hi, single, lreg, b, fb, s_fb);
+    }
+}
 
 // Persistent, one 1024-thread workgroup per CU (the region buffer is most of
 // the LDS); jobs are taken from a device counter.
 __global__ __launch_bounds__(GPS_BIN_THREADS) void bin_splat_kernel(
-    const SplatRecord* __restrict__ recs, const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ coff,
-    const uint32_t* __restrict__ list, const uint32_t* __restrict__ lpre, const uint32_t* __restrict__ reg_ecnt,
-    const uint32_t* __restrict__ reg_ptot, const uint32_t* __restrict__ reg_eoff, const uint32_t* __restrict__ reg_poff,
-    const uint32_t* __restrict__ reg_jobs, const uint32_t* __restrict__ job_reg, const uint32_t* __restrict__ job_p0,
-    uint32_t* __restrict__ state, unsigned long long* __restrict__ fb, BinSplat b, uint32_t job_points,
+    const SplatRecord* __restrict__ recs, const uint2* __restrict__ list, const uint32_t* __restrict__ reg_ptot,
+    const uint32_t* __restrict__ reg_poff, const uint32_t* __restrict__ job_reg, const uint32_t* __restrict__ job_p0,
+    uint32_t* __restrict__ state, unsigned long long* __restrict__ fb, BinSplat b,
     uint32_t* __restrict__ atomics_count) {
-    __shared__ unsigned long long s_fb[GPS_BIN_WORDS];
-    __shared__ uint32_t s_off[GPS_BIN_CHUNK + 1];
-    __shared__ uint32_t s_job, s_slot0;
+    __shared__ unsigned long long s_fb[GPS_BIN_LDS_WORDS];
+    __shared__ uint32_t s_job;
     if (state[3]) return;
-    const uint32_t njobs = state[1];
+    const uint32_t njobs = state[1], job_points = state[7];
     uint32_t merged = 0;
     for (;;) {
         if (threadIdx.x == 0) s_job = atomicAdd(&state[4], 1u);
         __syncthreads();
         const uint32_t job = s_job;
         if (job >= njobs) break;
-        const uint32_t reg = job_reg[job];
-        const uint32_t p_lo = job_p0[job];
-        const uint32_t p_hi = min(reg_ptot[reg], p_lo + job_points);
-        merged += bin_splat_job(recs, cidx, coff, list, lpre, reg_eoff[reg], reg_ecnt[reg], reg_poff[reg], p_lo, p_hi,
-                                reg_jobs[reg] == 1u, reg, b, fb, 0u, s_fb, s_off, &s_slot0);
+        const uint32_t reg = job_reg[job], p0 = job_p0[job], tot = reg_ptot[reg], off = reg_poff[reg];
+        merged += bin_splat_any(recs, list, off + p0, off + min(tot, p0 + job_points), tot <= job_points, reg, b, fb, s_fb);
     }
     if (atomics_count) add_count(atomics_count, merged);
-}
-
-// Gaussians too large to bin: all their points with global atomics, after
-// the regions are written.
-__global__ __launch_bounds__(256) void bin_big_kernel(const SplatRecord* __restrict__ recs,
-                                                      const uint32_t* __restrict__ cidx,
-                                                      const uint32_t* __restrict__ coff,
-                                                      const uint32_t* __restrict__ ew, const uint32_t* __restrict__ big,
-                                                      uint32_t* __restrict__ state, unsigned long long* __restrict__ fb,
-                                                      SplatConsts sc, uint32_t* __restrict__ atomics_count) {
-    __shared__ uint32_t s_e;
-    if (state[3]) return;
-    const int tid = threadIdx.x;
-    const uint32_t nbig = state[2];
-    uint32_t issued = 0;
-    for (;;) {
-        if (tid == 0) s_e = atomicAdd(&state[5], 1u);
-        __syncthreads();
-        const uint32_t e = s_e;
-        __syncthreads();
-        if (e >= nbig) break;
-        const uint32_t r = big[e];
-        const SplatRecord rec = load_record(recs, cidx[r]);
-        const uint32_t p0 = coff[r], w = ew[r];
-        int last = -1;  // one Gaussian throughout
-        for (uint32_t k = (uint32_t)tid; k < w; k += 256u)
-            issued += splat_point(rec, p0 + k, sc.frame_seed, sc.K, sc.spp, sc.up_w, sc.unbiased, fb, last);
-    }
-    if (atomics_count) add_count(atomics_count, issued);
 }
 
 // ------------------------------------------------------------------ binned splat, batches
@@ -2207,40 +2238,22 @@ __global__ __launch_bounds__(256) void bin_big_kernel(const SplatRecord* __restr
 // dense_points, are left to the point-parallel batch splat (their regions stay
 // empty).
 
-__global__ __launch_bounds__(256) void batch_bin_count_kernel(const SplatRecord* __restrict__ recs,
-                                                              const uint32_t* __restrict__ cidx,
-                                                              const uint32_t* __restrict__ coff,
-                                                              const BatchView* __restrict__ views,
-                                                              uint2* __restrict__ erect, uint32_t* __restrict__ ew,
-                                                              uint32_t* __restrict__ reg_cnt,
-                                                              uint32_t* __restrict__ reg_pts,
-                                                              uint32_t* __restrict__ big, uint32_t* __restrict__ state) {
-    extern __shared__ uint32_t s_dyn[];  // 2 * the largest view's regions
-    const BatchView& bv = views[blockIdx.y];
-    const BinGeom g = bv.bg;
-    if (g.nregions == 0u || bv.points > bv.dense_points) return;
-    const uint32_t V = bv.valid, eb = bv.ebase;
-    const uint32_t per = (V + gridDim.x - 1) / gridDim.x;
-    const uint32_t r0 = eb + min(V, blockIdx.x * per), r1 = eb + min(V, blockIdx.x * per + per);
-    bin_count_range(recs, cidx, coff, g, r0, r1, eb + V, bv.base + bv.total, bv.base + bv.points, bv.rbase, erect, ew,
-                    reg_cnt, reg_pts, big, state, s_dyn, s_dyn + g.nregions);
-}
-
-__global__ __launch_bounds__(256) void batch_bin_scatter_kernel(const BatchView* __restrict__ views,
-                                                                const uint2* __restrict__ erect,
-                                                                const uint32_t* __restrict__ ew,
-                                                                uint32_t* __restrict__ reg_cursor,
-                                                                uint32_t* __restrict__ list, uint32_t* __restrict__ lw,
-                                                                const uint32_t* __restrict__ state) {
+__global__ __launch_bounds__(GPS_LIST_THREADS) void batch_bin_scatter_kernel(
+    BinFrame f, const BatchView* __restrict__ views, uint32_t* __restrict__ reg_cursor, uint2* __restrict__ list,
+    const uint32_t* __restrict__ state, const uint32_t* __restrict__ reg_ptot, unsigned long long* __restrict__ fb) {
     extern __shared__ uint32_t s_dyn[];
-    if (state[3]) return;
     const BatchView& bv = views[blockIdx.y];
-    const BinGeom g = bv.bg;
-    if (g.nregions == 0u || bv.points > bv.dense_points) return;
-    const uint32_t V = bv.valid, eb = bv.ebase;
-    const uint32_t per = (V + gridDim.x - 1) / gridDim.x;
-    const uint32_t r0 = eb + min(V, blockIdx.x * per), r1 = eb + min(V, blockIdx.x * per + per);
-    bin_scatter_range(g, r0, r1, bv.rbase, erect, ew, reg_cursor, list, lw, s_dyn, s_dyn + g.nregions);
+    if (bv.bg.nregions == 0u) return;  // cleared by batch_clear_kernel
+    const bool pp = state[3] != 0u || bv.points > bv.dense_points;
+    bin_clear(bv.bg, bv.rbase, reg_ptot, state[7], pp, bv.fb_words, bv.background, fb + bv.fb_offset);
+    if (pp) return;
+    f.g = bv.bg;
+    if (!bv.write_bounds) f.bounds = nullptr;
+    f.v_end = bv.ebase + bv.valid;
+    f.t_end = bv.base + bv.total;
+    f.p_end = bv.base + bv.points;
+    f.rbase = bv.rbase;
+    bin_scatter_range(f, bv.ebase, f.v_end, bv.base, reg_cursor, list, s_dyn);
 }
 
 // The view that owns global region `reg`: the last view whose rbase <= reg
@@ -2256,18 +2269,15 @@ __device__ __forceinline__ int batch_region_view(const BatchView* __restrict__ v
 }
 
 __global__ __launch_bounds__(GPS_BIN_THREADS) void batch_bin_splat_kernel(
-    const SplatRecord* __restrict__ recs, const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ coff,
-    const uint32_t* __restrict__ list, const uint32_t* __restrict__ lpre, const uint32_t* __restrict__ reg_ecnt,
-    const uint32_t* __restrict__ reg_ptot, const uint32_t* __restrict__ reg_eoff, const uint32_t* __restrict__ reg_poff,
-    const uint32_t* __restrict__ reg_jobs, const uint32_t* __restrict__ job_reg, const uint32_t* __restrict__ job_p0,
+    const SplatRecord* __restrict__ recs, const uint2* __restrict__ list, const uint32_t* __restrict__ reg_ptot,
+    const uint32_t* __restrict__ reg_poff, const uint32_t* __restrict__ job_reg, const uint32_t* __restrict__ job_p0,
     uint32_t* __restrict__ state, const BatchView* __restrict__ views, int nviews,
-    unsigned long long* __restrict__ fb, uint32_t job_points, uint32_t* __restrict__ atomics_count) {
-    __shared__ unsigned long long s_fb[GPS_BIN_WORDS];
-    __shared__ uint32_t s_off[GPS_BIN_CHUNK + 1];
-    __shared__ uint32_t s_job, s_slot0;
+    unsigned long long* __restrict__ fb, uint32_t* __restrict__ atomics_count) {
+    __shared__ unsigned long long s_fb[GPS_BIN_LDS_WORDS];
+    __shared__ uint32_t s_job;
     __shared__ int s_view;
     if (state[3]) return;
-    const uint32_t njobs = state[1];
+    const uint32_t njobs = state[1], job_points = state[7];
     uint32_t merged = 0;
     for (;;) {
         if (threadIdx.x == 0) {
@@ -2281,15 +2291,12 @@ __global__ __launch_bounds__(GPS_BIN_THREADS) void batch_bin_splat_kernel(
         BinSplat b;
         b.g = bv.bg;
         b.K = bv.f.Ki;
-        b.unbiased = bv.f.unbiased;
         b.frame_seed = bv.f.frame_seed + 1u;
         b.background = bv.background;
-        const uint32_t reg = job_reg[job];
-        const uint32_t p_lo = job_p0[job];
-        const uint32_t p_hi = min(reg_ptot[reg], p_lo + job_points);
-        merged += bin_splat_job(recs, cidx, coff, list, lpre, reg_eoff[reg], reg_ecnt[reg], reg_poff[reg], p_lo, p_hi,
-                                reg_jobs[reg] == 1u, reg - bv.rbase, b, fb + bv.fb_offset, bv.base, s_fb, s_off,
-                                &s_slot0);
+        b.fresh = 1;
+        const uint32_t reg = job_reg[job], p0 = job_p0[job], tot = reg_ptot[reg], off = reg_poff[reg];
+        merged += bin_splat_any(recs, list, off + p0, off + min(tot, p0 + job_points), tot <= job_points,
+                                reg - bv.rbase, b, fb + bv.fb_offset, s_fb);
     }
     if (atomics_count) add_count(atomics_count, merged);
 }
@@ -2298,30 +2305,24 @@ __global__ __launch_bounds__(256) void batch_bin_big_kernel(const SplatRecord* _
                                                             const uint32_t* __restrict__ cidx,
                                                             const uint32_t* __restrict__ coff,
                                                             const uint8_t* __restrict__ cview,
-                                                            const uint32_t* __restrict__ ew,
-                                                            const uint32_t* __restrict__ big,
-                                                            uint32_t* __restrict__ state,
+                                                            const uint2* __restrict__ big,
+                                                            const uint32_t* __restrict__ state,
                                                             const BatchView* __restrict__ views,
                                                             unsigned long long* __restrict__ fb,
                                                             uint32_t* __restrict__ atomics_count) {
-    __shared__ uint32_t s_e;
     if (state[3]) return;
-    const int tid = threadIdx.x;
-    const uint32_t nbig = state[2];
+    const uint32_t n = state[6];
     uint32_t issued = 0;
-    for (;;) {
-        if (tid == 0) s_e = atomicAdd(&state[5], 1u);
-        __syncthreads();
-        const uint32_t e = s_e;
-        __syncthreads();
-        if (e >= nbig) break;
-        const uint32_t r = big[e];
-        const BatchView& bv = views[cview[r]];
-        const SplatRecord rec = load_record(recs, cidx[r]);
-        const uint32_t p0 = coff[r] - bv.base, w = ew[r];
+    for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
+        const uint2 it = big[e];
+        const BatchView& bv = views[cview[it.x]];
+        const SplatRecord rec = load_record(recs, cidx[it.x]);
+        const uint32_t p0 = coff[it.x] - bv.base;
+        const uint32_t w = min(entry_points(coff, it.x, bv.ebase + bv.valid, bv.base + bv.total, bv.base + bv.points),
+                               it.y + GPS_BIG_SLICE);
         const uint32_t seed = bv.f.frame_seed + 1u;
         int last = -1;  // one Gaussian throughout
-        for (uint32_t k = (uint32_t)tid; k < w; k += 256u)
+        for (uint32_t k = it.y + threadIdx.x; k < w; k += 256u)
             issued += splat_point(rec, p0 + k, seed, bv.f.Ki, bv.f.spp, bv.f.up_w, bv.f.unbiased, fb + bv.fb_offset,
                                   last);
     }
@@ -2692,6 +2693,7 @@ __global__ __launch_bounds__(256) void materialize_indices_kernel(const uint32_t
 
 __global__ __launch_bounds__(256) void batch_clear_kernel(const BatchView* __restrict__ views, uint4* __restrict__ fb) {
     const BatchView& bv = views[blockIdx.y];
+    if (bv.bg.nregions != 0u) return;  // cleared with the binned lists, as far as needed
     const uint64_t n2 = bv.fb_words / 2;
     const uint64_t value = bv.background;
     const uint4 v = make_uint4((uint32_t)value, (uint32_t)(value >> 32), (uint32_t)value, (uint32_t)(value >> 32));
@@ -2742,7 +2744,7 @@ __global__ __launch_bounds__(256) void batch_preprocess_kernel(DevScene s, const
                                                                SplatRecord* __restrict__ recs,
                                                                uint32_t* __restrict__ tile_sum,
                                                                uint32_t* __restrict__ tile_cnt, CullView cv,
-                                                               uint32_t mask_stride) {
+                                                               uint32_t mask_stride, uint2* __restrict__ bounds) {
     __shared__ uint32_t s_sum[GPS_BATCH_MAX_VIEWS], s_cnt[GPS_BATCH_MAX_VIEWS];
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t tile = blockIdx.x;
@@ -2764,7 +2766,9 @@ __global__ __launch_bounds__(256) void batch_preprocess_kernel(DevScene s, const
                 const uint32_t blk = g / cv.gpb;
                 const bool culled = f.hier && mask_bit(cv.mask + (uint64_t)v * mask_stride, blk);
                 if (!culled) {
-                    n = preprocess_one<FORMAT, DEG>(s, f, g, nullptr, no_hiz, recs + (uint64_t)v * npad + g);
+                    const uint64_t i = (uint64_t)v * npad + g;
+                    n = preprocess_one<FORMAT, DEG>(s, f, g, nullptr, no_hiz, recs + i,
+                                                    bounds && views[v].write_bounds ? bounds + i : nullptr);
                     weights[(uint64_t)v * npad + g] = n;
                 }
             }
@@ -2854,6 +2858,12 @@ __global__ __launch_bounds__(THREADS) void batch_splat_kernel(const SplatRecord*
     const uint32_t seg_hi = (uint32_t)(((uint64_t)nchunks * (xcd + 1)) / nx);
     for (uint32_t c = seg_lo + blockIdx.x / nx; c < seg_hi; c += per_xcd) {
         const uint32_t r_lo = chunk_start[c];
+        if (bin_ran) {
+            // a chunk inside one binned view: nothing to do here
+            const uint32_t r_hi = c + 1u < nchunks ? chunk_start[c + 1u] : V - 1u;
+            const int v = cview[r_lo];
+            if (v == (int)cview[r_hi] && views[v].bg.nregions != 0u && views[v].points <= views[v].dense_points) continue;
+        }
         for (int j = tid; j <= CHUNK; j += THREADS) {
             const uint32_t r = r_lo + (uint32_t)j;
             s_off[j] = r < V ? coff[r] : 0xFFFFFFFFu;
@@ -2924,15 +2934,15 @@ static void launch_pre(const PreprocessArgs& a, hipStream_t st) {
     if (a.rejects)  // reject-reason counters: the work-list kernel (same outputs) with counting
         hipLaunchKernelGGL((preprocess_kernel<FORMAT, DEG, true>), dim3(blocks), dim3(GPS_PRE_THREADS), 0, st,
                            a.scene, a.f, a.maskA, a.maskB, a.iteration, a.weights, a.recs, a.tile_sum, a.tile_cnt,
-                           a.cull, a.hiz, a.gocc, a.rejects, a.wg_live);
+                           a.cull, a.hiz, a.gocc, a.rejects, a.wg_live, a.bounds);
     else if (a.f.hier || a.f.occl)  // culled frames: work lists keep the later phases on full waves
         hipLaunchKernelGGL((preprocess_kernel<FORMAT, DEG, false>), dim3(blocks), dim3(GPS_PRE_THREADS), 0, st,
                            a.scene, a.f, a.maskA, a.maskB, a.iteration, a.weights, a.recs, a.tile_sum, a.tile_cnt,
-                           a.cull, a.hiz, a.gocc, nullptr, a.wg_live);
+                           a.cull, a.hiz, a.gocc, nullptr, a.wg_live, a.bounds);
     else
         hipLaunchKernelGGL((preprocess_flat_kernel<FORMAT, DEG>), dim3(blocks), dim3(GPS_PRE_THREADS), 0, st,
                            a.scene, a.f, a.maskA, a.maskB, a.iteration, a.weights, a.recs, a.tile_sum, a.tile_cnt,
-                           a.cull, a.hiz);
+                           a.cull, a.hiz, a.bounds);
 }
 
 void launch_preprocess(const PreprocessArgs& a, hipStream_t st) {
@@ -2989,9 +2999,20 @@ void launch_distribute(const DistributeArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(tile_scan_kernel, dim3(tile_scan_grid(a.ntiles)), dim3(1024), 0, st, a.tile_sum, a.tile_cnt,
                        a.ntiles, a.tile_off, a.tile_voff, a.ctr, a.budget, a.iteration);
     if (a.ntiles == 0) return;
-    hipLaunchKernelGGL(distribute_kernel, dim3(a.ntiles), dim3(256), 0, st, a.weights, a.tile_off, a.tile_voff,
+    BinCount bc{};
+    if (a.bin) {
+        bc.f.g = a.bin->g;
+        bc.f.bounds = a.bin->bounds;
+        bc.f.recs = a.bin->recs;
+        bc.dense_points = a.bin->dense_points;
+        bc.reg_pts = a.bin->reg_pts;
+        bc.big = a.bin->big;
+        bc.state = a.bin->state;
+    }
+    hipLaunchKernelGGL(a.bin ? distribute_kernel<true> : distribute_kernel<false>, dim3(a.ntiles), dim3(256),
+                       a.bin ? a.bin->g.nregions * sizeof(uint32_t) : 0, st, a.weights, a.tile_off, a.tile_voff,
                        a.ntiles, a.ctr, a.cidx, a.coff, a.chunk_start, a.cull, a.hier, a.N, a.ntiles, 0u, 0u,
-                       (uint8_t*)nullptr, GPS_SPLAT_CHUNK_SHIFT, a.tile_sum, a.tile_cnt);
+                       (uint8_t*)nullptr, GPS_SPLAT_CHUNK_SHIFT, a.tile_sum, a.tile_cnt, bc);
 }
 
 void launch_ordered_splat(const OrderedArgs& a, hipStream_t st) {
@@ -3009,16 +3030,18 @@ void launch_ordered_splat(const OrderedArgs& a, hipStream_t st) {
     gate.up_h = (uint32_t)a.up_h;
     gate.forced = a.forced;
     unsigned long long* fb = reinterpret_cast<unsigned long long*>(s.fb);
+    const uint32_t* only_if = s.bin_state ? s.bin_state + 3 : nullptr;  // the binned splat stood down
+    const BigSlices big{s.big, s.bin_state};
     hipLaunchKernelGGL(ord_key_kernel, dim3(a.cus), dim3(256), 0, st, s.recs, s.cidx, s.chunk_start, s.ctr, gate,
-                       s.only_if, a.bucket, a.hist);
-    hipLaunchKernelGGL(ord_scan_kernel, dim3(1), dim3(1024), 0, st, s.ctr, gate, s.only_if, a.hist, a.lim);
+                       only_if, a.bucket, a.hist);
+    hipLaunchKernelGGL(ord_scan_kernel, dim3(1), dim3(1024), 0, st, s.ctr, gate, only_if, a.hist, a.lim);
     for (int ph = 0; ph < GPS_ORD_PHASES; ++ph) {
         const bool test = ph > 0 || a.pre_test;
         if (test)
             hipLaunchKernelGGL(ord_tile_max_kernel, dim3((a.ntiles + 3u) / 4u), dim3(256), 0, st,
-                               (const unsigned long long*)fb, a.tmax, a.ntiles, s.spp, s.ctr, gate, s.only_if);
+                               (const unsigned long long*)fb, a.tmax, a.ntiles, s.spp, s.ctr, gate, only_if);
         hipLaunchKernelGGL(splat_ordered_kernel, dim3(s.grid), dim3(GPS_SPLAT_THREADS), 0, st, s.recs, s.cidx, s.coff,
-                           s.chunk_start, s.ctr, fb, sc, s.atomics_count, s.only_if, (const uint16_t*)a.bucket,
+                           s.chunk_start, s.ctr, fb, sc, s.atomics_count, big, (const uint16_t*)a.bucket,
                            (const uint32_t*)a.lim, (const uint32_t*)a.tmax, a.tw64, ph, test ? 1 : 0, gate,
                            a.skipped_count);
     }
@@ -3034,7 +3057,7 @@ void launch_splat(const SplatArgs& a, hipStream_t st) {
     sc.xcds = a.xcds;
     hipLaunchKernelGGL(splat_kernel, dim3(a.grid), dim3(GPS_SPLAT_THREADS), 0, st, a.recs, a.cidx, a.coff,
                        a.chunk_start, a.ctr, reinterpret_cast<unsigned long long*>(a.fb), sc, a.atomics_count,
-                       a.only_if);
+                       BigSlices{a.big, a.bin_state});
 }
 
 template <int SS, int SPP>
@@ -3156,7 +3179,7 @@ template <int FORMAT, int DEG> static void launch_batch_pre_t(const BatchArgs& a
     const int vpw = a.pre_views > 0 && a.pre_views < a.nviews ? a.pre_views : a.nviews;
     hipLaunchKernelGGL((batch_preprocess_kernel<FORMAT, DEG>), dim3(a.tiles_per_view, (a.nviews + vpw - 1) / vpw),
                        dim3(256), 0, st, a.scene, a.views, a.nviews, vpw, a.npad, a.tiles_per_view, a.weights, a.recs,
-                       a.tile_sum, a.tile_cnt, a.cull, a.mask_stride);
+                       a.tile_sum, a.tile_cnt, a.cull, a.mask_stride, a.bin.any ? a.bin.bounds : nullptr);
 }
 
 void launch_batch_preprocess(const BatchArgs& a, hipStream_t st) {
@@ -3187,10 +3210,21 @@ void launch_batch_distribute(const BatchArgs& a, hipStream_t st) {
     if (ntiles == 0) return;
     uint32_t shift = 0;
     while ((1u << shift) < (uint32_t)(a.threads * a.ppt)) ++shift;
-    hipLaunchKernelGGL(distribute_kernel, dim3(ntiles), dim3(256), 0, st, (const uint32_t*)a.weights,
+    BinCount bc{};
+    if (a.bin.any) {
+        launch_zero_u32(a.bin.state, 8, st);
+        bc.f.bounds = a.bin.bounds;
+        bc.f.recs = a.recs;
+        bc.views = a.views;
+        bc.reg_pts = a.bin.reg_pts;
+        bc.big = a.bin.big;
+        bc.state = a.bin.state;
+    }
+    hipLaunchKernelGGL(a.bin.any ? distribute_kernel<true> : distribute_kernel<false>, dim3(ntiles), dim3(256),
+                       a.bin.any ? a.bin.max_view_regions * sizeof(uint32_t) : 0, st, (const uint32_t*)a.weights,
                        (const uint32_t*)a.tile_off, (const uint32_t*)a.tile_voff, ntiles, (const PassCounters*)a.ctr,
                        a.cidx, a.coff, a.chunk_start, a.cull, a.hier, a.scene.N, a.tiles_per_view, a.npad,
-                       a.mask_stride, a.cview, shift, a.tile_sum, a.tile_cnt);
+                       a.mask_stride, a.cview, shift, a.tile_sum, a.tile_cnt, bc);
 }
 
 template <int THREADS, int PPT> static void launch_batch_splat_t(const BatchArgs& a, hipStream_t st) {
@@ -3224,34 +3258,19 @@ bool launch_batch_splat(const BatchArgs& a, hipStream_t st) {
 void launch_batch_binned(const BatchArgs& a, hipStream_t st) {
     const BatchBinArgs& b = a.bin;
     if (!b.any) return;
-    launch_zero_u32(b.state, 8, st);
-    uint32_t gx = (b.cus * 4u + (uint32_t)a.nviews - 1u) / (uint32_t)a.nviews;  // workgroups per view
-    if (gx < 2u) gx = 2u;
-    const size_t hist = 2u * b.max_view_regions * sizeof(uint32_t);
-    hipLaunchKernelGGL(batch_bin_count_kernel, dim3(gx, a.nviews), dim3(256), hist, st, (const SplatRecord*)a.recs,
-                       (const uint32_t*)a.cidx, (const uint32_t*)a.coff, (const BatchView*)a.views, b.erect, b.ew,
-                       b.reg_cnt, b.reg_pts, b.big, b.state);
-    BinGeom all{};
-    all.nregions = b.nregions;
-    hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, st, all, b.reg_cnt, b.reg_pts, b.reg_ecnt, b.reg_ptot,
-                       b.reg_eoff, b.reg_poff, b.reg_cursor, b.reg_jobs, b.job_reg, b.job_p0, b.state, b.list_cap,
-                       b.job_points, b.job_cap, (const PassCounters*)nullptr, 0xFFFFFFFFu);
-    hipLaunchKernelGGL(batch_bin_scatter_kernel, dim3(gx, a.nviews), dim3(256), hist, st, (const BatchView*)a.views,
-                       (const uint2*)b.erect, (const uint32_t*)b.ew, b.reg_cursor, b.list, b.lw,
-                       (const uint32_t*)b.state);
-    const uint32_t grid = b.cus * 4u;
-    hipLaunchKernelGGL(bin_tile_sum_kernel, dim3(grid), dim3(256), 0, st, (const uint32_t*)b.lw,
-                       (const uint32_t*)b.state, b.tsum);
-    hipLaunchKernelGGL(bin_tiles_scan_kernel, dim3(1), dim3(1024), 0, st, (const uint32_t*)b.tsum,
-                       (const uint32_t*)b.state, b.toff);
-    hipLaunchKernelGGL(bin_local_scan_kernel, dim3(grid), dim3(256), 0, st, (const uint32_t*)b.lw,
-                       (const uint32_t*)b.state, (const uint32_t*)b.toff, b.lpre);
+    const uint32_t gx = std::max(2u, (b.cus * GPS_LIST_WGS_PER_CU + b.views - 1u) / b.views);  // workgroups per view
+    const size_t hist = b.max_view_regions * sizeof(uint32_t);
+    const BinFrame f{a.cidx, a.coff, b.bounds, a.recs, BinGeom{}, 0u, 0u, 0u, 0u};
+    hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, st, b.nregions, b.reg_pts, b.reg_ptot, b.reg_poff,
+                       b.reg_cursor, b.job_reg, b.job_p0, b.state, b.list_cap, b.cus, b.job_cap,
+                       (const PassCounters*)nullptr, 0xFFFFFFFFu);
+    hipLaunchKernelGGL(batch_bin_scatter_kernel, dim3(gx, a.nviews), dim3(GPS_LIST_THREADS), hist, st, f,
+                       (const BatchView*)a.views, b.reg_cursor, b.list, (const uint32_t*)b.state,
+                       (const uint32_t*)b.reg_ptot, reinterpret_cast<unsigned long long*>(a.fb));
     hipLaunchKernelGGL(batch_bin_splat_kernel, dim3(b.cus), dim3(GPS_BIN_THREADS), 0, st, (const SplatRecord*)a.recs,
-                       (const uint32_t*)a.cidx, (const uint32_t*)a.coff, (const uint32_t*)b.list,
-                       (const uint32_t*)b.lpre, (const uint32_t*)b.reg_ecnt, (const uint32_t*)b.reg_ptot,
-                       (const uint32_t*)b.reg_eoff, (const uint32_t*)b.reg_poff, (const uint32_t*)b.reg_jobs,
+                       (const uint2*)b.list, (const uint32_t*)b.reg_ptot, (const uint32_t*)b.reg_poff,
                        (const uint32_t*)b.job_reg, (const uint32_t*)b.job_p0, b.state, (const BatchView*)a.views,
-                       a.nviews, reinterpret_cast<unsigned long long*>(a.fb), b.job_points, a.atomics);
+                       a.nviews, reinterpret_cast<unsigned long long*>(a.fb), a.atomics);
 }
 
 void launch_batch_bin_big(const BatchArgs& a, hipStream_t st) {
@@ -3259,47 +3278,48 @@ void launch_batch_bin_big(const BatchArgs& a, hipStream_t st) {
     if (!b.any) return;
     hipLaunchKernelGGL(batch_bin_big_kernel, dim3(b.cus * 4u), dim3(256), 0, st, (const SplatRecord*)a.recs,
                        (const uint32_t*)a.cidx, (const uint32_t*)a.coff, (const uint8_t*)a.cview,
-                       (const uint32_t*)b.ew, (const uint32_t*)b.big, b.state, (const BatchView*)a.views,
+                       (const uint2*)b.big, (const uint32_t*)b.state, (const BatchView*)a.views,
                        reinterpret_cast<unsigned long long*>(a.fb), a.atomics);
 }
 
 // ------------------------------------------------------------------ binned splat launcher
 void launch_binned_splat(const BinnedArgs& a, hipStream_t st) {
-    launch_zero_u32(a.state, 8, st);
-    const uint32_t grid = a.cus * 4u;
-    const size_t hist = 2u * a.g.nregions * sizeof(uint32_t);
-    hipLaunchKernelGGL(bin_count_kernel, dim3(grid), dim3(256), hist, st, a.recs, a.cidx, a.coff, a.ctr, a.g, a.erect,
-                       a.ew, a.reg_cnt, a.reg_pts, a.big, a.state, a.dense_points);
-    hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, st, a.g, a.reg_cnt, a.reg_pts, a.reg_ecnt, a.reg_ptot,
-                       a.reg_eoff, a.reg_poff, a.reg_cursor, a.reg_jobs, a.job_reg, a.job_p0, a.state, a.list_cap,
-                       a.job_points, a.job_cap, a.ctr, a.dense_points);
-    hipLaunchKernelGGL(bin_scatter_kernel, dim3(grid), dim3(256), hist, st, a.ctr, a.g, (const uint2*)a.erect,
-                       (const uint32_t*)a.ew, a.reg_cursor, a.list, a.lw, (const uint32_t*)a.state);
-    hipLaunchKernelGGL(bin_tile_sum_kernel, dim3(grid), dim3(256), 0, st, (const uint32_t*)a.lw,
-                       (const uint32_t*)a.state, a.tsum);
-    hipLaunchKernelGGL(bin_tiles_scan_kernel, dim3(1), dim3(1024), 0, st, (const uint32_t*)a.tsum,
-                       (const uint32_t*)a.state, a.toff);
-    hipLaunchKernelGGL(bin_local_scan_kernel, dim3(grid), dim3(256), 0, st, (const uint32_t*)a.lw,
-                       (const uint32_t*)a.state, (const uint32_t*)a.toff, a.lpre);
+    const size_t hist = a.g.nregions * sizeof(uint32_t);
+    const BinFrame f{a.cidx, a.coff, a.bounds, a.recs, a.g, 0u, 0u, 0u, 0u};
+    hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, st, a.g.nregions, a.reg_pts, a.reg_ptot, a.reg_poff,
+                       a.reg_cursor, a.job_reg, a.job_p0, a.state, a.list_cap, a.cus, a.job_cap, a.ctr,
+                       a.dense_points);
+    hipLaunchKernelGGL(bin_scatter_kernel, dim3(a.cus * GPS_LIST_WGS_PER_CU), dim3(GPS_LIST_THREADS), hist, st, f,
+                       a.ctr, a.reg_cursor, a.list, (const uint32_t*)a.state, (const uint32_t*)a.reg_ptot,
+                       reinterpret_cast<unsigned long long*>(a.fb), a.clear_words, a.background);
     BinSplat b;
     b.g = a.g;
     b.K = a.sc.K;
-    b.unbiased = a.sc.unbiased;
     b.frame_seed = a.sc.frame_seed;
     b.background = a.background;
-    hipLaunchKernelGGL(bin_splat_kernel, dim3(a.cus), dim3(GPS_BIN_THREADS), 0, st, a.recs, a.cidx, a.coff,
-                       (const uint32_t*)a.list, (const uint32_t*)a.lpre, (const uint32_t*)a.reg_ecnt,
-                       (const uint32_t*)a.reg_ptot, (const uint32_t*)a.reg_eoff, (const uint32_t*)a.reg_poff,
-                       (const uint32_t*)a.reg_jobs, (const uint32_t*)a.job_reg, (const uint32_t*)a.job_p0, a.state,
-                       reinterpret_cast<unsigned long long*>(a.fb), b, a.job_points, a.atomics_count);
-    hipLaunchKernelGGL(bin_big_kernel, dim3(grid), dim3(256), 0, st, a.recs, a.cidx, a.coff, (const uint32_t*)a.ew,
-                       (const uint32_t*)a.big, a.state, reinterpret_cast<unsigned long long*>(a.fb), a.sc,
+    b.fresh = a.fresh;
+    hipLaunchKernelGGL(bin_splat_kernel, dim3(a.cus), dim3(GPS_BIN_THREADS), 0, st, a.recs, (const uint2*)a.list,
+                       (const uint32_t*)a.reg_ptot, (const uint32_t*)a.reg_poff, (const uint32_t*)a.job_reg,
+                       (const uint32_t*)a.job_p0, a.state, reinterpret_cast<unsigned long long*>(a.fb), b,
                        a.atomics_count);
 }
 
-uint32_t binned_dense_points(int up_w, int up_h, int K) {
-    const uint64_t p = (uint64_t)GPS_BIN_DENSE_SAMPLES * (uint64_t)up_w * (uint64_t)up_h / (uint64_t)(K > 0 ? K : 1);
+uint32_t binned_dense_points(int up_w, int up_h, int spp, int K, bool batch) {
+    const uint64_t px = (uint64_t)up_w * (uint64_t)up_h, words = px * (uint64_t)spp;
+    uint64_t dense = GPS_BIN_DENSE_SAMPLES;
+    if (batch)
+        dense = words > GPS_BIN_LARGE_FB_BATCH ? GPS_BIN_DENSE_LARGE : dense;
+    else
+        dense = std::min<uint64_t>(std::max<uint64_t>(dense, 6 * words / GPS_BIN_LARGE_FB), GPS_BIN_DENSE_LARGE);
+    const uint64_t p = dense * px / (uint64_t)(K > 0 ? K : 1);
     return p < 0xFFFFFFFFull ? (uint32_t)p : 0xFFFFFFFFu;
+}
+
+bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool batch) {
+    const uint64_t words = (uint64_t)up_w * (uint64_t)up_h * (uint64_t)spp;
+    return K * spp >= GPS_BIN_AUTO_SAMPLES ||
+           (K * spp >= GPS_BIN_AUTO_SAMPLES_LARGE && words > (batch ? GPS_BIN_LARGE_FB_BATCH : GPS_BIN_LARGE_FB) &&
+            16ull * N >= words);
 }
 
 bool binned_geometry(int up_w, int up_h, int spp, BinGeom* g) {

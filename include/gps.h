@@ -140,7 +140,7 @@ typedef struct gps_stats {
     uint64_t num_blocks;           /* culling blocks (0 when block culling is off) */
     int32_t splat_binned;          /* 1: the last pass used the binned splat */
     int32_t splat_fallback;        /* the point-parallel splat ran instead: 1 region lists overflowed,
-                                      2 more than 8 samples per framebuffer word (GPS_SPLAT_AUTO) */
+                                      2 too many samples per framebuffer word (GPS_SPLAT_AUTO) */
     uint32_t bin_entries;          /* (Gaussian, region) pairs of the last pass */
     uint32_t bin_jobs;             /* region jobs of the last pass */
     uint32_t bin_big;              /* Gaussians splatted with global atomics (too many regions) */
@@ -202,15 +202,19 @@ gps_status gps_encode_quantized(const gps_scene_desc* desc, const gps_quantized_
 gps_status gps_pass_create(const gps_render_settings* settings, gps_scene* scene, gps_pass** out);
 void gps_pass_destroy(gps_pass* pass);
 /* Splat kernel choice.  GPS_SPLAT_BINNED: screen regions rendered in LDS,
- * no per-sample global atomics (spp <= 4, at most 8192 regions per frame,
- * else point-parallel).  GPS_SPLAT_POINT_PARALLEL: one 64-bit global
- * atomicMin per accepted sample.  GPS_SPLAT_AUTO (default): binned when a
- * point has at least 8 samples (K * spp) and the pass has at most 8 samples
- * per framebuffer word (points * K <= 8 * upscaled width * height, tested on
- * the device after the point count; denser passes splat point-parallel and
- * report gps_stats.splat_fallback = 2).  All give the same framebuffer bit
- * for bit.  No reference counterpart (the reference has only the
- * point-parallel form, gaussian_point_splatting.cu:383-432). */
+ * no per-sample global atomics (spp <= 4, at most 8192 regions per frame, the
+ * pass's point lists long enough, else point-parallel).
+ * GPS_SPLAT_POINT_PARALLEL: one 64-bit global atomicMin per accepted sample.
+ * GPS_SPLAT_AUTO (default): binned when a point has at least 8 samples (K *
+ * spp) and the pass has at most 8 samples per framebuffer word (points * K <=
+ * 8 * upscaled width * height, tested on the device after the point count;
+ * denser passes splat point-parallel and report gps_stats.splat_fallback = 2).
+ * Framebuffers of more than 2^22 words (upscaled width * height * spp; 2^20 in
+ * a batch) take wider limits: 4 samples per point if the scene has a Gaussian
+ * per 16 words, and 6 samples per word for every 2^22 words, up to 32 (32 in a
+ * batch).  All give the same framebuffer bit for bit.  No reference counterpart
+ * (the reference has only the point-parallel form,
+ * gaussian_point_splatting.cu:383-432). */
 #define GPS_SPLAT_AUTO 0
 #define GPS_SPLAT_POINT_PARALLEL 1
 #define GPS_SPLAT_BINNED 2
@@ -559,9 +563,10 @@ gps_status gps_batch_set_tuning(gps_batch* batch, const gps_batch_tuning* tuning
 /* Splat form per view, with the rule and modes of gps_pass_set_splat_mode:
  * the binned views of a batch share one set of binning launches (regions of
  * all of them in one job queue), the rest use the point-parallel batch
- * splat.  The binned buffers (16 B per compacted entry, 12 B per list slot,
- * about 1.5 slots per entry) are allocated on the first batch that bins a
- * view; if that allocation fails every view stays point-parallel.  No
+ * splat.  The binned buffers (16 B per compacted entry; 8 B per listed point,
+ * sized by the views, grown by a later batch that needs more) are allocated
+ * on the first batch that bins a view; if an allocation fails every view
+ * stays point-parallel.  No
  * reference counterpart. */
 gps_status gps_batch_set_splat_mode(gps_batch* batch, int32_t mode);
 /* Counters of view `view` of the last batch (atomics, bin_entries, bin_jobs,

@@ -1,0 +1,64 @@
+"""The binned splat at the edges of its lists, regions and jobs, bit for bit
+against the point-parallel splat (which the oracle's frames pin)."""
+import numpy as np
+import pytest
+
+import helpers as H
+from helpers import assert_same, flush
+
+pytestmark = pytest.mark.gpu
+
+
+def _frames(gpu, arrays, w, h, ss, spp, eye, modes, gpb=0, **kw):
+    st = gpu.RenderSettings(w, h, spp, ss, gaussians_per_block=gpb)
+    f = gpu.frame_params(eye, (0, 0, 0), (0, 1, 0), 45.0, w, h, ss=ss, frame=3, spp=spp, background=(0.2, 0.4, 0.6),
+                         **kw)
+    out = []
+    for mode in modes:
+        flush(f"{w}x{h} ss {ss} spp {spp} n {arrays.n} mode {mode}")
+        r = H.GpuRunner(arrays, st)
+        r.p.set_splat_mode(mode)
+        out.append(r.render(f, [gpu.DBG_FRAMEBUFFER]))
+    return out
+
+
+def _same(gpu, a, b, what):
+    assert_same(f"{what} fb", a.debug[gpu.DBG_FRAMEBUFFER], b.debug[gpu.DBG_FRAMEBUFFER])
+    assert_same(f"{what} colour", a.color, b.color)
+    assert_same(f"{what} depth", a.depth, b.depth)
+
+
+# one pixel, a region less one pixel, a region, a region and one pixel, ragged tiles
+@pytest.mark.parametrize("spp", [1, 2, 3, 4])
+@pytest.mark.parametrize("size", [(1, 1), (127, 63), (128, 64), (129, 65), (333, 190)])
+def test_binned_region_edges(gpu, size, spp):
+    """Regions cut by the screen, regions without a point (cleared with the
+    lists) and regions of one and of several jobs."""
+    w, h = size
+    arrays = H.scene(0x5EED0801 + spp, 9_000, dict(H.C1, half_extent=4.0, log_scale_mu=-2.5)).morton_sorted()
+    a, b = _frames(gpu, arrays, w, h, 1, spp, (0.0, 3.0, -25.0), (gpu.Pass.SPLAT_BINNED, gpu.Pass.SPLAT_POINT_PARALLEL))
+    assert a.stats["splat_binned"] == 1 and a.stats["splat_fallback"] == 0, a.stats
+    _same(gpu, a, b, f"{size} spp {spp}")
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 4097])
+def test_binned_big_gaussians(gpu, n):
+    """Gaussians over more than four regions (their points in slices of 1024,
+    splatted after the regions), alone and beside small ones."""
+    arrays = H.scene(0x5EED0811, n, dict(H.C1, half_extent=3.0, log_scale_mu=-3.0)).morton_sorted()
+    k = max(1, n // 50)
+    arrays.scales[:k] = np.float32(1.5)
+    arrays.opacities[:k] = np.float32(0.7)
+    a, b = _frames(gpu, arrays, 640, 360, 2, 4, (0.0, 1.0, -9.0), (gpu.Pass.SPLAT_BINNED, gpu.Pass.SPLAT_POINT_PARALLEL))
+    assert a.stats["splat_fallback"] == 0 and a.stats["bin_big"] >= 1, a.stats
+    assert a.stats["num_points"][0] > 1024
+    _same(gpu, a, b, f"{n} Gaussians")
+
+
+def test_binned_auto_large_framebuffer(gpu):
+    """More than 2^22 framebuffer words: 4 samples a point are binned too, and
+    passes of up to 6 samples per word and 2^22 words."""
+    arrays = H.scene(0x5EED0821, 400_000, dict(H.C1, half_extent=8.0)).morton_sorted()
+    a, b = _frames(gpu, arrays, 1400, 780, 2, 1, (0.0, 3.0, -25.0), (gpu.Pass.SPLAT_AUTO, gpu.Pass.SPLAT_POINT_PARALLEL))
+    assert a.stats["splat_binned"] == 1 and a.stats["splat_fallback"] == 0, a.stats
+    _same(gpu, a, b, "large framebuffer")
