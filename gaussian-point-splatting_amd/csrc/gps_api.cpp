@@ -943,6 +943,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
         sa.frame_seed = frame_seed + 1u;
         sa.grid = p->splat_grid;
         sa.xcds = p->xcds;
+        if (fold_tiles(p->ntiles)) sa.sums = TileSums{p->tile_sum, p->tile_cnt, p->ntiles, &p->ctr->iteration};
         stage_mark(p, 4, slot, 0, st);
         p->last_binned = binned ? 1 : 0;
         if (binned) {

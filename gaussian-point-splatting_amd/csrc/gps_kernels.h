@@ -45,6 +45,14 @@ struct DistributeArgs {
     uint32_t N;
 };
 
+// The tile sums of a pass without a scan launch, for the splat kernel to clear
+// (n = 0: the pass had one, distribute_kernel has cleared them).
+struct TileSums {
+    uint32_t *sum, *cnt;
+    uint32_t n;
+    uint32_t* iteration;
+};
+
 struct SplatArgs {
     const SplatRecord* recs;
     const uint32_t* cidx;
@@ -61,6 +69,7 @@ struct SplatArgs {
     // (bin_state[3] == 0) only its big slices are splatted
     const uint32_t* bin_state = nullptr;
     const uint2* big = nullptr;
+    TileSums sums{};
 };
 
 // Ordered point-parallel splat (dense passes, GPS_ORD_BINS): the splat

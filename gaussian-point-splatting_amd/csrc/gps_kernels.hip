@@ -922,7 +922,8 @@ __global__ __launch_bounds__(GPS_PRE_THREADS) void preprocess_flat_kernel(
 // takes its carry by reducing the raw sums of steps 0 .. s-1 itself, so no
 // workgroup waits for another (sums are modulo 2^32, as a sequential scan's).
 // The tile sums are cleared for the next pass by distribute_kernel, which
-// runs after this kernel on every tile.
+// runs after this kernel on every tile.  A pass of at most GPS_FOLD_TILES tiles
+// does without this launch (distribute_kernel's `fold`).
 __global__ __launch_bounds__(1024) void tile_scan_kernel(const uint32_t* __restrict__ tile_sum,
                                                          const uint32_t* __restrict__ tile_cnt, uint32_t ntiles,
                                                          uint32_t* __restrict__ tile_off,
@@ -1104,26 +1105,72 @@ template <bool BIN>
 __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restrict__ weights,
                                                          const uint32_t* __restrict__ tile_off,
                                                          const uint32_t* __restrict__ tile_voff, uint32_t ntiles,
-                                                         const PassCounters* __restrict__ ctr, uint32_t* __restrict__ cidx,
+                                                         PassCounters* __restrict__ ctr, uint32_t* __restrict__ cidx,
                                                          uint32_t* __restrict__ coff, uint32_t* __restrict__ chunk_start,
                                                          CullView cv, int hier, uint32_t N, uint32_t tiles_per_view,
                                                          uint32_t npad, uint32_t mask_stride,
                                                          uint8_t* __restrict__ cview, uint32_t chunk_shift,
                                                          uint32_t* __restrict__ tile_sum, uint32_t* __restrict__ tile_cnt,
-                                                         BinCount bc) {
+                                                         BinCount bc, int fold, uint32_t budget) {
     extern __shared__ uint32_t s_pts[];  // BIN: the regions of the frame, or of the batch's largest view
     __shared__ uint32_t s_a[4], s_c[4];
+    __shared__ uint4 s_fold[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t tile = blockIdx.x;
-    if (tid == 0) {  // the scan has consumed them: clear for the next pass
-        tile_sum[tile] = 0u;
-        tile_cnt[tile] = 0u;
+    uint32_t v0, vend, a0;
+    uint64_t P;
+    if (fold) {
+        // few tiles: every workgroup adds up the sums before its own and all of
+        // them, and the last one publishes the totals (sums modulo 2^32)
+        constexpr int PER = GPS_FOLD_TILES / 256u;
+        uint32_t xs[PER], xc[PER];
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const uint32_t i = (uint32_t)k * 256u + (uint32_t)tid, ic = min(i, ntiles - 1u);
+            const uint32_t x = tile_sum[ic], y = tile_cnt[ic];
+            xs[k] = i < ntiles ? x : 0u;
+            xc[k] = i < ntiles ? y : 0u;
+        }
+        uint4 t = make_uint4(0u, 0u, 0u, 0u);  // points, valid: before this tile, of all
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const bool before = (uint32_t)k * 256u + (uint32_t)tid < tile;
+            t.x += before ? xs[k] : 0u;
+            t.y += before ? xc[k] : 0u;
+            t.z += xs[k];
+            t.w += xc[k];
+        }
+        t = make_uint4(wave_reduce_add(t.x), wave_reduce_add(t.y), wave_reduce_add(t.z), wave_reduce_add(t.w));
+        if (lane == 0) s_fold[wave] = t;
+        const uint32_t own = tile_cnt[tile];
+        __syncthreads();
+        t = s_fold[0];
+        for (int q = 1; q < 4; ++q) {
+            const uint4 o = s_fold[q];
+            t = make_uint4(t.x + o.x, t.y + o.y, t.z + o.z, t.w + o.w);
+        }
+        a0 = t.x;
+        v0 = t.y;
+        vend = v0 + own;
+        const uint32_t p32 = min(t.z, budget);
+        P = p32;
+        if (tile + 1u == ntiles && tid == 0) {
+            ctr->total = t.z;
+            ctr->valid = t.w;
+            ctr->points = p32;
+            ctr->chunks = (uint32_t)(((uint64_t)p32 + GPS_SPLAT_CHUNK - 1) / GPS_SPLAT_CHUNK);
+        }
+    } else {
+        if (tid == 0) {  // the scan has consumed them: clear for the next pass
+            tile_sum[tile] = 0u;
+            tile_cnt[tile] = 0u;
+        }
+        // The workgroup's offsets and the pass totals are read up front, together.
+        v0 = tile_voff[tile];
+        vend = tile + 1 < ntiles ? tile_voff[tile + 1] : ctr->valid;
+        a0 = tile_off[tile];
+        P = ctr->points;
     }
-    // The workgroup's offsets and the pass totals are read up front, together.
-    const uint32_t v0 = tile_voff[tile];
-    const uint32_t vend = tile + 1 < ntiles ? tile_voff[tile + 1] : ctr->valid;
-    const uint32_t a0 = tile_off[tile];
-    const uint64_t P = ctr->points;
     if (vend == v0) return;  // uniform over the workgroup
     const uint32_t view = tile / tiles_per_view;
     const uint32_t* cmask = cv.mask + (uint64_t)view * mask_stride;
@@ -1601,6 +1648,19 @@ __device__ __forceinline__ uint32_t splat_big(const BigSlices& b, const SplatRec
     return issued;
 }
 
+// The end of a pass whose distributor took the tile sums without a scan launch
+// (every workgroup read them, so only a later kernel may clear them): clears
+// them for the next pass and flips the mask ping-pong, which the reference does
+// only when the pass produced points (workload_distributor.cu:111-115,144).
+__device__ __forceinline__ void end_sums(const TileSums& t, const PassCounters* __restrict__ ctr) {
+    if (t.n == 0u || blockIdx.x != 0u) return;
+    for (uint32_t i = threadIdx.x; i < t.n; i += blockDim.x) {
+        t.sum[i] = 0u;
+        t.cnt[i] = 0u;
+    }
+    if (threadIdx.x == 0 && ctr->points > 0u) *t.iteration = *t.iteration + 1u;
+}
+
 __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_kernel(const SplatRecord* __restrict__ recs,
                                                                   const uint32_t* __restrict__ cidx,
                                                                   const uint32_t* __restrict__ coff,
@@ -1608,7 +1668,7 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_kernel(const SplatRec
                                                                   const PassCounters* __restrict__ ctr,
                                                                   unsigned long long* __restrict__ fb, SplatConsts sc,
                                                                   uint32_t* __restrict__ atomics_count,
-                                                                  BigSlices big) {
+                                                                  BigSlices big, TileSums sums) {
     __shared__ uint32_t s_off[GPS_SPLAT_CHUNK + 1];
 #if GPS_SPLAT_SLOTS
     __shared__ uint32_t s_key[GPS_SPLAT_SLOTS];
@@ -1617,6 +1677,7 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_kernel(const SplatRec
     uint32_t* const s_key = nullptr;
     unsigned long long* const s_val = nullptr;
 #endif
+    end_sums(sums, ctr);
     if (big.state && big.state[3] == 0u) {  // the binned splat covers this pass
         const uint32_t n = splat_big(big, recs, cidx, coff, ctr, sc, fb);
         if (atomics_count) add_count(atomics_count, n);
@@ -1768,7 +1829,7 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_ordered_kernel(
     const uint32_t* __restrict__ chunk_start, const PassCounters* __restrict__ ctr, unsigned long long* __restrict__ fb,
     SplatConsts sc, uint32_t* __restrict__ atomics_count, BigSlices big,
     const uint16_t* __restrict__ bucket, const uint32_t* __restrict__ lim, const uint32_t* __restrict__ tmax,
-    int tw64, int phase, int test, OrdGate gate, uint32_t* __restrict__ skipped_count) {
+    int tw64, int phase, int test, OrdGate gate, uint32_t* __restrict__ skipped_count, TileSums sums) {
     __shared__ uint32_t s_off[GPS_SPLAT_CHUNK + 1];
 #if GPS_SPLAT_SLOTS
     __shared__ uint32_t s_key[GPS_SPLAT_SLOTS];
@@ -1777,6 +1838,7 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_ordered_kernel(
     uint32_t* const s_key = nullptr;
     unsigned long long* const s_val = nullptr;
 #endif
+    if (phase == 0) end_sums(sums, ctr);
     if (big.state && big.state[3] == 0u) {  // the binned splat covers this pass
         if (phase > 0) return;
         const uint32_t n = splat_big(big, recs, cidx, coff, ctr, sc, fb);
@@ -3065,8 +3127,10 @@ void launch_cull(const CullView& cv, const float planes[24], const Mat4& vp, con
 static uint32_t tile_scan_grid(uint32_t ntiles) { return ntiles ? (ntiles + 8191u) / 8192u : 1u; }
 
 void launch_distribute(const DistributeArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(tile_scan_grid(a.ntiles)), dim3(1024), 0, st, a.tile_sum, a.tile_cnt,
-                       a.ntiles, a.tile_off, a.tile_voff, a.ctr, a.budget, a.iteration);
+    const bool fold = fold_tiles(a.ntiles);
+    if (!fold)
+        hipLaunchKernelGGL(tile_scan_kernel, dim3(tile_scan_grid(a.ntiles)), dim3(1024), 0, st, a.tile_sum, a.tile_cnt,
+                           a.ntiles, a.tile_off, a.tile_voff, a.ctr, a.budget, a.iteration);
     if (a.ntiles == 0) return;
     BinCount bc{};
     if (a.bin) {
@@ -3081,7 +3145,7 @@ void launch_distribute(const DistributeArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(a.bin ? distribute_kernel<true> : distribute_kernel<false>, dim3(a.ntiles), dim3(256),
                        a.bin ? a.bin->g.nregions * sizeof(uint32_t) : 0, st, a.weights, a.tile_off, a.tile_voff,
                        a.ntiles, a.ctr, a.cidx, a.coff, a.chunk_start, a.cull, a.hier, a.N, a.ntiles, 0u, 0u,
-                       (uint8_t*)nullptr, GPS_SPLAT_CHUNK_SHIFT, a.tile_sum, a.tile_cnt, bc);
+                       (uint8_t*)nullptr, GPS_SPLAT_CHUNK_SHIFT, a.tile_sum, a.tile_cnt, bc, fold ? 1 : 0, a.budget);
 }
 
 void launch_ordered_splat(const OrderedArgs& a, hipStream_t st) {
@@ -3112,7 +3176,7 @@ void launch_ordered_splat(const OrderedArgs& a, hipStream_t st) {
         hipLaunchKernelGGL(splat_ordered_kernel, dim3(s.grid), dim3(GPS_SPLAT_THREADS), 0, st, s.recs, s.cidx, s.coff,
                            s.chunk_start, s.ctr, fb, sc, s.atomics_count, big, (const uint16_t*)a.bucket,
                            (const uint32_t*)a.lim, (const uint32_t*)a.tmax, a.tw64, ph, test ? 1 : 0, gate,
-                           a.skipped_count);
+                           a.skipped_count, s.sums);
     }
 }
 
@@ -3126,7 +3190,7 @@ void launch_splat(const SplatArgs& a, hipStream_t st) {
     sc.xcds = a.xcds;
     hipLaunchKernelGGL(splat_kernel, dim3(a.grid), dim3(GPS_SPLAT_THREADS), 0, st, a.recs, a.cidx, a.coff,
                        a.chunk_start, a.ctr, reinterpret_cast<unsigned long long*>(a.fb), sc, a.atomics_count,
-                       BigSlices{a.big, a.bin_state});
+                       BigSlices{a.big, a.bin_state}, a.sums);
 }
 
 template <int SS, int SPP>
@@ -3296,9 +3360,9 @@ void launch_batch_distribute(const BatchArgs& a, hipStream_t st) {
     }
     hipLaunchKernelGGL(a.bin.any ? distribute_kernel<true> : distribute_kernel<false>, dim3(ntiles), dim3(256),
                        a.bin.any ? a.bin.max_view_regions * sizeof(uint32_t) : 0, st, (const uint32_t*)a.weights,
-                       (const uint32_t*)a.tile_off, (const uint32_t*)a.tile_voff, ntiles, (const PassCounters*)a.ctr,
+                       (const uint32_t*)a.tile_off, (const uint32_t*)a.tile_voff, ntiles, a.ctr,
                        a.cidx, a.coff, a.chunk_start, a.cull, a.hier, a.scene.N, a.tiles_per_view, a.npad,
-                       a.mask_stride, a.cview, shift, a.tile_sum, a.tile_cnt, bc);
+                       a.mask_stride, a.cview, shift, a.tile_sum, a.tile_cnt, bc, 0, 0u);
 }
 
 template <int THREADS, int PPT> static void launch_batch_splat_t(const BatchArgs& a, hipStream_t st) {
