@@ -213,15 +213,18 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 // and denser frames reject most samples at the point-parallel splat's
 // pre-read, which the binned form cannot skip.  A framebuffer of more than
 // GPS_BIN_LARGE_FB words (32 MB) misses the caches, so there both limits are
-// wider: 4 samples per point (given a Gaussian per 16 words, for the launches),
-// and 6 samples per word for every GPS_BIN_LARGE_FB words, up to
-// GPS_BIN_DENSE_LARGE (above that dense frames are splatted nearest first,
-// GPS_ORD_DENSE_SAMPLES).  Whole frames, us, point-parallel / binned, by samples
+// wider: 4 samples per point (given a Gaussian per 16 words, for the launches,
+// and at most 4 per word, as the distributor counts per tile of the scene), and
+// 6 samples per word for every GPS_BIN_LARGE_FB words, up to GPS_BIN_DENSE_LARGE
+// (above that dense frames are splatted nearest first, GPS_ORD_DENSE_SAMPLES).
+// Whole frames, us, point-parallel / binned, by samples
 // per word:
 //   16 samples a point  33M words 18.7: 6132 / 3945, 3.0: 1551 / 824;
 //                       6.6M words 12.4: 640 / 706; 0.9M words 4.4: 150 / 128
 //   4 samples a point   8.3M words 2.4: 415 / 324, 18.7: 2149 / 2142;
 //                       1.6M words 12.4: 325 / 402, 4.8: 180 / 192
+//   occlusion-culled fly-throughs, 4 samples a point, 8.4M words, 4 to 5 samples
+//                       per word: 25M Gaussians 2027 / 1968, 100M 1891 / 1947
 // A batch shares the lists' launches among its views and has no ordered form:
 // views of more than GPS_BIN_LARGE_FB_BATCH words take the wide limits (batch of
 // 16 views from 1.2M to 33M words, 4 to 13 samples per word: all point-parallel

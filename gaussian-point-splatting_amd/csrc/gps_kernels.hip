@@ -3457,7 +3457,7 @@ bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool batch) {
     const uint64_t words = (uint64_t)up_w * (uint64_t)up_h * (uint64_t)spp;
     return K * spp >= GPS_BIN_AUTO_SAMPLES ||
            (K * spp >= GPS_BIN_AUTO_SAMPLES_LARGE && words > (batch ? GPS_BIN_LARGE_FB_BATCH : GPS_BIN_LARGE_FB) &&
-            16ull * N >= words);
+            16ull * N >= words && (batch || N <= 4ull * words));
 }
 
 bool binned_geometry(int up_w, int up_h, int spp, BinGeom* g) {
