@@ -582,12 +582,10 @@ __device__ __forceinline__ uint32_t preprocess_one(const DevScene& s, const Fram
     r[1] = make_uint4(__float_as_uint(c2), __float_as_uint(pr.cc * inv_det), __float_as_uint(-pr.cb * inv_det),
                       __float_as_uint(pr.ca * inv_det));
     r[2] = make_uint4(__float_as_uint(op), __float_as_uint(corrected_inv_alpha(op)), __float_as_uint(dl),
-                      (uint32_t)pr.minx | ((uint32_t)pr.miny << 16));
-    r[3] = make_uint4((uint32_t)pr.maxx | ((uint32_t)pr.maxy << 16), (uint32_t)packed, (uint32_t)(packed >> 32),
+                      pack_bounds_min(pr));
+    r[3] = make_uint4(pack_bounds_max(pr), (uint32_t)packed, (uint32_t)(packed >> 32),
                       __float_as_uint(alpha_threshold(op)));
-    if (bounds_out)
-        *bounds_out = make_uint2((uint32_t)pr.minx | ((uint32_t)pr.miny << 16),
-                                 (uint32_t)pr.maxx | ((uint32_t)pr.maxy << 16));
+    if (bounds_out) *bounds_out = make_uint2(pack_bounds_min(pr), pack_bounds_max(pr));
     return cnt;
 }
 
@@ -618,8 +616,8 @@ __device__ __forceinline__ void push_item(PreItem* s_item, uint32_t* s_n, uint32
     q.cb = pr.cb;
     q.cc = pr.cc;
     q.det = pr.det;
-    q.bmin = (uint32_t)pr.minx | ((uint32_t)pr.miny << 16);
-    q.bmax = (uint32_t)pr.maxx | ((uint32_t)pr.maxy << 16);
+    q.bmin = pack_bounds_min(pr);
+    q.bmax = pack_bounds_max(pr);
     q.mx = mx;
     q.my = my;
     q.mz = mz;
@@ -1363,16 +1361,6 @@ __device__ __forceinline__ uint32_t add_color_sample(unsigned long long* __restr
     return 1u;
 }
 
-// Screen rectangle [x0, x0 + w) x [y0, y0 + h) that a Gaussian's samples may
-// land in.
-struct SampleRect {
-    int x0, y0;
-    uint32_t w, h;
-};
-__device__ __forceinline__ SampleRect record_rect(const SplatRecord& rec) {
-    const int x0 = (int)(rec.bmin & 0xFFFFu), y0 = (int)(rec.bmin >> 16);
-    return SampleRect{x0, y0, (rec.bmax & 0xFFFFu) - (uint32_t)x0, (rec.bmax >> 16) - (uint32_t)y0};
-}
 // One sample of the unbiased splat from an RNG state (splatGaussianPoint,
 // gaussian_point_splatting.cu:67-128): whether it lands in the rectangle and
 // passes the alpha test, and its pixel relative to the rectangle's corner.
@@ -1426,7 +1414,7 @@ __device__ __forceinline__ uint32_t splat_point(const SplatRecord& rec, uint32_t
                                                 int& last, uint32_t* s_key = nullptr,
                                                 unsigned long long* s_val = nullptr, uint32_t key_base = 0u) {
     if (!unbiased) return splat_point_biased(rec, p, frame_seed, K, spp, up_w, fb);
-    const SampleRect rect = record_rect(rec);
+    const SampleRect rect = packed_rect(rec.bmin, rec.bmax);
     const unsigned long long packed = ((unsigned long long)rec.packed_hi << 32) | rec.packed_lo;
     const unsigned long long depth_bits = packed & ~(unsigned long long)GPS_COLOR_MASK;
     const int samples = spp * K;
@@ -1539,11 +1527,10 @@ __device__ __forceinline__ uint32_t flush_word_table(uint32_t* s_key, unsigned l
 // bounds on a word that is already nearer, so none can lower a word.
 __device__ __forceinline__ bool tile_behind(const SplatRecord& rec, const uint32_t* __restrict__ tmax, int tw64) {
     const uint32_t gd = rec.packed_hi >> 4;  // depth28 of the packed word
-    const int tx0 = (int)(rec.bmin & 0xFFFFu) >> 4, ty0 = (int)(rec.bmin >> 20);
-    const int tx1 = (int)(rec.bmax & 0xFFFFu) >> 4, ty1 = (int)(rec.bmax >> 20);
-    if ((tx1 - tx0) * (ty1 - ty0) > GPS_ORD_MAX_TILES) return false;
-    for (int ty = ty0; ty < ty1; ++ty)
-        for (int tx = tx0; tx < tx1; ++tx) {
+    const TileRect q = packed_tiles(rec.bmin, rec.bmax);
+    if ((q.x1 - q.x0) * (q.y1 - q.y0) > GPS_ORD_MAX_TILES) return false;
+    for (int ty = q.y0; ty < q.y1; ++ty)
+        for (int tx = q.x0; tx < q.x1; ++tx) {
             const uint32_t t = ((uint32_t)((ty >> 2) * tw64 + (tx >> 2)) << 4) |
                                (uint32_t)((tx & 1) | ((ty & 1) << 1) | ((tx & 2) << 1) | ((ty & 2) << 2));
             if (tmax[t] >= gd) return false;
@@ -2206,7 +2193,7 @@ __device__ __forceinline__ uint32_t bin_splat_job(const SplatRecord* __restrict_
         if (more) nrec = load_record(recs, nxt.x);
         if (p_hi - p > 2u * GPS_BIN_THREADS) nnxt = list[p + 2u * GPS_BIN_THREADS];
         // the Gaussian's bounds inside the region
-        SampleRect rect = record_rect(rec);
+        SampleRect rect = packed_rect(rec.bmin, rec.bmax);
         const int ox = max(rect.x0 - rx0, 0), oy = max(rect.y0 - ry0, 0);
         rect.w = (uint32_t)max(min(rect.x0 + (int)rect.w, rx0 + (1 << L::W_SHIFT)) - (rx0 + ox), 0);
         rect.h = (uint32_t)max(min(rect.y0 + (int)rect.h, ry0 + (1 << L::H_SHIFT)) - (ry0 + oy), 0);

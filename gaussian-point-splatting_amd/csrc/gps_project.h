@@ -200,6 +200,33 @@ GPS_HD bool project_gaussian(const FrameConsts& f, float mx, float my, float mz,
     return front && project_footprint(f, ce, qw, qx, qy, qz, sx, sy, sz, o);
 }
 
+// Tile-aligned bounds as a splat record holds them, 16 bits an axis.  A frame
+// is at most 65535 pixels wide and high, but its last tile can end at 65536:
+// that maximum is stored as 65535, a pixel that no frame shows.
+GPS_HD uint32_t pack_bounds_min(const Projected& o) { return (uint32_t)o.minx | ((uint32_t)o.miny << 16); }
+GPS_HD uint32_t pack_bounds_max(const Projected& o) {
+    const uint32_t x = (uint32_t)(o.maxx < 65535 ? o.maxx : 65535), y = (uint32_t)(o.maxy < 65535 ? o.maxy : 65535);
+    return x | (y << 16);
+}
+// Screen rectangle [x0, x0 + w) x [y0, y0 + h) that a Gaussian's samples may
+// land in (the packed maxima are never below the minima).
+struct SampleRect {
+    int x0, y0;
+    uint32_t w, h;
+};
+GPS_HD SampleRect packed_rect(uint32_t bmin, uint32_t bmax) {
+    const int x0 = (int)(bmin & 0xFFFFu), y0 = (int)(bmin >> 16);
+    return SampleRect{x0, y0, (bmax & 0xFFFFu) - (uint32_t)x0, (bmax >> 16) - (uint32_t)y0};
+}
+// ... and its 16x16 tiles [x0, x1) x [y0, y1).
+struct TileRect {
+    int x0, y0, x1, y1;
+};
+GPS_HD TileRect packed_tiles(uint32_t bmin, uint32_t bmax) {
+    return TileRect{(int)((bmin & 0xFFFFu) >> 4), (int)(bmin >> 20), (int)(((bmax & 0xFFFFu) + 15u) >> 4),
+                    (int)(((bmax >> 16) + 15u) >> 4)};
+}
+
 // SH basis constants (sh.cuh:137-169).
 #define GPS_SH_C0 0.28209479177387814f
 #define GPS_SH_C1 0.4886025119029199f
