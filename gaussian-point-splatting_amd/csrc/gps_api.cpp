@@ -899,7 +899,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
             ba.job_reg = p->job_reg;
             ba.job_p0 = p->job_p0;
             ba.list = p->list;
-            ba.big = p->big;
+            ba.big = BigList{p->big, p->N, p->budget / GPS_BIG_SLICE + 1};
             ba.state = p->ctr->bin_state[slot];
             p->bin_state = ba.state;
             ba.list_cap = p->list_cap;

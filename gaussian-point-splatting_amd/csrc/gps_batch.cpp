@@ -97,7 +97,7 @@ template <typename T> gps_status balloc(gps_batch* b, T** p, uint64_t count, boo
 
 void free_binned(gps_batch* b) {
     BatchBinArgs& a = b->bin;
-    for (void* p : {(void*)a.bounds, (void*)a.big, (void*)a.reg_pts, (void*)a.reg_ptot, (void*)a.reg_poff,
+    for (void* p : {(void*)a.bounds, (void*)a.big.items, (void*)a.reg_pts, (void*)a.reg_ptot, (void*)a.reg_poff,
                     (void*)a.reg_cursor, (void*)a.job_reg, (void*)a.job_p0, (void*)a.list, (void*)a.state})
         if (p) (void)hipFree(p);
     for (uint2* p : b->old_lists) (void)hipFree(p);
@@ -132,7 +132,9 @@ bool ensure_binned(gps_batch* b) {
         if (s == GPS_OK) s = r;
     };
     chk(balloc(b, &a.bounds, std::max<uint64_t>(V * b->npad, 1), false));  // per record
-    chk(balloc(b, &a.big, entries + (1ull << 32) / GPS_BIG_SLICE, false));
+    a.big.slice0 = (uint32_t)entries;
+    a.big.slice_cap = (uint32_t)((1ull << 32) / GPS_BIG_SLICE);
+    chk(balloc(b, &a.big.items, entries + a.big.slice_cap, false));
     chk(balloc(b, &a.reg_pts, regions, true));
     for (uint32_t** p : {&a.reg_ptot, &a.reg_poff, &a.reg_cursor}) chk(balloc(b, p, regions, false));
     chk(balloc(b, &a.job_reg, a.job_cap, false));

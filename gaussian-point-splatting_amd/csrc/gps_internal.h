@@ -7,6 +7,7 @@
 
 #include "../../include/gps.h"
 #include "gps_hiz.h"
+#include "gps_big.h"
 #include "gps_project.h"
 
 namespace gps {
@@ -205,7 +206,6 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 #define GPS_BIN_HIST 8192u
 #define GPS_BIN_JOB_POINTS 2048u       // smallest full job (bin_scan_kernel)
 #define GPS_BIN_JOB_POINTS_MAX 32768u
-#define GPS_BIG_SLICE 1024u  // points of a Gaussian too large to bin that one workgroup takes at a time
 // GPS_SPLAT_AUTO bins a frame when a point has >= GPS_BIN_AUTO_SAMPLES
 // samples (K * spp) and at most GPS_BIN_DENSE_SAMPLES samples land on a
 // framebuffer word (points * K <= 8 * up_w * up_h, tested on the device once

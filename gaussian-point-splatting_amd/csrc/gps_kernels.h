@@ -53,6 +53,13 @@ struct TileSums {
     uint32_t* iteration;
 };
 
+// (entry, start) items of the Gaussians too large to bin (big_items): the first
+// slices, one per Gaussian, then slice_cap further ones from items[slice0] on.
+struct BigList {
+    uint2* items;
+    uint32_t slice0, slice_cap;
+};
+
 struct SplatArgs {
     const SplatRecord* recs;
     const uint32_t* cidx;
@@ -68,7 +75,7 @@ struct SplatArgs {
     // a pass that may be binned: when the binned splat did not stand down
     // (bin_state[3] == 0) only its big slices are splatted
     const uint32_t* bin_state = nullptr;
-    const uint2* big = nullptr;
+    BigList big{};
     TileSums sums{};
 };
 
@@ -113,9 +120,9 @@ struct BinnedArgs {
     uint32_t *reg_ptot, *reg_poff, *reg_cursor;
     uint32_t *job_reg, *job_p0;
     uint2* list;          // (record, point) of every point and region, region by region
-    uint2* big;           // (entry, first point) slices of the Gaussians too large to bin
-    uint32_t* state;      // 8 words: (entry, region) pairs, jobs, big Gaussians, stand-down, job cursor, unused,
-                          // slices, points per job
+    BigList big;
+    uint32_t* state;      // 8 words: (entry, region) pairs, jobs, big Gaussians, stand-down, job cursor, a tile's
+                          // points did not fit their sums, further slices, points per job
     uint32_t list_cap, job_cap;
     uint32_t cus;
     uint32_t dense_points;  // more points than this: the binned kernels stand down (state[3] = 2)
@@ -138,7 +145,7 @@ struct BatchBinArgs {
     uint32_t nregions;          // regions of all binned views
     uint32_t max_view_regions;  // largest view's regions (LDS histogram size)
     uint2* bounds;
-    uint2* big;
+    BigList big;
     unsigned long long* reg_pts;
     uint32_t *reg_ptot, *reg_poff, *reg_cursor;
     uint32_t *job_reg, *job_p0;

@@ -1077,7 +1077,7 @@ struct BinCount {
     uint32_t dense_points;        // single frame
     const BatchView* views;       // batch: the views' own geometry and limits
     unsigned long long* reg_pts;  // points per region
-    uint2* big;
+    BigList big;
     uint32_t* state;
 };
 
@@ -1113,6 +1113,7 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
     extern __shared__ uint32_t s_pts[];  // BIN: the regions of the frame, or of the batch's largest view
     __shared__ uint32_t s_a[4], s_c[4];
     __shared__ uint4 s_fold[4];
+    __shared__ uint32_t s_units;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t tile = blockIdx.x;
     uint32_t v0, vend, a0;
@@ -1212,8 +1213,10 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
             bc.f.p_end = (uint32_t)P;
             bin = P <= bc.dense_points;  // else too dense to bin: bin_scan_kernel stands the binned kernels down
         }
-        if (bin)
+        if (bin) {
+            if (tid == 0) s_units = 0u;
             for (uint32_t i = (uint32_t)tid; i < bc.f.g.nregions; i += 256u) s_pts[i] = 0u;
+        }
     }
     const uint4* wp = reinterpret_cast<const uint4*>(weights + g0);
     // Groups of 4 without a live element re-read the first live group's
@@ -1263,7 +1266,7 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
         uint2 bnd[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) bnd[k] = w[k] ? record_bounds(bc.f, g0 + (uint32_t)k) : make_uint2(0u, 0u);
-        uint32_t o = off, rr = r, pairs = 0u;
+        uint32_t o = off, rr = r, pairs = 0u, units = 0u;
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
             if (!w[k]) continue;
@@ -1272,13 +1275,21 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
             const BinRect q = bounds_rect(bc.f.g, bnd[k], pts);
             if (q.n > GPS_BIN_MAX_REGIONS) {
                 // too large to bin: its points in slices (a few hold hundreds
-                // of thousands), which bin_big_kernel takes one by one
-                atomicAdd(&bc.state[2], 1u);
-                const uint32_t slices = (pts + GPS_BIG_SLICE - 1u) / GPS_BIG_SLICE;
-                const uint32_t at = atomicAdd(&bc.state[6], slices);
-                for (uint32_t j = 0; j < slices; ++j) bc.big[at + j] = make_uint2(rr, j * GPS_BIG_SLICE);
+                // of thousands), which splat_big and batch_bin_big_kernel take
+                // one by one
+                const uint32_t start = big_items(
+                    pts, bc.big.slice_cap,
+                    [&](uint32_t n) {  // full: not counted further, the counter must not wrap
+                        return __hip_atomic_load(&bc.state[6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                                       bc.big.slice_cap
+                                   ? atomicAdd(&bc.state[6], n)
+                                   : bc.big.slice_cap;
+                    },
+                    [&](uint32_t i, uint32_t s) { bc.big.items[bc.big.slice0 + i] = make_uint2(rr, s); });
+                bc.big.items[atomicAdd(&bc.state[2], 1u)] = make_uint2(rr, start);
             } else if (q.n) {
                 pairs += q.n;
+                units += point_units(pts);
                 for (uint32_t ry = q.ry0; ry <= q.ry1; ++ry)
                     for (uint32_t rx = q.rx0; rx <= q.rx1; ++rx)
                         atomicAdd(&s_pts[ry * (uint32_t)bc.f.g.nrx + rx], pts);
@@ -1286,7 +1297,9 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
             o += w[k];
             ++rr;
         }
+        if (units) atomicAdd(&s_units, units);
         add_count(&bc.state[0], pairs);  // (its barriers order the histogram too)
+        if (tid == 0 && tile_too_large(s_units)) bc.state[5] = 1u;  // no list is long enough
         for (uint32_t i = (uint32_t)tid; i < bc.f.g.nregions; i += 256u)
             if (s_pts[i]) atomicAdd(&bc.reg_pts[bc.f.rbase + i], (unsigned long long)s_pts[i]);
     }
@@ -1614,22 +1627,30 @@ __device__ __forceinline__ uint32_t splat_chunk(uint32_t c, const SplatRecord* _
 // global atomics, by the kernel that follows the binned splat and would take the
 // whole pass had it stood down.
 struct BigSlices {
-    const uint2* big;
+    BigList big;
     const uint32_t* state;  // null: the pass is not binned
 };
+// Item e of the list, first slices first.
+__device__ __forceinline__ uint32_t big_count(const BigList& b, const uint32_t* __restrict__ state) {
+    return state[2] + min(state[6], b.slice_cap);
+}
+__device__ __forceinline__ uint2 big_item(const BigList& b, const uint32_t* __restrict__ state, uint32_t e) {
+    const uint32_t n = state[2];
+    return b.items[e < n ? e : b.slice0 + (e - n)];
+}
 __device__ __forceinline__ uint32_t splat_big(const BigSlices& b, const SplatRecord* __restrict__ recs,
                                               const uint32_t* __restrict__ cidx, const uint32_t* __restrict__ coff,
                                               const PassCounters* __restrict__ ctr, const SplatConsts& sc,
                                               unsigned long long* __restrict__ fb) {
-    const uint32_t n = b.state[6];
+    const uint32_t n = big_count(b.big, b.state);
     uint32_t issued = 0;
     for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
-        const uint2 it = b.big[e];
+        const uint2 it = big_item(b.big, b.state, e);
         const SplatRecord rec = load_record(recs, cidx[it.x]);
         const uint32_t p0 = coff[it.x];
-        const uint32_t w = min(entry_points(coff, it.x, ctr->valid, ctr->total, ctr->points), it.y + GPS_BIG_SLICE);
+        const uint32_t w = big_hi(it.y, entry_points(coff, it.x, ctr->valid, ctr->total, ctr->points));
         int last = -1;  // one Gaussian throughout
-        for (uint32_t k = it.y + threadIdx.x; k < w; k += blockDim.x)
+        for (uint32_t k = big_lo(it.y) + threadIdx.x; k < w; k += blockDim.x)
             issued += splat_point(rec, p0 + k, sc.frame_seed, sc.K, sc.spp, sc.up_w, 1, fb, last);
     }
     return issued;
@@ -1963,12 +1984,12 @@ __global__ __launch_bounds__(1024) void bin_scan_kernel(uint32_t nregions, unsig
         s_jobs = run;
         const bool dense = ctr && ctr->points > dense_points;
         state[1] = min(run, job_cap);
-        state[3] = dense ? 2u : (s_carry > list_cap || run > job_cap) ? 1u : 0u;
+        state[3] = dense ? 2u : (s_carry > list_cap || run > job_cap || state[5]) ? 1u : 0u;
         state[4] = 0u;
         state[7] = job_points;
     }
     __syncthreads();
-    if (s_jobs > job_cap || s_carry > list_cap) return;
+    if (s_jobs > job_cap || s_carry > list_cap || state[5]) return;
     for (uint32_t i = (uint32_t)tid; i < nregions; i += 1024) {
         const uint32_t p32 = reg_ptot[i];
         const uint32_t full = p32 / job_points, rest = p32 - full * job_points;
@@ -2354,24 +2375,24 @@ __global__ __launch_bounds__(256) void batch_bin_big_kernel(const SplatRecord* _
                                                             const uint32_t* __restrict__ cidx,
                                                             const uint32_t* __restrict__ coff,
                                                             const uint8_t* __restrict__ cview,
-                                                            const uint2* __restrict__ big,
+                                                            BigList big,
                                                             const uint32_t* __restrict__ state,
                                                             const BatchView* __restrict__ views,
                                                             unsigned long long* __restrict__ fb,
                                                             uint32_t* __restrict__ atomics_count) {
     if (state[3]) return;
-    const uint32_t n = state[6];
+    const uint32_t n = big_count(big, state);
     uint32_t issued = 0;
     for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
-        const uint2 it = big[e];
+        const uint2 it = big_item(big, state, e);
         const BatchView& bv = views[cview[it.x]];
         const SplatRecord rec = load_record(recs, cidx[it.x]);
         const uint32_t p0 = coff[it.x] - bv.base;
-        const uint32_t w = min(entry_points(coff, it.x, bv.ebase + bv.valid, bv.base + bv.total, bv.base + bv.points),
-                               it.y + GPS_BIG_SLICE);
+        const uint32_t w =
+            big_hi(it.y, entry_points(coff, it.x, bv.ebase + bv.valid, bv.base + bv.total, bv.base + bv.points));
         const uint32_t seed = bv.f.frame_seed + 1u;
         int last = -1;  // one Gaussian throughout
-        for (uint32_t k = it.y + threadIdx.x; k < w; k += 256u)
+        for (uint32_t k = big_lo(it.y) + threadIdx.x; k < w; k += 256u)
             issued += splat_point(rec, p0 + k, seed, bv.f.Ki, bv.f.spp, bv.f.up_w, bv.f.unbiased, fb + bv.fb_offset,
                                   last);
     }
@@ -3403,7 +3424,7 @@ void launch_batch_bin_big(const BatchArgs& a, hipStream_t st) {
     if (!b.any) return;
     hipLaunchKernelGGL(batch_bin_big_kernel, dim3(b.cus * 4u), dim3(256), 0, st, (const SplatRecord*)a.recs,
                        (const uint32_t*)a.cidx, (const uint32_t*)a.coff, (const uint8_t*)a.cview,
-                       (const uint2*)b.big, (const uint32_t*)b.state, (const BatchView*)a.views,
+                       b.big, (const uint32_t*)b.state, (const BatchView*)a.views,
                        reinterpret_cast<unsigned long long*>(a.fb), a.atomics);
 }
 

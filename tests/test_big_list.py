@@ -1,0 +1,85 @@
+"""The binned splat's lists where a frame's point total passes 2^32: offsets
+wrap and points below the budget are handed out once per turn, so the items of
+the Gaussians too large to bin can outnumber Gaussians + budget / 1024, and a
+tile's points per region their 32-bit sums."""
+import os
+import re
+import subprocess
+import zlib
+
+import numpy as np
+import pytest
+
+import helpers as H
+from helpers import assert_same, flush
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+GOLDEN_FRAMEBUFFER = 2740137265
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("big_list") / "check")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wno-unknown-pragmas", "-I",
+                    os.path.join(ROOT, "gaussian-point-splatting_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "big_list_check.cpp"), "-o", exe], check=True, capture_output=True)
+
+    def run(*args):
+        out = subprocess.run([exe, *map(str, args)], check=True, capture_output=True, text=True, timeout=300).stdout
+        return dict((k, int(v)) for k, v in re.findall(r"(\w+) (\d+)", out))
+    return run
+
+
+# Gaussians, points each, budget; turns of 2^32 points, items run out, a tile's sum too large
+@pytest.mark.parametrize("n,most,budget,turns,short,wide", [
+    (1, 1, 10, 0, False, False),
+    (5000, 1024, 10_000_000, 0, False, False),
+    (5000, 1025, 3_000, 0, False, False),
+    (3000, 1 << 20, 250_000_000, 0, False, False),
+    (40_000, 131_072, 48_000_000, 0, False, False),
+    (60_000, 131_072, 48_000_000, 1, True, False),
+    (20_000, 1 << 21, 250_000_000, 7, True, False),
+    (20_000, 1 << 21, 10_000, 7, False, False),
+    (8192, 1 << 23, 2_147_483_647, 11, True, True),
+    (4096, 1 << 20, 2_147_483_647, 0, False, False),
+])
+def test_items_and_sums(check, n, most, budget, turns, short, wide):
+    r = check(n, most, budget, 7)
+    assert r["faults"] == 0, r
+    assert r["turns"] == turns and (r["short"] > 0) == short and (r["wide"] > 0) == wide, r
+
+
+def _scene(n):
+    """Gaussians of some hundreds of pixels on a 512 x 512 screen: each has
+    the most points that a frame allows one, 131072."""
+    rng = np.random.default_rng(77)
+    m = np.concatenate([rng.uniform(-1.0, 1.0, (n, 2)), rng.uniform(-2.0, 2.0, (n, 1))], 1)
+    q = np.tile(np.array([1.0, 0.0, 0.0, 0.0]), (n, 1))
+    return H.G.SceneArrays(m.astype(np.float32), q.astype(np.float32), np.full((n, 3), 4.0, np.float32),
+                           np.full(n, 0.99, np.float32), rng.normal(0, 0.4, (n, 3)).astype(np.float32), 0)
+
+
+@pytest.mark.gpu
+def test_point_total_past_32_bits(gpu):
+    """5.2e9 points, a budget of 48M: the points below the budget are handed
+    out twice, and the shared items run out.  The framebuffer's checksum was
+    recorded from the form that gave each Gaussian one item."""
+    arrays = _scene(40_000)
+    st = gpu.RenderSettings(512, 512, 1, 1, max_number_of_points=48_000_000, fully_disable_hierarchical_culling=True)
+    f = gpu.frame_params((0.0, 0.0, 10.0), (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 45.0, 512, 512, ss=1, spp=1)
+    flush("point total past 32 bits: single pass")
+    r = H.GpuRunner(arrays, st)
+    r.p.set_splat_mode(gpu.Pass.SPLAT_BINNED)
+    a = r.render(f, [gpu.DBG_FRAMEBUFFER])
+    print(a.stats)
+    assert a.stats["valid_gaussians"][0] == 40_000 and a.stats["num_points"][0] == 48_000_000
+    assert a.stats["splat_binned"] == 1 and a.stats["splat_fallback"] == 0
+    assert 700 < a.stats["bin_big"] < 800
+    assert zlib.crc32(a.debug[gpu.DBG_FRAMEBUFFER].tobytes()) == GOLDEN_FRAMEBUFFER
+    flush("point total past 32 bits: the next frame")
+    g = gpu.frame_params((0.0, 0.0, 4000.0), (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 45.0, 512, 512, ss=1, spp=1)
+    b = r.render(g, [gpu.DBG_FRAMEBUFFER])
+    r.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
+    c = r.render(g, [gpu.DBG_FRAMEBUFFER])
+    assert_same("next frame", b.debug[gpu.DBG_FRAMEBUFFER], c.debug[gpu.DBG_FRAMEBUFFER])
+
