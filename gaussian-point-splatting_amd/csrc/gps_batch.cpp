@@ -26,6 +26,7 @@
 #include "gps_fb.h"
 #include "gps_internal.h"
 #include "gps_kernels.h"
+#include "gps_list_growth.h"
 
 using namespace gps;
 
@@ -75,7 +76,8 @@ struct gps_batch {
     bool bin_ready = false, bin_failed = false;
     BatchBinArgs bin{};
     uint32_t bin_regions_cap = 0;
-    std::vector<uint2*> old_lists;  // replaced by larger ones (see ensure_list)
+    ListGrowth list;
+    std::vector<uint2*> old_lists;  // replaced by longer ones (see ensure_list)
     bool use_graph = false;
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
@@ -108,9 +110,9 @@ void free_binned(gps_batch* b) {
 // Binned splat buffers for every compacted entry of a full batch and the
 // regions of max_views views of the largest size.  On failure the batch
 // keeps rendering every view with the point-parallel splat.
-bool ensure_binned(gps_batch* b) {
+bool ensure_binned(gps_batch* b, bool may_alloc) {
     if (b->bin_ready) return true;
-    if (b->bin_failed) return false;
+    if (b->bin_failed || !may_alloc) return false;
     const uint64_t V = (uint64_t)b->settings.max_views;
     const uint64_t entries = std::max<uint64_t>(V * b->N, 1);
     uint32_t max_regions = 0;
@@ -159,27 +161,42 @@ void drop_graph(gps_batch* b) {
     b->layout = Layout{};
 }
 
-// The binned views' point list: room for `points`, replaced by one of at
-// least twice the size when a batch needs more.  The replaced lists stay until
-// the batch goes: batches in flight and graphs that a caller captured write to
-// them.  False when it cannot be had: the batch then renders every view
-// point-parallel.
-bool ensure_list(gps_batch* b, uint64_t points) {
+// Points that a view's list holds under the automatic choice: its densest
+// binnable points twice, as a pass's list, and no more than the budget twice.
+uint64_t view_list_points(uint64_t width, uint64_t height, uint64_t N, uint64_t budget) {
+    const uint64_t px = width * height;
+    const uint64_t dense =
+        std::max<uint64_t>(2 * GPS_BIN_DENSE_SAMPLES * px, std::min<uint64_t>(8 * N, px * GPS_BIN_DENSE_LARGE * 5 / 4));
+    return std::min<uint64_t>(dense, 2 * std::max<uint64_t>(budget, 1ull << 20));
+}
+
+// The binned views' point list, room for `points` where it can be had (see
+// ListGrowth).  The first one takes 9/4 points per Gaussian and view of a full
+// batch, or what the largest views can use if that is less, so that few batches
+// need a longer one.  The replaced lists stay until the batch goes: batches in
+// flight and graphs that a caller captured write to them.  False when there is
+// none: the batch then renders every view point-parallel.
+bool ensure_list(gps_batch* b, uint64_t points, bool may_alloc) {
     BatchBinArgs& a = b->bin;
     constexpr uint64_t kMost = 0xFFFFF000ull;
+    const uint64_t V = (uint64_t)b->settings.max_views;
+    const uint64_t full = std::min<uint64_t>(
+        V * b->N * 9 / 4, V * view_list_points(b->settings.max_width, b->settings.max_height, b->N,
+                                               (uint64_t)b->settings.max_number_of_points));
     points = std::min<uint64_t>(std::max<uint64_t>(points, 1ull << 21), kMost);
-    if (points <= a.list_cap) return true;
-    drop_graph(b);
-    uint2* list = nullptr;
-    uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(points, 2ull * a.list_cap), kMost);
-    if (balloc(b, &list, cap, false) != GPS_OK) {
-        (void)hipGetLastError();
-        return false;
-    }
-    if (a.list) b->old_lists.push_back(a.list);
-    a.list = list;
-    a.list_cap = (uint32_t)cap;
-    return true;
+    return b->list.reserve(points, std::min(full, kMost), may_alloc, [&](uint64_t n) {
+        uint2* list = nullptr;
+        n = std::min(n, kMost);
+        if (balloc(b, &list, n, false) != GPS_OK) {
+            (void)hipGetLastError();
+            return false;
+        }
+        drop_graph(b);  // it writes to the list that was
+        if (a.list) b->old_lists.push_back(a.list);
+        a.list = list;
+        a.list_cap = (uint32_t)n;
+        return true;
+    });
 }
 
 BatchArgs args(gps_batch* b, int nviews) {
@@ -337,10 +354,15 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
     lay.ppt = b->ppt;
     lay.pre_views = b->pre_views;
     uint32_t regions = 0, max_view_regions = 0, bin_views = 0;
-    // Room of the binned views' list: their densest binnable points twice, as
-    // a pass's list; at least 2^24 points a view (128 MB), and two per
-    // Gaussian, where forced binning takes denser views too.
+    // Room of the binned views' list: under the automatic choice what each can
+    // use; where forced binning takes denser views too, at least 2^24 points a
+    // view (128 MB) and two per Gaussian.
     uint64_t list_points = 0;
+    // A caller that captures this call gets no allocation: the list there is
+    // serves, or the point-parallel splat.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool may_alloc = !stream || (hipStreamIsCapturing(st, &capture) == hipSuccess &&
+                                       capture == hipStreamCaptureStatusNone);
     for (int v = 0; v < nviews; ++v) {
         const gps_frame_params& f = views[v];
         const int spp = f.samples_per_pixel > 0 ? f.samples_per_pixel : b->settings.max_spp;
@@ -367,7 +389,7 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
         BinGeom g;
         if (bv.f.unbiased && b->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
             (b->splat_mode == GPS_SPLAT_BINNED || binned_auto(bv.f.up_w, bv.f.up_h, bv.f.spp, bv.f.Ki, b->N, true)) &&
-            binned_geometry(bv.f.up_w, bv.f.up_h, bv.f.spp, &g) && ensure_binned(b) &&
+            binned_geometry(bv.f.up_w, bv.f.up_h, bv.f.spp, &g) && ensure_binned(b, may_alloc) &&
             regions + g.nregions <= b->bin_regions_cap) {
             bv.bg = g;
             bv.rbase = regions;
@@ -378,9 +400,7 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
             regions += g.nregions;
             ++bin_views;
             max_view_regions = std::max(max_view_regions, g.nregions);
-            const uint64_t px = (uint64_t)f.width * (uint64_t)f.height;
-            const uint64_t dense = std::max<uint64_t>(2 * GPS_BIN_DENSE_SAMPLES * px,
-                                                      std::min<uint64_t>(8ull * b->N, px * GPS_BIN_DENSE_LARGE * 5 / 4));
+            const uint64_t dense = view_list_points((uint64_t)f.width, (uint64_t)f.height, b->N, bv.budget);
             list_points += b->splat_mode == GPS_SPLAT_BINNED ? std::max<uint64_t>({dense, 2ull * b->N, 1ull << 24}) : dense;
         } else {
             bv.rbase = regions;  // bg.nregions == 0: point-parallel
@@ -390,7 +410,7 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
         lay.outs.push_back(colors[v]);
         lay.outs.push_back(depths[v]);
     }
-    if (regions > 0 && !ensure_list(b, list_points)) {
+    if (regions > 0 && !ensure_list(b, list_points, may_alloc)) {
         for (int v = 0; v < nviews; ++v) {
             b->h_views[v].bg = BinGeom{};
             b->h_views[v].rbase = 0;

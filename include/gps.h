@@ -563,11 +563,16 @@ gps_status gps_batch_set_tuning(gps_batch* batch, const gps_batch_tuning* tuning
 /* Splat form per view, with the rule and modes of gps_pass_set_splat_mode:
  * the binned views of a batch share one set of binning launches (regions of
  * all of them in one job queue), the rest use the point-parallel batch
- * splat.  The binned buffers (16 B per compacted entry; 8 B per listed point,
- * sized by the views, grown by a later batch that needs more) are allocated
- * on the first batch that bins a view; if an allocation fails every view
- * stays point-parallel.  No
- * reference counterpart. */
+ * splat.  The binned buffers are allocated on the first batch that bins a
+ * view: 16 B per compacted entry, and 8 B per listed point, room for 9/4
+ * points per Gaussian and view of a full batch or what this batch's views can
+ * use if that is more.  A later batch of larger views may replace the list by
+ * a longer one (the old one is kept until the batch is destroyed); if that
+ * fails, or while the caller captures `stream`, the list there is serves, and
+ * a batch with more points than it holds splats point-parallel.  To capture a
+ * batch with its binned form, render one of the same views beforehand.  If
+ * there is no list every view stays point-parallel.  No reference
+ * counterpart. */
 gps_status gps_batch_set_splat_mode(gps_batch* batch, int32_t mode);
 /* Counters of view `view` of the last batch (atomics, bin_entries, bin_jobs,
  * bin_big: whole batch). */
