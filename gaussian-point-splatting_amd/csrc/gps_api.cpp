@@ -66,6 +66,17 @@ namespace {
 
 }  // namespace
 
+namespace {
+
+// The binned splat's point list and the job table that goes with its length.
+struct BinList {
+    uint2* points = nullptr;
+    uint32_t *job_reg = nullptr, *job_p0 = nullptr;
+    uint32_t cap = 0, job_cap = 0;
+};
+
+}  // namespace
+
 struct gps_pass {
     gps_scene* scene = nullptr;
     gps_render_settings settings{};
@@ -86,15 +97,16 @@ struct gps_pass {
     int32_t count_atomics = 0;
     int32_t count_rejects = 0;
     uint32_t cus = 256;
+    // allocated once a frame can be binned (ensure_bin)
     uint2* bounds = nullptr;  // the records' bounds, written while the frame may be binned
     unsigned long long* reg_pts = nullptr;
     uint32_t *reg_ptot = nullptr, *reg_poff = nullptr, *reg_cursor = nullptr;
-    uint32_t *job_reg = nullptr, *job_p0 = nullptr;
-    uint2* list = nullptr;
-    uint2* first_list = nullptr;  // replaced by a longer one when binning was forced
+    BinList list;
+    BinList first_list;       // replaced by a longer one when binning was forced
+    uint64_t max_list = ~0ull; // the automatic list is no longer than this
+    int32_t bin_ss = 0;       // supersampling factor that the automatic list was sized for
     uint2* big = nullptr;
     const uint32_t* bin_state = nullptr;  // of the last binned pass, in ctr
-    uint32_t list_cap = 0, first_list_cap = 0, job_cap = 0;
     int last_binned = 0;
     uint64_t dbg_indices_cap = 0;
     // framebuffers
@@ -194,19 +206,97 @@ gps_status ensure_fb(gps_pass* p, int ss, uint64_t frame_words) {
     return GPS_OK;
 }
 
-// Points that the binned splat's list holds: the automatic choice bins at most
-// GPS_BIN_DENSE_SAMPLES samples per framebuffer word, i.e. that many points per
-// output pixel (a binned frame's points carry ss^2 samples per layer), or
-// GPS_BIN_DENSE_LARGE in a large framebuffer, which takes millions of Gaussians.
-// Room for the first twice and for the second 1.25 times (Gaussians straddling
-// regions are replayed in each: 1.15 to 1.3 times).
-uint64_t bin_list_points(const gps_render_settings& st, uint64_t N) {
-    const uint64_t px = (uint64_t)st.width * (uint64_t)st.height;
-    const uint64_t most = std::min<uint64_t>(8 * N, px * GPS_BIN_DENSE_LARGE * 5 / 4);
-    return std::min<uint64_t>(std::max<uint64_t>({2 * GPS_BIN_DENSE_SAMPLES * px, 2 * N, most}), 0xFFFFF000ull);
+// Points that a list needs for the automatic choice in frames of the settings'
+// size at supersampling `ss`, 0 where it bins none of them (a frame's points
+// have ss^2 or 1 samples per layer).  Gaussians that straddle regions are listed
+// in each, 1.15 to 1.3 times in all: room twice for GPS_BIN_DENSE_SAMPLES per
+// framebuffer word, and 1.25 times for what only large framebuffers take (there
+// at most 8 per Gaussian, which scenes of millions do not reach, but two per
+// Gaussian twice); never more than the point budget twice.
+uint64_t bin_list_points(const gps_render_settings& st, int ss, uint64_t N) {
+    const uint64_t up = (uint64_t)st.width * ss * (uint64_t)st.height * ss;
+    uint64_t need = 0;
+    for (const int K : {ss * ss, 1})
+        for (int spp = st.flexible_frame_size ? 1 : st.render_pass_count; spp <= std::min(st.render_pass_count, 4); ++spp) {
+            BinGeom g;
+            const bool can = st.flexible_frame_size  // any smaller frame too
+                                 ? K * spp >= GPS_BIN_AUTO_SAMPLES ||
+                                       (K * spp >= GPS_BIN_AUTO_SAMPLES_LARGE && up * spp > GPS_BIN_LARGE_FB)
+                                 : binned_auto(st.width * ss, st.height * ss, spp, K, N, false) &&
+                                       binned_geometry(st.width * ss, st.height * ss, spp, &g);
+            if (!can) continue;
+            const uint64_t dense = binned_dense_points(st.width * ss, st.height * ss, spp, K, false);
+            const uint64_t always = K * spp >= GPS_BIN_AUTO_SAMPLES ? 2 * GPS_BIN_DENSE_SAMPLES * up / (uint64_t)K : 0;
+            need = std::max<uint64_t>({need, always, std::min<uint64_t>(8 * N, dense * 5 / 4),
+                                       std::min<uint64_t>(2 * N, 2 * dense)});
+        }
+    const uint64_t budget = (uint64_t)std::max<int64_t>(st.max_number_of_points, 1 << 20);
+    return std::min<uint64_t>({need, 2 * budget, 0xFFFFF000ull});
 }
 // ... and room for the whole point budget, up to 2 GiB, once binning is forced.
-uint32_t bin_forced_points(int64_t budget) { return (uint32_t)std::min<int64_t>(2 * std::max<int64_t>(budget, 1 << 20), 1 << 28); }
+uint64_t bin_forced_points(uint64_t budget) { return std::min<uint64_t>(2 * std::max<uint64_t>(budget, 1 << 20), 1 << 28); }
+
+uint32_t bin_job_cap(uint64_t list_points) { return GPS_BIN_HIST + (uint32_t)(list_points / GPS_BIN_JOB_POINTS) + 1; }
+uint64_t bin_list_bytes(uint64_t points) { return points ? 8 * points + 8ull * bin_job_cap(points) : 0; }
+// The binned buffers without the list.
+uint64_t bin_fixed_bytes(uint64_t N, uint64_t budget) {
+    return std::max<uint64_t>(N, 1) * 8 + (N + budget / GPS_BIG_SLICE + 1) * 8 + 20ull * GPS_BIN_HIST;
+}
+
+void free_list(BinList& l) {
+    dfree(l.points);
+    dfree(l.job_reg);
+    dfree(l.job_p0);
+    l = BinList{};
+}
+void free_bin(gps_pass* p) {
+    dfree(p->bounds);
+    dfree(p->big);
+    dfree(p->reg_pts);
+    for (uint32_t** a : {&p->reg_ptot, &p->reg_poff, &p->reg_cursor}) dfree(*a);
+    free_list(p->list);
+    free_list(p->first_list);
+}
+
+// The binned buffers, with a list of at least `points` points.  A list that is
+// there and too short is kept as first_list (a captured frame may write to it)
+// or, with `replace`, freed.  Without the memory the pass keeps what it has: the
+// device falls back where a list is too short, and without one every frame is
+// splatted point-parallel.
+void ensure_bin(gps_pass* p, uint64_t points, bool replace) {
+    if (points <= p->list.cap) return;
+    bool ok = true;
+    auto chk = [&](gps_status r) { ok = ok && r == GPS_OK; };
+    const bool fixed = p->bounds != nullptr;
+    if (!fixed) {
+        chk(dalloc(&p->bounds, p->N, false));
+        if (ok) chk(dalloc(&p->big, (uint64_t)p->N + p->budget / GPS_BIG_SLICE + 1, false));
+        if (ok) chk(dalloc(&p->reg_pts, GPS_BIN_HIST, true));
+        for (uint32_t** a : {&p->reg_ptot, &p->reg_poff, &p->reg_cursor})
+            if (ok) chk(dalloc(a, GPS_BIN_HIST, false));
+    }
+    BinList l;
+    l.cap = (uint32_t)points;
+    l.job_cap = bin_job_cap(points);
+    if (ok && replace) free_list(p->list);
+    if (ok) chk(dalloc(&l.points, points, false));
+    if (ok) chk(dalloc(&l.job_reg, l.job_cap, false));
+    if (ok) chk(dalloc(&l.job_p0, l.job_cap, false));
+    if (!ok) {
+        (void)hipGetLastError();
+        free_list(l);
+        if (!fixed) free_bin(p);
+        return;
+    }
+    if (p->list.points) p->first_list = p->list;
+    p->list = l;
+}
+// ... as the automatic choice needs them at supersampling `ss`.
+void ensure_bin_auto(gps_pass* p, int ss, bool replace) {
+    if (p->bin_ss == ss) return;
+    p->bin_ss = ss;
+    ensure_bin(p, std::min(bin_list_points(p->settings, ss, p->N), p->max_list), replace);
+}
 
 constexpr int kOcc = 2;
 inline int ev_index(int slot, int stage, int occ, int which) {
@@ -472,6 +562,12 @@ uint64_t gps_scene_device_bytes(const gps_scene* s) { return s ? s->bytes : 0; }
 
 // ------------------------------------------------------------------ passes
 gps_status gps_pass_create(const gps_render_settings* st, gps_scene* scene, gps_pass** out) {
+    return pass_create(st, scene, ~0ull, out);
+}
+
+}  // extern "C"
+
+gps_status gps::pass_create(const gps_render_settings* st, gps_scene* scene, uint64_t max_list, gps_pass** out) {
     if (!st || !scene || !out) return GPS_ERR_INVALID_ARG;
     *out = nullptr;
     if (st->width <= 0 || st->height <= 0 || st->render_pass_count < 1 || st->supersampling_factor < 1 ||
@@ -510,21 +606,6 @@ gps_status gps_pass_create(const gps_render_settings* st, gps_scene* scene, gps_
     chk(dalloc(&p->ord_bucket, (uint64_t)p->budget / GPS_SPLAT_CHUNK + 2, false));
     chk(dalloc(&p->ord_hist, GPS_ORD_BINS, true));
     chk(dalloc(&p->ord_lim, GPS_ORD_PHASES, true));
-    // Binned splat: its list holds a pass's points once per region they are
-    // replayed in (overflow falls back to the point-parallel splat on the
-    // device).
-    {
-        const uint64_t cap = bin_list_points(*st, N);
-        p->list_cap = (uint32_t)cap;
-        p->job_cap = GPS_BIN_HIST + (uint32_t)(std::max<uint64_t>(cap, bin_forced_points(p->budget)) / GPS_BIN_JOB_POINTS) + 1;
-        chk(dalloc(&p->bounds, std::max<uint64_t>(N, 1), false));
-        chk(dalloc(&p->big, N + (uint64_t)p->budget / GPS_BIG_SLICE + 1, false));
-        chk(dalloc(&p->reg_pts, GPS_BIN_HIST, true));
-        for (uint32_t** a : {&p->reg_ptot, &p->reg_poff, &p->reg_cursor}) chk(dalloc(a, GPS_BIN_HIST, false));
-        chk(dalloc(&p->job_reg, p->job_cap, false));
-        chk(dalloc(&p->job_p0, p->job_cap, false));
-        chk(dalloc(&p->list, cap, false));
-    }
     chk(dalloc(&p->ctr, 1, true));
     // Hi-Z pyramid at output resolution, initialised to +inf (nothing occluded).
     p->hiz_size = (uint32_t)mip_total(p->hiz, st->width, st->height);
@@ -564,6 +645,9 @@ gps_status gps_pass_create(const gps_render_settings* st, gps_scene* scene, gps_
         s = ensure_fb(p, st->supersampling_factor,
                       fb_words(st->width * st->supersampling_factor, st->height * st->supersampling_factor,
                                st->render_pass_count));
+    // last: a pass that cannot have these renders point-parallel
+    p->max_list = max_list;
+    if (s == GPS_OK) ensure_bin_auto(p, st->supersampling_factor, false);
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
         hipDeviceProp_t prop;
@@ -587,6 +671,8 @@ gps_status gps_pass_create(const gps_render_settings* st, gps_scene* scene, gps_
     return GPS_OK;
 }
 
+extern "C" {
+
 gps_status gps_pass_set_ordered_splat(gps_pass* p, int32_t mode) {
     if (!p || (mode != GPS_ORDERED_AUTO && mode != GPS_ORDERED_OFF && mode != GPS_ORDERED_ALWAYS))
         return GPS_ERR_INVALID_ARG;
@@ -596,20 +682,8 @@ gps_status gps_pass_set_ordered_splat(gps_pass* p, int32_t mode) {
 
 gps_status gps_pass_set_splat_mode(gps_pass* p, int32_t mode) {
     if (!p || mode < GPS_SPLAT_AUTO || mode > GPS_SPLAT_BINNED) return GPS_ERR_INVALID_ARG;
-    // Forced binning takes denser frames than the automatic choice: a longer
-    // list.  The first one stays (a captured frame may write to it).
-    const uint32_t want = bin_forced_points(p->budget);
-    if (mode == GPS_SPLAT_BINNED && p->list_cap < want) {
-        uint2* list = nullptr;
-        if (dalloc(&list, want, false) == GPS_OK) {
-            p->first_list = p->list;
-            p->first_list_cap = p->list_cap;
-            p->list = list;
-            p->list_cap = want;
-        } else {
-            (void)hipGetLastError();  // the list there is serves, up to its length
-        }
-    }
+    // Forced binning takes denser frames than the automatic choice: a longer list.
+    if (mode == GPS_SPLAT_BINNED) ensure_bin(p, bin_forced_points(p->budget), false);
     p->splat_mode = mode;
     return GPS_OK;
 }
@@ -628,7 +702,16 @@ gps_status gps_pass_set_counters(gps_pass* p, int32_t flags) {
 }
 
 uint64_t gps_pass_estimate_bytes(const gps_render_settings* st, const gps_scene* scene) {
-    if (!st || !scene) return 0;
+    return st && scene ? pass_bytes(st, scene, ~0ull) : 0;
+}
+
+}  // extern "C"
+
+uint64_t gps::pass_list_points(const gps_render_settings* st, const gps_scene* scene) {
+    return bin_list_points(*st, st->supersampling_factor, scene->view.N);
+}
+
+uint64_t gps::pass_bytes(const gps_render_settings* st, const gps_scene* scene, uint64_t max_list) {
     const uint64_t N = scene->view.N;
     const uint64_t ntiles = (N + GPS_TILE - 1) / GPS_TILE, npad = ntiles * GPS_TILE, nwords = (N + 31) / 32 + 2;
     const uint64_t budget = (uint64_t)std::min<int64_t>(st->max_number_of_points, 0x7FFFFFFFll);
@@ -640,11 +723,8 @@ uint64_t gps_pass_estimate_bytes(const gps_render_settings* st, const gps_scene*
                  16 * ntiles + (budget / GPS_SPLAT_CHUNK + 2) * 4 + sizeof(FrameCounters) + hiz * 4 + 2 * fb * 8;
     b += (budget / GPS_SPLAT_CHUNK + 2) * 2 + 4ull * (GPS_ORD_BINS + GPS_ORD_PHASES) +
          fb / (256ull * (uint64_t)st->render_pass_count) * 4;  // ordered splat
-    {
-        const uint64_t cap = bin_list_points(*st, N);
-        b += std::max<uint64_t>(N, 1) * 8 + (N + budget / GPS_BIG_SLICE + 1) * 8 + cap * 8 + 20ull * GPS_BIN_HIST +
-             2ull * 4 * (GPS_BIN_HIST + std::max<uint64_t>(cap, bin_forced_points((int64_t)budget)) / GPS_BIN_JOB_POINTS + 1) + 32;
-    }
+    if (const uint64_t points = std::min(pass_list_points(st, scene), max_list))
+        b += bin_fixed_bytes(N, budget) + bin_list_bytes(points);
     if (!st->fully_disable_hierarchical_culling) {
         const uint64_t gpb = st->gaussians_per_block > 0 ? (uint64_t)st->gaussians_per_block
                                                          : (uint64_t)std::max(4.0f, std::floor((float)N / 1e6f));
@@ -661,6 +741,8 @@ uint64_t gps_pass_estimate_bytes(const gps_render_settings* st, const gps_scene*
     return b;
 }
 
+extern "C" {
+
 uint64_t gps_pass_device_bytes(const gps_pass* p) {
     if (!p) return 0;
     const uint64_t N = p->N, npad = (uint64_t)p->ntiles * GPS_TILE, nwords = (N + 31) / 32 + 2;
@@ -673,8 +755,8 @@ uint64_t gps_pass_device_bytes(const gps_pass* p) {
              p->fb_cap / (256ull * (uint64_t)p->settings.render_pass_count) * 4;
     if (p->gboxes) b += (uint64_t)p->group.count * sizeof(GroupBox) + round_up(p->group.count, 4) + 4;
     if (p->live) b += (uint64_t)p->cull.node_count * 4 + (N + GPS_PRE_THREADS - 1) / GPS_PRE_THREADS;
-    b += std::max<uint64_t>(N, 1) * 8 + (N + (uint64_t)p->budget / GPS_BIG_SLICE + 1) * 8 +
-         8ull * ((uint64_t)p->list_cap + p->first_list_cap) + 20ull * GPS_BIN_HIST + 2ull * 4 * p->job_cap + 32;
+    if (p->bounds)
+        b += bin_fixed_bytes(N, p->budget) + bin_list_bytes(p->list.cap) + bin_list_bytes(p->first_list.cap);
     return b;
 }
 
@@ -707,12 +789,7 @@ void gps_pass_destroy(gps_pass* p) {
     dfree(p->gocc);
     dfree(p->live);
     dfree(p->wg_live);
-    dfree(p->bounds);
-    dfree(p->big);
-    dfree(p->reg_pts);
-    dfree(p->list);
-    dfree(p->first_list);
-    for (uint32_t** a : {&p->reg_ptot, &p->reg_poff, &p->reg_cursor, &p->job_reg, &p->job_p0}) dfree(*a);
+    free_bin(p);
     delete p;
 }
 
@@ -790,6 +867,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     hipStream_t st = (hipStream_t)stream;
     gps_status s = ensure_fb(p, ss, fb_words(fp->width * ss, fp->height * ss, spp));
     if (s != GPS_OK) return s;
+    ensure_bin_auto(p, ss, true);  // as the framebuffers: only when ss changed
 
     FrameConsts f;
     make_frame_consts(fp, spp, &f);
@@ -812,7 +890,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     BinGeom bg_geom;
     // the biased splat adds colours per sample and has only the
     // point-parallel form
-    const bool binned = f.unbiased && p->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
+    const bool binned = f.unbiased && p->list.points && p->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
                         (p->splat_mode == GPS_SPLAT_BINNED || binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, false)) &&
                         binned_geometry(f.up_w, f.up_h, f.spp, &bg_geom);
     stage_mark(p, 0, 0, 0, st);
@@ -896,14 +974,14 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
             ba.reg_ptot = p->reg_ptot;
             ba.reg_poff = p->reg_poff;
             ba.reg_cursor = p->reg_cursor;
-            ba.job_reg = p->job_reg;
-            ba.job_p0 = p->job_p0;
-            ba.list = p->list;
+            ba.job_reg = p->list.job_reg;
+            ba.job_p0 = p->list.job_p0;
+            ba.list = p->list.points;
             ba.big = BigList{p->big, p->N, p->budget / GPS_BIG_SLICE + 1};
             ba.state = p->ctr->bin_state[slot];
             p->bin_state = ba.state;
-            ba.list_cap = p->list_cap;
-            ba.job_cap = p->job_cap;
+            ba.list_cap = p->list.cap;
+            ba.job_cap = p->list.job_cap;
             ba.cus = p->cus;
             ba.dense_points = dense_points;
             ba.atomics_count = p->count_atomics ? &p->ctr->atomics : nullptr;
@@ -1091,6 +1169,7 @@ gps_status render_in_workspace(gps_scene* scene, const gps_frame_params* fp, int
     p.fb_words = words;
     p.fb_ss = ss;
     p.splat_mode = GPS_SPLAT_POINT_PARALLEL;
+    p.bin_ss = ss;  // no list
     p.hier_available = false;
     const uint32_t gpb = (uint32_t)std::max(4.0f, std::floor((float)N / (float)1e6));
     p.cull.gpb = gpb;

@@ -307,6 +307,13 @@ __device__ __forceinline__ float fp8_e4m3_to_float_hw(uint32_t, int) { return 0.
 // (gaussian_point_splatting.cu:605-615).
 void make_frame_consts(const gps_frame_params* fp, int spp, FrameConsts* f);
 
+// gps_pass_create with a point list of the binned splat of at most `max_list`
+// points (0: every frame is splatted point-parallel unless binning is forced),
+// the points that such a pass's list would take, and its bytes.
+gps_status pass_create(const gps_render_settings* st, gps_scene* scene, uint64_t max_list, gps_pass** out);
+uint64_t pass_list_points(const gps_render_settings* st, const gps_scene* scene);
+uint64_t pass_bytes(const gps_render_settings* st, const gps_scene* scene, uint64_t max_list);
+
 }  // namespace gps
 
 // Resident scene behind the gps_scene handle.

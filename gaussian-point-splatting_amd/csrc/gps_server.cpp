@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "../../include/gps.h"
+#include "gps_internal.h"
 
 namespace {
 
@@ -81,6 +82,7 @@ struct gps_server {
     uint64_t next_ticket = 1;
     uint64_t in_flight = 0;  // queued + running
     uint64_t budget = 0, used = 0;
+    uint64_t buffers = 0;  // of `used`: the slots' own
     uint64_t stamp = 0;
     gps_server_stats st{};
     std::string error;
@@ -110,6 +112,30 @@ gps_render_settings slot_settings(const gps_server* s) {
     return rs;
 }
 
+// Longest point list of `scene`'s passes.  The lists make a pass faster, not
+// possible, so they take what the budget has over: with room for every slot's
+// pass of every scene each list is full; with less each keeps about three
+// points per Gaussian (the memory that the passes took before their lists held
+// points, so a budget that held a set of passes then still does) and the same
+// share of the rest.
+uint64_t slot_list_points(const gps_server* s, int scene) {
+    const gps_render_settings rs = slot_settings(s);
+    uint64_t low = 0, more = 0, low_of = 0, more_of = 0;  // bytes of all passes; points of this scene's
+    for (int q = 0; q < (int)s->scenes.size(); ++q) {
+        const uint64_t full = gps::pass_list_points(&rs, s->scenes[q]);
+        const uint64_t n = 3ull * s->scenes[q]->view.N, few = std::min<uint64_t>(full, n > (1ull << 18) ? n - (1ull << 18) : 0);
+        low += s->slots.size() * gps::pass_bytes(&rs, s->scenes[q], few);
+        more += s->slots.size() * (gps::pass_bytes(&rs, s->scenes[q], full) - gps::pass_bytes(&rs, s->scenes[q], few));
+        if (q == scene) {
+            low_of = few;
+            more_of = full - few;
+        }
+    }
+    const uint64_t room = s->budget > s->buffers ? s->budget - s->buffers : 0;
+    if (room >= low + more) return low_of + more_of;
+    return room > low ? low_of + (uint64_t)((double)more_of * ((double)(room - low) / (double)more)) : low_of;
+}
+
 // Pass of `scene` on slot `k`, created (and others evicted) within budget.
 // Returns nullptr when the budget cannot hold it right now.
 gps_pass* slot_pass(gps_server* s, int k, int scene) {
@@ -119,7 +145,8 @@ gps_pass* slot_pass(gps_server* s, int k, int scene) {
         return sl.pass[scene];
     }
     const gps_render_settings rs = slot_settings(s);
-    const uint64_t need = gps_pass_estimate_bytes(&rs, s->scenes[scene]);
+    const uint64_t list = slot_list_points(s, scene);
+    const uint64_t need = gps::pass_bytes(&rs, s->scenes[scene], list);
     while (s->used + need > s->budget) {
         // Evict the least recently used pass held by an idle slot.
         int bk = -1, bs = -1;
@@ -140,7 +167,7 @@ gps_pass* slot_pass(gps_server* s, int k, int scene) {
         ++s->st.passes_evicted;
     }
     gps_pass* p = nullptr;
-    if (gps_pass_create(&rs, s->scenes[scene], &p) != GPS_OK) {
+    if (gps::pass_create(&rs, s->scenes[scene], list, &p) != GPS_OK) {
         s->error = std::string("pass create: ") + gps_last_error();
         return nullptr;
     }
@@ -297,6 +324,7 @@ gps_status gps_server_create(const gps_server_config* cfg, gps_server** out) {
         }
         s->used += px * 31;
     }
+    s->buffers = s->used;
     *out = s;
     return GPS_OK;
 }
@@ -317,7 +345,8 @@ gps_status gps_server_prepare(gps_server* s) {
     for (int q = 0; q < (int)s->scenes.size(); ++q)
         for (int k = 0; k < (int)s->slots.size(); ++k) {
             const gps_render_settings rs = slot_settings(s);
-            if (s->slots[k].pass[q] || s->used + gps_pass_estimate_bytes(&rs, s->scenes[q]) > s->budget) continue;
+            if (s->slots[k].pass[q] || s->used + gps::pass_bytes(&rs, s->scenes[q], slot_list_points(s, q)) > s->budget)
+                continue;
             if (!slot_pass(s, k, q)) return GPS_ERR_OUT_OF_MEMORY;
         }
     return hipDeviceSynchronize() == hipSuccess ? GPS_OK : GPS_ERR_HIP;

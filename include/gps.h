@@ -218,6 +218,12 @@ void gps_pass_destroy(gps_pass* pass);
 #define GPS_SPLAT_AUTO 0
 #define GPS_SPLAT_POINT_PARALLEL 1
 #define GPS_SPLAT_BINNED 2
+/* GPS_SPLAT_BINNED allocates: the binned buffers if the pass has none, and a
+ * list for twice the point budget (8 B a point, at most 2 GiB) if its list is
+ * shorter.  They stay until the pass is destroyed, as does the list that was
+ * there (a captured frame may write to it), also after a later GPS_SPLAT_AUTO.
+ * Without the memory the pass keeps what it has: frames with more points than
+ * its list holds, or all if it has none, splat point-parallel. */
 gps_status gps_pass_set_splat_mode(gps_pass* pass, int32_t mode);
 /* Diagnostic counters, off by default.  GPS_COUNT_ATOMICS: the splat's
  * global atomics into gps_stats.atomics (one atomic per workgroup on a single
@@ -256,7 +262,15 @@ gps_status gps_pass_set_group_culling(gps_pass* pass, int32_t enable);
 #define GPS_ORDERED_ALWAYS 2
 gps_status gps_pass_set_ordered_splat(gps_pass* pass, int32_t mode);
 /* Device memory held by the pass (scene not included), and what
- * gps_pass_create would allocate for these settings. */
+ * gps_pass_create allocates for these settings.  Where GPS_SPLAT_AUTO can bin
+ * frames of the settings both count the binned buffers: 16 B per Gaussian and
+ * 8 B per listed point: room for 16 points per output pixel where a point has
+ * at least 8 samples, in large framebuffers for 8 points per Gaussian or up to
+ * 40 per pixel, and for at most twice the point budget.  A pass that
+ * cannot have this part is created without it and splats point-parallel.  A
+ * frame of another supersampling factor than the pass's last reallocates
+ * framebuffers, and the list if it needs a longer one.  The estimate does not
+ * count what gps_pass_set_splat_mode adds. */
 uint64_t gps_pass_device_bytes(const gps_pass* pass);
 uint64_t gps_pass_estimate_bytes(const gps_render_settings* settings, const gps_scene* scene);
 
@@ -591,7 +605,8 @@ void gps_batch_destroy(gps_batch* batch);
  * thread admits every arrived request that finds an idle slot (HIP stream)
  * with a pass for its scene, or HBM budget to create one (evicting idle
  * passes least-recently-used); work of different slots overlaps on the
- * GPU.  Results are bit-identical whatever ran beside them. */
+ * GPU.  Point lists of the binned splat are as long as the budget leaves room
+ * for once every slot has a pass of every scene.  Results are bit-identical whatever ran beside them. */
 typedef struct gps_server gps_server;
 typedef struct gps_server_config {
     int32_t slots;                 /* requests in flight on the GPU, 1..64 */
