@@ -119,6 +119,7 @@ struct gps_pass {
     // occlusion
     HiZView hiz{};
     uint32_t hiz_size = 0;
+    bool hiz_written = false;  // a frame has built the chain (it starts with nothing occluded)
     CullNode* nodes = nullptr;
     uint32_t* cull_mask = nullptr;
     CullView cull{};
@@ -887,11 +888,22 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     } else {
         p->timing_slot = -1;
     }
+    // the automatic choice also tests the pass's density on the device
+    const uint32_t dense_points =
+        p->splat_mode == GPS_SPLAT_BINNED ? 0xFFFFFFFFu : binned_dense_points(f.up_w, f.up_h, f.spp, f.Ki, false);
+    const bool may_be_dense = 2ull * p->N > dense_points;
+    // The first frame with occlusion culling draws all that is in view in its first
+    // pass and next to nothing in the second.  Where the first may be too dense to
+    // bin, points of few samples are not worth the lists in either (25M Gaussians
+    // at 1080p, ss 2, us: lists, bounds and binned second pass 3076, without
+    // 2949).
+    const bool unculled = f.occl && !p->hiz_written && may_be_dense && f.Ki * f.spp < GPS_BIN_AUTO_SAMPLES;
     BinGeom bg_geom;
     // the biased splat adds colours per sample and has only the
     // point-parallel form
     const bool binned = f.unbiased && p->list.points && p->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
-                        (p->splat_mode == GPS_SPLAT_BINNED || binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, false)) &&
+                        (p->splat_mode == GPS_SPLAT_BINNED ||
+                         (!unculled && binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, false))) &&
                         binned_geometry(f.up_w, f.up_h, f.spp, &bg_geom);
     stage_mark(p, 0, 0, 0, st);
     // The clear also resets the per-frame counters (pass results, culled
@@ -943,10 +955,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
         a.cull = p->cull;
         a.hiz = p->hiz;
         a.gocc = group_test ? p->gocc : nullptr;
-        // the automatic choice also tests the pass's density on the device
-        const uint32_t dense_points =
-            p->splat_mode == GPS_SPLAT_BINNED ? 0xFFFFFFFFu : binned_dense_points(f.up_w, f.up_h, f.spp, f.Ki, false);
-        a.bounds = binned && (f.occl || 2ull * p->N <= dense_points) ? p->bounds : nullptr;
+        a.bounds = binned && (f.occl || !may_be_dense) ? p->bounds : nullptr;
         if (live_mode) a.wg_live = p->wg_live;
         a.rejects = p->count_rejects ? &p->ctr->rejects[0][0] : nullptr;
         stage_mark(p, 2, slot, 0, st);
@@ -1081,6 +1090,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
         stage_mark(p, 6, 1, 1, st);
     }
     p->last_occl = fp->enable_occlusion_culling ? 1 : 0;
+    p->hiz_written |= fp->enable_occlusion_culling != 0;
     p->last_hier = f.hier;
     p->last_K = f.Ki;
     p->last_spp = f.spp;

@@ -211,8 +211,11 @@ void gps_pass_destroy(gps_pass* pass);
  * denser passes splat point-parallel and report gps_stats.splat_fallback = 2).
  * Framebuffers of more than 2^22 words (upscaled width * height * spp; 2^20 in
  * a batch) take wider limits: 4 samples per point if the scene has a Gaussian
- * per 16 words and, in a single pass, at most 4 per word, and 6 samples per word for every 2^22 words, up to 32 (32 in a
- * batch).  All give the same framebuffer bit for bit.  No reference counterpart
+ * per 16 words and, in a single pass, at most 4 per word, and 6 samples per
+ * word for every 2^22 words, up to 32 (32 in a batch).  A pass's first frame
+ * with occlusion culling, which nothing culls, takes the 4-sample limit only
+ * in scenes too small to be too dense (twice as many points as Gaussians).
+ * All give the same framebuffer bit for bit.  No reference counterpart
  * (the reference has only the point-parallel form,
  * gaussian_point_splatting.cu:383-432). */
 #define GPS_SPLAT_AUTO 0

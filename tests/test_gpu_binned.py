@@ -62,3 +62,21 @@ def test_binned_auto_large_framebuffer(gpu):
     a, b = _frames(gpu, arrays, 1400, 780, 2, 1, (0.0, 3.0, -25.0), (gpu.Pass.SPLAT_AUTO, gpu.Pass.SPLAT_POINT_PARALLEL))
     assert a.stats["splat_binned"] == 1 and a.stats["splat_fallback"] == 0, a.stats
     _same(gpu, a, b, "large framebuffer")
+
+
+def test_first_culled_frame_is_point_parallel(gpu):
+    """4 samples a point in a scene that may be too dense to bin: the first
+    frame with occlusion culling, which nothing culls, takes no lists; later
+    ones do.  The same images as point-parallel throughout."""
+    arrays = H.scene(0x5EED0831, 4_500_000, dict(H.C1, half_extent=30.0, log_scale_mu=-4.0)).morton_sorted()
+    w, h = 1400, 780
+    st = gpu.RenderSettings(w, h, 1, 2, gaussians_per_block=256)
+    a, b = H.GpuRunner(arrays, st), H.GpuRunner(arrays, st)
+    b.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
+    for k in range(3):
+        f = gpu.frame_params((0.1 * k, 3.0, -20.0), (0, 0, 0), (0, 1, 0), 45.0, w, h, ss=2, frame=k + 1,
+                             occlusion=True, hierarchical=True, background=(0.2, 0.4, 0.6))
+        flush(f"first culled frame: frame {k}")
+        x, y = (r.render(f, [gpu.DBG_FRAMEBUFFER]) for r in (a, b))
+        assert x.stats["splat_binned"] == (0 if k == 0 else 1), (k, x.stats)
+        _same(gpu, x, y, f"frame {k}")
