@@ -2670,17 +2670,20 @@ __device__ __forceinline__ uint32_t rgb8_byte(float c) {
     return (uint32_t)(uint8_t)__builtin_roundf(glm_clamp(c, 0.0f, 1.0f) * 255.0f);
 }
 
-// TAA over tiles of 64x16 pixels, four rows of one column per thread.  A wave
+// TAA over tiles of 64x8 pixels, two rows of one column per thread.  A wave
 // reading a colour image at 12 bytes a lane takes as many cycles for 4 bytes as
 // for 12, and the 3x3 neighbourhood needs 27 words a pixel, so the tile's colours
 // with a rim of one pixel pass through LDS (the rim clamped to the image: a
 // pixel of the neighbourhood again), a thread's row minima and maxima serve
-// three of its pixels, the history is read 12 bytes at a time, and the bytes of
+// both of its pixels, the history is read 12 bytes at a time, and the bytes of
 // a row leave as words, put together from two lanes' pixels (rows and image on 4-byte
 // boundaries; else byte by byte).  Each XCD has a band of the image (workgroups
 // go round the XCDs), so that rims and history hit its own L2: without, half as
-// much again came from memory.  3840x2160: 144 -> 101 us (358 MB to move).
-constexpr int TAA_W = 64, TAA_ROWS = 4, TAA_H = 4 * TAA_ROWS, TAA_PITCH = 3 * (TAA_W + 2);
+// much again came from memory.  3840x2160: 144 -> 90 us (358 MB to move).  Back
+// to back, us, without LDS / 1 / 2 / 4 rows a thread: 320x180 5.6 / 5.6 / 5.5 / 6.2,
+// 640x480 6.3 / 5.9 / 6.1 / 7.4, 1920x1080 27.1 / 21.7 / 19.7 / 20.5, 3840x2160 129.9
+// / 89.9 / 76.6 / 80.6.
+constexpr int TAA_W = 64, TAA_ROWS = 2, TAA_H = 4 * TAA_ROWS, TAA_PITCH = 3 * (TAA_W + 2);
 __global__ __launch_bounds__(256) void taa_kernel(const float* __restrict__ cur, const float* __restrict__ cur_depth,
                                                   const float* __restrict__ prev, Mat4 M, float blend, int W, int H,
                                                   int frame_number, float* __restrict__ out, uint8_t* __restrict__ rgb8,
@@ -2689,7 +2692,11 @@ __global__ __launch_bounds__(256) void taa_kernel(const float* __restrict__ cur,
     const int tile = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);
     if (tile >= tiles) return;
     const int bx = tile % tiles_x * TAA_W, by = tile / tiles_x * TAA_H;
-    {
+    const int lane = threadIdx.x & 63, ly0 = (threadIdx.x >> 6) * TAA_ROWS;
+    const int x = bx + lane;
+    const bool in_x = x < W;
+    float mn[TAA_ROWS + 2][3], mx[TAA_ROWS + 2][3], mid[TAA_ROWS][3];
+    if (frame_number > 0) {
         constexpr int N = (TAA_H + 2) * TAA_PITCH, PER = (N + 255) / 256;
         float v[PER];  // all of a thread's loads are in flight together
 #pragma unroll
@@ -2702,21 +2709,24 @@ __global__ __launch_bounds__(256) void taa_kernel(const float* __restrict__ cur,
 #pragma unroll
         for (int k = 0; k < PER; ++k)
             if ((int)threadIdx.x + 256 * k < N) s[threadIdx.x + 256 * k] = v[k];
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, ly0 = (threadIdx.x >> 6) * TAA_ROWS;
-    const int x = bx + lane;
-    const bool in_x = x < W;
-    float mn[TAA_ROWS + 2][3], mx[TAA_ROWS + 2][3], mid[TAA_ROWS][3];
+        __syncthreads();
 #pragma unroll
-    for (int r = 0; r < TAA_ROWS + 2; ++r) {
-        const float* q = s + (ly0 + r) * TAA_PITCH + 3 * lane;
+        for (int r = 0; r < TAA_ROWS + 2; ++r) {
+            const float* q = s + (ly0 + r) * TAA_PITCH + 3 * lane;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const float v0 = q[k], v1 = q[3 + k], v2 = q[6 + k];
-            mn[r][k] = __builtin_fminf(__builtin_fminf(v0, v1), v2);
-            mx[r][k] = __builtin_fmaxf(__builtin_fmaxf(v0, v1), v2);
-            if (r >= 1 && r <= TAA_ROWS) mid[r - 1][k] = v1;
+            for (int k = 0; k < 3; ++k) {
+                const float v0 = q[k], v1 = q[3 + k], v2 = q[6 + k];
+                mn[r][k] = __builtin_fminf(__builtin_fminf(v0, v1), v2);
+                mx[r][k] = __builtin_fmaxf(__builtin_fmaxf(v0, v1), v2);
+                if (r >= 1 && r <= TAA_ROWS) mid[r - 1][k] = v1;
+            }
+        }
+    } else {  // the first frame: no history, so no neighbourhood
+#pragma unroll
+        for (int r = 0; r < TAA_ROWS; ++r) {
+            const int gx = min(x, W - 1), gy = min(by + ly0 + r, H - 1);
+            const Rgb v = reinterpret_cast<const Rgb*>(cur)[(int64_t)gy * W + gx];
+            mid[r][0] = v.r, mid[r][1] = v.g, mid[r][2] = v.b;
         }
     }
     const float cx = ((float)x + 0.5f) / (float)W * 2.0f - 1.0f;
