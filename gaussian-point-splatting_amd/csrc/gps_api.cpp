@@ -1262,7 +1262,7 @@ gps_status gps_pass_stats(gps_pass* p, gps_stats* out, void* stream) {
         out->splat_fallback = (int32_t)bs[3];
         out->bin_entries = bs[0];
         out->bin_jobs = bs[1];
-        out->bin_big = bs[2];
+        out->bin_big = bs[6];
     }
     if (p->hier_available) {
         out->gaussians_per_block = (int32_t)p->cull.gpb;

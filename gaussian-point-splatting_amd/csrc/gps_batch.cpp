@@ -566,7 +566,7 @@ gps_status gps_batch_view_stats(gps_batch* b, int32_t view, gps_stats* out, void
         out->splat_fallback = st[3] ? 1 : dense ? 2 : 0;
         out->bin_entries = st[0];  // whole batch
         out->bin_jobs = st[1];
-        out->bin_big = st[2];
+        out->bin_big = st[6];
     }
     return GPS_OK;
 }

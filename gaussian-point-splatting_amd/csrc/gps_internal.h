@@ -110,9 +110,9 @@ struct FrameCounters {
     uint32_t rejects[2][9];  // per pass: preprocess reject reasons (diagnostic; see RejectReason)
     uint32_t group_violations[2];  // per pass, with the reasons: members of culled groups that survived (must be 0)
     uint32_t ordered_skipped[2];   // per pass, with the reasons: points the ordered splat skipped (diagnostic)
-    uint32_t bin_state[2][8];      // per pass: the binned splat's counters (BinnedArgs::state)
+    alignas(8) uint32_t bin_state[2][8];  // per pass: the binned splat's counters (BinnedArgs::state)
 };
-static_assert(sizeof(FrameCounters) == 220, "counter words zeroed by the clear kernel");
+static_assert(sizeof(FrameCounters) == 224, "counter words zeroed by the clear kernel");
 
 // Region geometry of the binned splat for one framebuffer.
 struct BinGeom {
@@ -203,6 +203,7 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 #define GPS_BIN_WORDS 16384u
 #define GPS_BIN_LDS_WORDS 17408u
 #define GPS_BIN_MAX_REGIONS 4u
+#define GPS_BIN_MAX_POINTS 16384u  // per Gaussian
 #define GPS_BIN_HIST 8192u
 #define GPS_BIN_JOB_POINTS 2048u       // smallest full job (bin_scan_kernel)
 #define GPS_BIN_JOB_POINTS_MAX 32768u

@@ -121,8 +121,8 @@ struct BinnedArgs {
     uint32_t *job_reg, *job_p0;
     uint2* list;          // (record, point) of every point and region, region by region
     BigList big;
-    uint32_t* state;      // 8 words: (entry, region) pairs, jobs, big Gaussians, stand-down, job cursor, a tile's
-                          // points did not fit their sums, further slices, points per job
+    uint32_t* state;      // 8 words: (entry, region) pairs, jobs, points per job, stand-down, job cursor, unused,
+                          // big Gaussians and further slices (one 64-bit counter)
     uint32_t list_cap, job_cap;
     uint32_t cus;
     uint32_t dense_points;  // more points than this: the binned kernels stand down (state[3] = 2)

@@ -1069,6 +1069,15 @@ __device__ __forceinline__ BinRect bounds_rect(const BinGeom& g, uint2 b, uint32
     return q;
 }
 
+// Whether an entry of w points is left to the point-parallel splat: each of too
+// many regions would replay it, or it is too long for the one wave that writes
+// its points to the lists.
+__device__ __forceinline__ bool too_large(const BinRect& q, uint32_t w) {
+    return q.n > GPS_BIN_MAX_REGIONS || (q.n != 0u && w > GPS_BIN_MAX_POINTS);
+}
+static_assert((uint64_t)GPS_TILE * GPS_BIN_MAX_POINTS < 1ull << 32, "a tile's points per region are 32-bit sums");
+static_assert((uint64_t)GPS_LIST_ENTRIES * GPS_BIN_MAX_POINTS < 1ull << 32, "as are those of a step of the lists");
+
 // Counting for the binned splat, done by the distributor while it holds the
 // counts (a kernel of its own read the compacted lists again: 57 us at 7.7M
 // valid Gaussians).  state[0]: (entry, region) pairs.
@@ -1113,7 +1122,6 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
     extern __shared__ uint32_t s_pts[];  // BIN: the regions of the frame, or of the batch's largest view
     __shared__ uint32_t s_a[4], s_c[4];
     __shared__ uint4 s_fold[4];
-    __shared__ uint32_t s_units;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t tile = blockIdx.x;
     uint32_t v0, vend, a0;
@@ -1213,10 +1221,8 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
             bc.f.p_end = (uint32_t)P;
             bin = P <= bc.dense_points;  // else too dense to bin: bin_scan_kernel stands the binned kernels down
         }
-        if (bin) {
-            if (tid == 0) s_units = 0u;
+        if (bin)
             for (uint32_t i = (uint32_t)tid; i < bc.f.g.nregions; i += 256u) s_pts[i] = 0u;
-        }
     }
     const uint4* wp = reinterpret_cast<const uint4*>(weights + g0);
     // Groups of 4 without a live element re-read the first live group's
@@ -1266,30 +1272,25 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
         uint2 bnd[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) bnd[k] = w[k] ? record_bounds(bc.f, g0 + (uint32_t)k) : make_uint2(0u, 0u);
-        uint32_t o = off, rr = r, pairs = 0u, units = 0u;
+        uint32_t o = off, rr = r, pairs = 0u;
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
             if (!w[k]) continue;
             const uint32_t hi = min(o + w[k], bc.f.p_end);
             const uint32_t pts = o < hi ? hi - o : 0u;
             const BinRect q = bounds_rect(bc.f.g, bnd[k], pts);
-            if (q.n > GPS_BIN_MAX_REGIONS) {
-                // too large to bin: its points in slices (a few hold hundreds
-                // of thousands), which splat_big and batch_bin_big_kernel take
-                // one by one
-                const uint32_t start = big_items(
-                    pts, bc.big.slice_cap,
-                    [&](uint32_t n) {  // full: not counted further, the counter must not wrap
-                        return __hip_atomic_load(&bc.state[6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-                                       bc.big.slice_cap
-                                   ? atomicAdd(&bc.state[6], n)
-                                   : bc.big.slice_cap;
-                    },
-                    [&](uint32_t i, uint32_t s) { bc.big.items[bc.big.slice0 + i] = make_uint2(rr, s); });
-                bc.big.items[atomicAdd(&bc.state[2], 1u)] = make_uint2(rr, start);
+            if (too_large(q, pts)) {
+                // its points in slices (a few hold hundreds of thousands),
+                // which splat_big and batch_bin_big_kernel take one by one
+                const uint32_t rest = big_rest(pts, bc.big.slice_cap);
+                const uint64_t at = atomicAdd(reinterpret_cast<unsigned long long*>(&bc.state[6]),
+                                              ((unsigned long long)rest << 32) + 1ull);
+                bc.big.items[(uint32_t)at] = make_uint2(
+                    rr, big_items(pts, rest, (uint32_t)(at >> 32), bc.big.slice_cap, [&](uint32_t i, uint32_t s) {
+                        bc.big.items[bc.big.slice0 + i] = make_uint2(rr, s);
+                    }));
             } else if (q.n) {
                 pairs += q.n;
-                units += point_units(pts);
                 for (uint32_t ry = q.ry0; ry <= q.ry1; ++ry)
                     for (uint32_t rx = q.rx0; rx <= q.rx1; ++rx)
                         atomicAdd(&s_pts[ry * (uint32_t)bc.f.g.nrx + rx], pts);
@@ -1297,9 +1298,7 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
             o += w[k];
             ++rr;
         }
-        if (units) atomicAdd(&s_units, units);
         add_count(&bc.state[0], pairs);  // (its barriers order the histogram too)
-        if (tid == 0 && tile_too_large(s_units)) bc.state[5] = 1u;  // no list is long enough
         for (uint32_t i = (uint32_t)tid; i < bc.f.g.nregions; i += 256u)
             if (s_pts[i]) atomicAdd(&bc.reg_pts[bc.f.rbase + i], (unsigned long long)s_pts[i]);
     }
@@ -1632,10 +1631,10 @@ struct BigSlices {
 };
 // Item e of the list, first slices first.
 __device__ __forceinline__ uint32_t big_count(const BigList& b, const uint32_t* __restrict__ state) {
-    return state[2] + min(state[6], b.slice_cap);
+    return state[6] + min(state[7], b.slice_cap);
 }
 __device__ __forceinline__ uint2 big_item(const BigList& b, const uint32_t* __restrict__ state, uint32_t e) {
-    const uint32_t n = state[2];
+    const uint32_t n = state[6];
     return b.items[e < n ? e : b.slice0 + (e - n)];
 }
 __device__ __forceinline__ uint32_t splat_big(const BigSlices& b, const SplatRecord* __restrict__ recs,
@@ -1912,7 +1911,7 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_ordered_kernel(
 // point-parallel splat runs instead.
 
 // One workgroup: the regions' list offsets, and the job table: jobs of at most
-// state[7] points, the largest first (eight size classes), so that the
+// state[2] points, the largest first (eight size classes), so that the
 // persistent splat does not end on a long one.  Large jobs start and store
 // fewer regions twice, small ones share out evenly: a little more than one a CU
 // between GPS_BIN_JOB_POINTS and 32768 points (splat, us, at 8192 / 16384 /
@@ -1984,12 +1983,12 @@ __global__ __launch_bounds__(1024) void bin_scan_kernel(uint32_t nregions, unsig
         s_jobs = run;
         const bool dense = ctr && ctr->points > dense_points;
         state[1] = min(run, job_cap);
-        state[3] = dense ? 2u : (s_carry > list_cap || run > job_cap || state[5]) ? 1u : 0u;
+        state[2] = job_points;
+        state[3] = dense ? 2u : (s_carry > list_cap || run > job_cap) ? 1u : 0u;
         state[4] = 0u;
-        state[7] = job_points;
     }
     __syncthreads();
-    if (s_jobs > job_cap || s_carry > list_cap || state[5]) return;
+    if (s_jobs > job_cap || s_carry > list_cap) return;
     for (uint32_t i = (uint32_t)tid; i < nregions; i += 1024) {
         const uint32_t p32 = reg_ptot[i];
         const uint32_t full = p32 / job_points, rest = p32 - full * job_points;
@@ -2042,7 +2041,7 @@ __device__ __forceinline__ void bin_scatter_range(const BinFrame& f, uint32_t r0
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             const BinRect q = bounds_rect(f.g, bnd[k], w[k]);
-            if (q.n == 0u || q.n > GPS_BIN_MAX_REGIONS) continue;
+            if (q.n == 0u || too_large(q, w[k])) continue;
             for (uint32_t ry = q.ry0; ry <= q.ry1; ++ry)
                 for (uint32_t rx = q.rx0; rx <= q.rx1; ++rx) atomicAdd(&s_pos[ry * nrx + rx], w[k]);
         }
@@ -2053,7 +2052,7 @@ __device__ __forceinline__ void bin_scatter_range(const BinFrame& f, uint32_t r0
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             BinRect q = bounds_rect(f.g, bnd[k], w[k]);
-            if (q.n > GPS_BIN_MAX_REGIONS) q.n = 0u;
+            if (too_large(q, w[k])) q.n = 0u;
             const uint32_t pk = p[k] - pbias, wk = w[k], rk = rec[k];
             uint32_t rx = q.rx0, ry = q.ry0;
             for (uint32_t j = 0; __ballot(j < q.n) != 0ull; ++j) {
@@ -2122,7 +2121,7 @@ __global__ __launch_bounds__(GPS_LIST_THREADS) void bin_scatter_kernel(BinFrame 
                                                                        unsigned long long* __restrict__ fb,
                                                                        uint64_t clear_words, uint64_t background) {
     extern __shared__ uint32_t s_dyn[];  // nregions words
-    if (clear_words) bin_clear(f.g, 0u, reg_ptot, state[7], state[3] != 0u, clear_words, background, fb);
+    if (clear_words) bin_clear(f.g, 0u, reg_ptot, state[2], state[3] != 0u, clear_words, background, fb);
     if (state[3]) return;
     f.v_end = ctr->valid;
     f.t_end = ctr->total;
@@ -2285,7 +2284,7 @@ __global__ __launch_bounds__(GPS_BIN_THREADS) void bin_splat_kernel(
     __shared__ unsigned long long s_fb[GPS_BIN_LDS_WORDS];
     __shared__ uint32_t s_job;
     if (state[3]) return;
-    const uint32_t njobs = state[1], job_points = state[7];
+    const uint32_t njobs = state[1], job_points = state[2];
     uint32_t merged = 0;
     for (;;) {
         if (threadIdx.x == 0) s_job = atomicAdd(&state[4], 1u);
@@ -2315,7 +2314,7 @@ __global__ __launch_bounds__(GPS_LIST_THREADS) void batch_bin_scatter_kernel(
     const BatchView& bv = views[blockIdx.y];
     if (bv.bg.nregions == 0u) return;  // cleared by batch_clear_kernel
     const bool pp = state[3] != 0u || bv.points > bv.dense_points;
-    bin_clear(bv.bg, bv.rbase, reg_ptot, state[7], pp, bv.fb_words, bv.background, fb + bv.fb_offset);
+    bin_clear(bv.bg, bv.rbase, reg_ptot, state[2], pp, bv.fb_words, bv.background, fb + bv.fb_offset);
     if (pp) return;
     f.g = bv.bg;
     if (!bv.write_bounds) f.bounds = nullptr;
@@ -2347,7 +2346,7 @@ __global__ __launch_bounds__(GPS_BIN_THREADS) void batch_bin_splat_kernel(
     __shared__ uint32_t s_job;
     __shared__ int s_view;
     if (state[3]) return;
-    const uint32_t njobs = state[1], job_points = state[7];
+    const uint32_t njobs = state[1], job_points = state[2];
     uint32_t merged = 0;
     for (;;) {
         if (threadIdx.x == 0) {

@@ -143,7 +143,7 @@ typedef struct gps_stats {
                                       2 too many samples per framebuffer word (GPS_SPLAT_AUTO) */
     uint32_t bin_entries;          /* (Gaussian, region) pairs of the last pass */
     uint32_t bin_jobs;             /* region jobs of the last pass */
-    uint32_t bin_big;              /* Gaussians splatted with global atomics (too many regions) */
+    uint32_t bin_big;              /* Gaussians splatted with global atomics (too many regions or points) */
     uint32_t reserved;
     uint64_t culled_groups[2];     /* per pass: 64-Gaussian groups the group occlusion test skipped
                                       (counted with gps_pass_set_counters flags on, else 0) */

@@ -1,11 +1,9 @@
-// The bounds of the binned splat's lists (gps_big.h, the source the GPU
+// The bounds of the list of large Gaussians (gps_big.h, the source the GPU
 // distributor compiles) on the CPU, as the distributor uses them: Gaussians
 // get 32-bit offsets that wrap past 2^32, and the points of each that lie
 // below the budget.
-//   items:  no item outside its range, every point of every Gaussian too large
-//           to bin in an item, and each once while nothing wraps
-//   sums:   a tile whose 32-bit sum would wrap is noticed, one of less than
-//           2^31 points never is
+// no item may lie outside its range, every point of every Gaussian must be in an
+// item, and each once while nothing wraps.
 // argv: Gaussians, points each (at most), budget, seed.  Prints the number of
 // Gaussians with points, the turns, the items' shortfall and the faults.
 #include <cstdio>
@@ -27,8 +25,8 @@ int main(int, char** argv) {
     std::vector<Item> first, shared(cap, Item{0, 0});
     std::vector<uint8_t> written(cap, 0);
     std::vector<uint32_t> pts(n);
-    uint64_t total = 0, faults = 0, all = 0, with = 0, sum = 0, wide = 0;
-    uint32_t used = 0, tile = 0, flagged = 0;
+    uint64_t total = 0, faults = 0, all = 0, with = 0;
+    uint32_t used = 0;
     std::vector<uint32_t> w(n);
     for (uint32_t r = 0; r < n; ++r) {
         x ^= x << 13, x ^= x >> 7, x ^= x << 17;
@@ -43,21 +41,15 @@ int main(int, char** argv) {
         o += w[r];
         if (pts[r]) {
             ++with;
-            const uint32_t start = big_items(
-                pts[r], cap, [&](uint32_t k) { return used < cap ? (used += k) - k : cap; },
-                [&](uint32_t i, uint32_t s) {
-                    if (i >= cap || written[i]) ++faults;
-                    else shared[i] = Item{r, s}, written[i] = 1;
-                });
+            const uint32_t rest = big_rest(pts[r], cap), at = used;
+            used += rest;
+            const uint32_t start = big_items(pts[r], rest, at, cap, [&](uint32_t i, uint32_t s) {
+                if (i >= cap || written[i]) ++faults;
+                else shared[i] = Item{r, s}, written[i] = 1;
+            });
             first.push_back(Item{r, start});
             all += start == GPS_BIG_ALL;
         }
-        // one region takes every point of the tile's 4096 Gaussians
-        if (r % 4096 == 0) tile = 0, sum = 0, wide += flagged, flagged = 0;
-        tile += point_units(pts[r]);
-        sum += pts[r];
-        flagged = tile_too_large(tile);
-        if ((sum >= (1ull << 32) && !flagged) || (sum < (1ull << 31) && flagged)) ++faults;
     }
     const uint32_t n2 = used < cap ? used : cap;
     std::vector<uint64_t> covered(n, 0);
@@ -73,8 +65,7 @@ int main(int, char** argv) {
     for (uint32_t r = 0; r < n; ++r)
         if (covered[r] < pts[r] || (total < (1ull << 32) && covered[r] != pts[r])) ++faults;
     if (first.size() > n) ++faults;
-    std::printf("with %llu turns %llu short %llu wide %llu faults %llu\n", (unsigned long long)with,
-                (unsigned long long)(total >> 32), (unsigned long long)all, (unsigned long long)(wide + flagged),
-                (unsigned long long)faults);
+    std::printf("with %llu turns %llu short %llu faults %llu\n", (unsigned long long)with,
+                (unsigned long long)(total >> 32), (unsigned long long)all, (unsigned long long)faults);
     return 0;
 }

@@ -55,6 +55,19 @@ def test_binned_big_gaussians(gpu, n):
     _same(gpu, a, b, f"{n} Gaussians")
 
 
+@pytest.mark.parametrize("spp", [1, 4])
+def test_binned_long_gaussians(gpu, spp):
+    """Gaussians in few regions with more points than one wave should list
+    (16384; a frame of 240 x 240 pixels allows one 28800)."""
+    arrays = H.scene(0x5EED0841, 2000, dict(H.C1, half_extent=3.0, log_scale_mu=-3.0)).morton_sorted()
+    arrays.scales[::500] = np.float32(40.0)
+    arrays.opacities[::500] = np.float32(0.9)
+    a, b = _frames(gpu, arrays, 240, 240, 1, spp, (0.0, 1.0, -9.0), (gpu.Pass.SPLAT_BINNED, gpu.Pass.SPLAT_POINT_PARALLEL))
+    assert a.stats["splat_fallback"] == 0 and a.stats["num_points"][0] > 4 * 16384, a.stats
+    assert (a.stats["bin_big"] >= 4) if spp < 3 else (a.stats["bin_big"] >= 1), a.stats
+    _same(gpu, a, b, f"spp {spp}")
+
+
 def test_binned_auto_large_framebuffer(gpu):
     """More than 2^22 framebuffer words: 4 samples a point are binned too, and
     passes of up to 6 samples per word and 2^22 words."""
