@@ -199,7 +199,6 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 // 1576, 1024 x 2 136 / 970, 1024 x 4 126 / 658, 512 x 8 124 / 617).
 #define GPS_LIST_THREADS 512
 #define GPS_LIST_WGS_PER_CU 8
-#define GPS_LIST_ENTRIES 4096  // entries of one step
 #define GPS_BIN_WORDS 16384u
 #define GPS_BIN_LDS_WORDS 17408u
 #define GPS_BIN_MAX_REGIONS 4u

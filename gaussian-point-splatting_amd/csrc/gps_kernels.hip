@@ -1076,7 +1076,7 @@ __device__ __forceinline__ bool too_large(const BinRect& q, uint32_t w) {
     return q.n > GPS_BIN_MAX_REGIONS || (q.n != 0u && w > GPS_BIN_MAX_POINTS);
 }
 static_assert((uint64_t)GPS_TILE * GPS_BIN_MAX_POINTS < 1ull << 32, "a tile's points per region are 32-bit sums");
-static_assert((uint64_t)GPS_LIST_ENTRIES * GPS_BIN_MAX_POINTS < 1ull << 32, "as are those of a step of the lists");
+static_assert((uint64_t)GPS_LIST_THREADS * 8 * GPS_BIN_MAX_POINTS < 1ull << 32, "as are those of a step of the lists");
 
 // Counting for the binned splat, done by the distributor while it holds the
 // counts (a kernel of its own read the compacted lists again: 57 us at 7.7M
@@ -2007,7 +2007,7 @@ __global__ __launch_bounds__(1024) void bin_scan_kernel(uint32_t nregions, unsig
     }
 }
 
-// Point lists of the regions, 4096 entries at a time: the workgroup adds up
+// Point lists of the regions, PER entries a thread at a time: the workgroup adds up
 // its entries' points per region in LDS (the Morton-ordered entries touch few
 // regions), reserves one range per region with a single global atomic, and
 // fills it.  The entries stay in registers in between.  A lane writes the
@@ -2015,13 +2015,14 @@ __global__ __launch_bounds__(1024) void bin_scan_kernel(uint32_t nregions, unsig
 // over the wave's lanes by prefix sums measured 180 us against 145 at 20M
 // points); an entry of more than 16 points is written by its whole wave.
 // `pbias` turns point offsets into the frame's own indices.
-__device__ __forceinline__ void bin_scatter_range(const BinFrame& f, uint32_t r0, uint32_t r1, uint32_t pbias,
+template <int PER>
+__device__ __forceinline__ void bin_scatter_steps(const BinFrame& f, uint32_t r0, uint32_t r1, uint32_t pbias,
                                                   uint32_t* __restrict__ reg_cursor, uint2* __restrict__ list,
                                                   uint32_t* s_pos) {
-    constexpr int PER = GPS_LIST_ENTRIES / GPS_LIST_THREADS;
+    constexpr uint32_t STEP = PER * GPS_LIST_THREADS;
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t nrx = (uint32_t)f.g.nrx;
-    for (uint32_t base = r0 + blockIdx.x * GPS_LIST_ENTRIES; base < r1; base += gridDim.x * GPS_LIST_ENTRIES) {
+    for (uint32_t base = r0 + blockIdx.x * STEP; base < r1; base += gridDim.x * STEP) {
         for (uint32_t i = tid; i < f.g.nregions; i += GPS_LIST_THREADS) s_pos[i] = 0u;
         uint32_t rec[PER], p[PER], w[PER];
         uint2 bnd[PER];
@@ -2079,6 +2080,18 @@ __device__ __forceinline__ void bin_scatter_range(const BinFrame& f, uint32_t r0
         }
         __syncthreads();
     }
+}
+// Few entries are shared out in smaller steps: a wave writes the longer entries
+// one after another (2M close-up Gaussians, 0.6M of them valid with 9 points
+// each: 353 us in steps of 4096, 78 in steps of 512).
+__device__ __forceinline__ void bin_scatter_range(const BinFrame& f, uint32_t r0, uint32_t r1, uint32_t pbias,
+                                                  uint32_t* __restrict__ reg_cursor, uint2* __restrict__ list,
+                                                  uint32_t* s_pos) {
+    const uint32_t per = (uint32_t)((uint64_t)(r1 - r0) / (gridDim.x * (uint64_t)GPS_LIST_THREADS));
+    if (per < 1u) bin_scatter_steps<1>(f, r0, r1, pbias, reg_cursor, list, s_pos);
+    else if (per < 2u) bin_scatter_steps<2>(f, r0, r1, pbias, reg_cursor, list, s_pos);
+    else if (per < 4u) bin_scatter_steps<4>(f, r0, r1, pbias, reg_cursor, list, s_pos);
+    else bin_scatter_steps<8>(f, r0, r1, pbias, reg_cursor, list, s_pos);
 }
 
 // The frame's clear, where the binned splat does not make it needless: with

@@ -68,6 +68,32 @@ def test_binned_long_gaussians(gpu, spp):
     _same(gpu, a, b, f"spp {spp}")
 
 
+@pytest.mark.parametrize("n", [30_000, 90_000, 190_000, 400_000])
+def test_binned_batch_list_steps(gpu, n):
+    """Lists written in steps of 1, 2, 4 and 8 entries a thread (16 views share
+    the workgroups: 65536 threads each), ragged at the end."""
+    w, h, v = 160, 90, 16
+    arrays = H.scene(0x5EED0851, n + 37, dict(H.C1, half_extent=6.0, log_scale_mu=-3.0))
+    scene, stream = gpu.Scene(arrays), gpu.Stream()
+    frames = [gpu.frame_params((0.1 * i, 1.0, -22.0), (0, 0, 0), (0, 1, 0), 45.0, w, h, ss=2, frame=2 + i, spp=2)
+              for i in range(v)]
+    out = [(gpu.DeviceArray((h, w, 3), np.float32, zero=True), gpu.DeviceArray((h, w), np.float32, zero=True))
+           for _ in range(v)]
+    got = []
+    for mode in (gpu.Pass.SPLAT_BINNED, gpu.Pass.SPLAT_POINT_PARALLEL):
+        flush(f"list steps n {n} mode {mode}")
+        b = gpu.Batch(scene, v, w, h, 2, 2)
+        b.set_splat_mode(mode)
+        b.render(frames, [c for c, _ in out], [d for _, d in out], stream)
+        stats = b.view_stats(0, stream)
+        assert stats["splat_binned"] == (mode == gpu.Pass.SPLAT_BINNED) and stats["splat_fallback"] == 0, stats
+        got.append([(c.download(), d.download()) for c, d in out])
+        b.close()
+    for i, (x, y) in enumerate(zip(*got)):
+        assert_same(f"view {i} colour", x[0], y[0])
+        assert_same(f"view {i} depth", x[1], y[1])
+
+
 def test_binned_auto_large_framebuffer(gpu):
     """More than 2^22 framebuffer words: 4 samples a point are binned too, and
     passes of up to 6 samples per word and 2^22 words."""
