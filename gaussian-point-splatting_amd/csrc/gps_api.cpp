@@ -211,9 +211,9 @@ gps_status ensure_fb(gps_pass* p, int ss, uint64_t frame_words) {
 // size at supersampling `ss`, 0 where it bins none of them (a frame's points
 // have ss^2 or 1 samples per layer).  Gaussians that straddle regions are listed
 // in each, 1.15 to 1.3 times in all: room twice for GPS_BIN_DENSE_SAMPLES per
-// framebuffer word, and 1.25 times for what only large framebuffers take (there
-// at most 8 per Gaussian, which scenes of millions do not reach, but two per
-// Gaussian twice); never more than the point budget twice.
+// framebuffer word (points of few samples: at most for 16 per Gaussian), and
+// 1.25 times for the denser frames that large framebuffers take (at most 8 per
+// Gaussian, but two per Gaussian twice); never more than the point budget twice.
 uint64_t bin_list_points(const gps_render_settings& st, int ss, uint64_t N) {
     const uint64_t up = (uint64_t)st.width * ss * (uint64_t)st.height * ss;
     uint64_t need = 0;
@@ -222,12 +222,14 @@ uint64_t bin_list_points(const gps_render_settings& st, int ss, uint64_t N) {
             BinGeom g;
             const bool can = st.flexible_frame_size  // any smaller frame too
                                  ? K * spp >= GPS_BIN_AUTO_SAMPLES ||
-                                       (K * spp >= GPS_BIN_AUTO_SAMPLES_LARGE && up * spp > GPS_BIN_LARGE_FB)
-                                 : binned_auto(st.width * ss, st.height * ss, spp, K, N, false) &&
+                                       (K * spp >= GPS_BIN_AUTO_SAMPLES_FEW && up * spp >= GPS_BIN_FEW_FB)
+                                 : (binned_auto(st.width * ss, st.height * ss, spp, K, N, false, false) ||
+                                    binned_auto(st.width * ss, st.height * ss, spp, K, N, true, false)) &&
                                        binned_geometry(st.width * ss, st.height * ss, spp, &g);
             if (!can) continue;
             const uint64_t dense = binned_dense_points(st.width * ss, st.height * ss, spp, K, false);
-            const uint64_t always = K * spp >= GPS_BIN_AUTO_SAMPLES ? 2 * GPS_BIN_DENSE_SAMPLES * up / (uint64_t)K : 0;
+            uint64_t always = 2 * GPS_BIN_DENSE_SAMPLES * up / (uint64_t)K;
+            if (K * spp < GPS_BIN_AUTO_SAMPLES) always = std::min<uint64_t>(always, 16 * N + (1 << 20));
             need = std::max<uint64_t>({need, always, std::min<uint64_t>(8 * N, dense * 5 / 4),
                                        std::min<uint64_t>(2 * N, 2 * dense)});
         }
@@ -888,9 +890,12 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     } else {
         p->timing_slot = -1;
     }
-    // the automatic choice also tests the pass's density on the device
+    // the automatic choice also tests the pass's density on the device, and that
+    // the list is not too short from the outset
     const uint32_t dense_points =
-        p->splat_mode == GPS_SPLAT_BINNED ? 0xFFFFFFFFu : binned_dense_points(f.up_w, f.up_h, f.spp, f.Ki, false);
+        p->splat_mode == GPS_SPLAT_BINNED
+            ? 0xFFFFFFFFu
+            : std::min(binned_dense_points(f.up_w, f.up_h, f.spp, f.Ki, false), p->list.cap);
     const bool may_be_dense = 2ull * p->N > dense_points;
     // The first frame with occlusion culling draws all that is in view in its first
     // pass and next to nothing in the second.  Where the first may be too dense to
@@ -903,7 +908,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     // point-parallel form
     const bool binned = f.unbiased && p->list.points && p->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
                         (p->splat_mode == GPS_SPLAT_BINNED ||
-                         (!unculled && binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, false))) &&
+                         (!unculled && binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, f.occl, false))) &&
                         binned_geometry(f.up_w, f.up_h, f.spp, &bg_geom);
     stage_mark(p, 0, 0, 0, st);
     // The clear also resets the per-frame counters (pass results, culled
@@ -993,6 +998,8 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
             ba.job_cap = p->list.job_cap;
             ba.cus = p->cus;
             ba.dense_points = dense_points;
+            ba.sparse_points =
+                p->splat_mode == GPS_SPLAT_BINNED ? 0u : binned_sparse_points(f.up_w, f.up_h, f.spp, f.Ki);
             ba.atomics_count = p->count_atomics ? &p->ctr->atomics : nullptr;
         }
         DistributeArgs da;

@@ -212,19 +212,34 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 // the point count is known).  Fewer samples per point do not pay for the lists,
 // and denser frames reject most samples at the point-parallel splat's
 // pre-read, which the binned form cannot skip.  A framebuffer of more than
-// GPS_BIN_LARGE_FB words (32 MB) misses the caches, so there both limits are
-// wider: 4 samples per point (given a Gaussian per 16 words, for the launches,
-// and at most 4 per word, as the distributor counts per tile of the scene), and
+// GPS_BIN_LARGE_FB words (32 MB) misses the caches, so there the second limit is
 // 6 samples per word for every GPS_BIN_LARGE_FB words, up to GPS_BIN_DENSE_LARGE
 // (above that dense frames are splatted nearest first, GPS_ORD_DENSE_SAMPLES).
-// Whole frames, us, point-parallel / binned, by samples
-// per word:
+// Whole frames, us, point-parallel / binned, by samples per word:
 //   16 samples a point  33M words 18.7: 6132 / 3945, 3.0: 1551 / 824;
 //                       6.6M words 12.4: 640 / 706; 0.9M words 4.4: 150 / 128
-//   4 samples a point   8.3M words 2.4: 415 / 324, 18.7: 2149 / 2142;
-//                       1.6M words 12.4: 325 / 402, 4.8: 180 / 192
-//   occlusion-culled fly-throughs, 4 samples a point, 8.4M words, 4 to 5 samples
-//                       per word: 25M Gaussians 2027 / 1968, 100M 1891 / 1947
+// Points of 4 to 7 samples pay for the lists only where they are many and their
+// atomics expensive: from GPS_BIN_FEW_FB words on, and with at least
+// GPS_BIN_FEW_WORK / words points, tested on the device (fewer: state[3] = 3).  So
+// that few passes pay for that test, the scene has as many Gaussians where
+// occluded ones are culled, a fifth as many where not (there also few enough not
+// to be too dense, for the bounds below), a Gaussian per 16 words, and at most 4
+// per word (the distributor counts per tile of the scene).  Point-parallel over
+// binned time at 4 samples a point, from clustered scenes seen from outside (c),
+// from a third (c3) and a twelfth (c12) of that distance, a uniform cube seen from
+// twice (u2) and once (u) the distance that fills the frame, from inside (ui), and
+// occlusion-culled fly-throughs (f); * below the limit:
+//   words, Gaussians  c      c3     c12    u2     u     ui    f
+//   4.4M       1M     .78*   .92*   .76*   .84*   1.18* .96*  .84*
+//              4M     .88*   1.01*  .97*   .88*   1.30* 1.13* .94*
+//   6.5M       1M     .84*   .92*   .74*   .90*   1.36* 1.08  .86*
+//              4M     .98    1.07   1.08   .91    1.29  1.14  1.02*
+//   8.3M       1M     .88*   .88*   .72*   .97*   1.43  1.16  .88*
+//              2M     .99*   .95    .85*   .99    1.43  1.16  .99*
+//              4M     1.01   1.14   1.10   .95    1.35  1.17  1.06
+//   14.7M      1M     1.03*  1.02   .81*   1.08   1.68  1.17  .95*
+//              2M     1.13   1.02   .94    1.15   1.58  1.20  1.05
+//   33M        1M     1.15   1.23   .95    1.32   1.70  1.09  1.03
 // A batch shares the lists' launches among its views and has no ordered form:
 // views of more than GPS_BIN_LARGE_FB_BATCH words take the wide limits (batch of
 // 16 views from 1.2M to 33M words, 4 to 13 samples per word: all point-parallel
@@ -233,7 +248,9 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 #define GPS_BIN_DENSE_SAMPLES 8u
 #define GPS_BIN_LARGE_FB (1ull << 22)
 #define GPS_BIN_LARGE_FB_BATCH (1ull << 20)
-#define GPS_BIN_AUTO_SAMPLES_LARGE 4
+#define GPS_BIN_AUTO_SAMPLES_FEW 4
+#define GPS_BIN_FEW_FB (6ull << 20)
+#define GPS_BIN_FEW_WORK 30000000000000ull  // points * words
 #define GPS_BIN_DENSE_LARGE 32u
 // The preprocess writes the records' bounds once more, 8 bytes each, for the
 // binned lists (which otherwise fetch a 64-byte record line for them: 168

@@ -126,6 +126,7 @@ struct BinnedArgs {
     uint32_t list_cap, job_cap;
     uint32_t cus;
     uint32_t dense_points;  // more points than this: the binned kernels stand down (state[3] = 2)
+    uint32_t sparse_points; // fewer: likewise (state[3] = 3)
     uint32_t* atomics_count;
 };
 bool binned_geometry(int up_w, int up_h, int spp, BinGeom* g);
@@ -133,8 +134,9 @@ bool binned_geometry(int up_w, int up_h, int spp, BinGeom* g);
 // above which such a frame is too dense to bin, tested on the device
 // (GPS_BIN_AUTO_SAMPLES, GPS_BIN_DENSE_SAMPLES; a point writes K * spp samples
 // into up_w * up_h * spp words).
-bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool batch);
+bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool occl, bool batch);
 uint32_t binned_dense_points(int up_w, int up_h, int spp, int K, bool batch);
+uint32_t binned_sparse_points(int up_w, int up_h, int spp, int K);  // too few (single frames)
 void launch_binned_splat(const BinnedArgs& a, hipStream_t st);
 
 // Binned splat buffers of a batch: entries are the batch's compacted entries,

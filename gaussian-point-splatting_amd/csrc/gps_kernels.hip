@@ -1083,7 +1083,7 @@ static_assert((uint64_t)GPS_LIST_THREADS * 8 * GPS_BIN_MAX_POINTS < 1ull << 32, 
 // valid Gaussians).  state[0]: (entry, region) pairs.
 struct BinCount {
     BinFrame f;                   // single frame: g, bounds, recs
-    uint32_t dense_points;        // single frame
+    uint32_t dense_points, sparse_points;  // single frame
     const BatchView* views;       // batch: the views' own geometry and limits
     unsigned long long* reg_pts;  // points per region
     BigList big;
@@ -1219,7 +1219,7 @@ __global__ __launch_bounds__(256) void distribute_kernel(const uint32_t* __restr
             bin = bv.bg.nregions != 0u && bv.points <= bv.dense_points;
         } else {
             bc.f.p_end = (uint32_t)P;
-            bin = P <= bc.dense_points;  // else too dense to bin: bin_scan_kernel stands the binned kernels down
+            bin = P <= bc.dense_points && P >= bc.sparse_points;  // else bin_scan_kernel stands the binned kernels down
         }
         if (bin)
             for (uint32_t i = (uint32_t)tid; i < bc.f.g.nregions; i += 256u) s_pts[i] = 0u;
@@ -1906,9 +1906,9 @@ __global__ __launch_bounds__(GPS_SPLAT_THREADS) void splat_ordered_kernel(
 // GPS_BIN_MAX_REGIONS regions are splatted afterwards with global atomics (no
 // replay).  Since min is order-independent the framebuffer is bit-identical
 // to the point-parallel splat.  If the list overflows its allocation
-// (state[3] = 1), or the pass has more points than dense_points (state[3] = 2,
-// the automatic choice's density test), the binned kernels stand down and the
-// point-parallel splat runs instead.
+// (state[3] = 1), or the pass has more points than dense_points (state[3] = 2)
+// or fewer than sparse_points (state[3] = 3; the automatic choice's tests), the
+// binned kernels stand down and the point-parallel splat runs instead.
 
 // One workgroup: the regions' list offsets, and the job table: jobs of at most
 // state[2] points, the largest first (eight size classes), so that the
@@ -1926,7 +1926,8 @@ __global__ __launch_bounds__(1024) void bin_scan_kernel(uint32_t nregions, unsig
                                                         uint32_t* __restrict__ job_reg, uint32_t* __restrict__ job_p0,
                                                         uint32_t* __restrict__ state, uint32_t list_cap,
                                                         uint32_t cus, uint32_t job_cap,
-                                                        const PassCounters* __restrict__ ctr, uint32_t dense_points) {
+                                                        const PassCounters* __restrict__ ctr, uint32_t dense_points,
+                                                        uint32_t sparse_points) {
     constexpr uint32_t CLASSES = 8;
     __shared__ unsigned long long s_w[16], s_carry;  // 64-bit: an overflowing list must not wrap
     __shared__ uint32_t s_cls[CLASSES];
@@ -1981,10 +1982,10 @@ __global__ __launch_bounds__(1024) void bin_scan_kernel(uint32_t nregions, unsig
             run += n;
         }
         s_jobs = run;
-        const bool dense = ctr && ctr->points > dense_points;
+        const bool dense = ctr && ctr->points > dense_points, sparse = ctr && ctr->points < sparse_points;
         state[1] = min(run, job_cap);
         state[2] = job_points;
-        state[3] = dense ? 2u : (s_carry > list_cap || run > job_cap) ? 1u : 0u;
+        state[3] = dense ? 2u : sparse ? 3u : (s_carry > list_cap || run > job_cap) ? 1u : 0u;
         state[4] = 0u;
     }
     __syncthreads();
@@ -3168,6 +3169,7 @@ void launch_distribute(const DistributeArgs& a, hipStream_t st) {
         bc.f.bounds = a.bin->bounds;
         bc.f.recs = a.bin->recs;
         bc.dense_points = a.bin->dense_points;
+        bc.sparse_points = a.bin->sparse_points;
         bc.reg_pts = a.bin->reg_pts;
         bc.big = a.bin->big;
         bc.state = a.bin->state;
@@ -3431,7 +3433,7 @@ void launch_batch_binned(const BatchArgs& a, hipStream_t st) {
     const BinFrame f{a.cidx, a.coff, b.bounds, a.recs, BinGeom{}, 0u, 0u, 0u, 0u};
     hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, st, b.nregions, b.reg_pts, b.reg_ptot, b.reg_poff,
                        b.reg_cursor, b.job_reg, b.job_p0, b.state, b.list_cap, b.cus, b.job_cap,
-                       (const PassCounters*)nullptr, 0xFFFFFFFFu);
+                       (const PassCounters*)nullptr, 0xFFFFFFFFu, 0u);
     hipLaunchKernelGGL(batch_bin_scatter_kernel, dim3(gx, a.nviews), dim3(GPS_LIST_THREADS), hist, st, f,
                        (const BatchView*)a.views, b.reg_cursor, b.list, (const uint32_t*)b.state,
                        (const uint32_t*)b.reg_ptot, reinterpret_cast<unsigned long long*>(a.fb));
@@ -3456,7 +3458,7 @@ void launch_binned_splat(const BinnedArgs& a, hipStream_t st) {
     const BinFrame f{a.cidx, a.coff, a.bounds, a.recs, a.g, 0u, 0u, 0u, 0u};
     hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(1024), 0, st, a.g.nregions, a.reg_pts, a.reg_ptot, a.reg_poff,
                        a.reg_cursor, a.job_reg, a.job_p0, a.state, a.list_cap, a.cus, a.job_cap, a.ctr,
-                       a.dense_points);
+                       a.dense_points, a.sparse_points);
     hipLaunchKernelGGL(bin_scatter_kernel, dim3(a.cus * GPS_LIST_WGS_PER_CU), dim3(GPS_LIST_THREADS), hist, st, f,
                        a.ctr, a.reg_cursor, a.list, (const uint32_t*)a.state, (const uint32_t*)a.reg_ptot,
                        reinterpret_cast<unsigned long long*>(a.fb), a.clear_words, a.background);
@@ -3483,11 +3485,20 @@ uint32_t binned_dense_points(int up_w, int up_h, int spp, int K, bool batch) {
     return p < 0xFFFFFFFFull ? (uint32_t)p : 0xFFFFFFFFu;
 }
 
-bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool batch) {
+uint32_t binned_sparse_points(int up_w, int up_h, int spp, int K) {
     const uint64_t words = (uint64_t)up_w * (uint64_t)up_h * (uint64_t)spp;
-    return K * spp >= GPS_BIN_AUTO_SAMPLES ||
-           (K * spp >= GPS_BIN_AUTO_SAMPLES_LARGE && words > (batch ? GPS_BIN_LARGE_FB_BATCH : GPS_BIN_LARGE_FB) &&
-            16ull * N >= words && (batch || N <= 4ull * words));
+    return K * spp >= GPS_BIN_AUTO_SAMPLES ? 0u : (uint32_t)std::min<uint64_t>(GPS_BIN_FEW_WORK / words, 0xFFFFFFFFull);
+}
+
+bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool occl, bool batch) {
+    const uint64_t words = (uint64_t)up_w * (uint64_t)up_h * (uint64_t)spp;
+    if (K * spp >= GPS_BIN_AUTO_SAMPLES) return true;
+    if (K * spp < GPS_BIN_AUTO_SAMPLES_FEW || 16ull * N < words) return false;
+    if (batch) return words > GPS_BIN_LARGE_FB_BATCH;
+    return words >= GPS_BIN_FEW_FB && N <= 4ull * words &&
+           (occl ? N >= binned_sparse_points(up_w, up_h, spp, K)
+                 : 5ull * N >= binned_sparse_points(up_w, up_h, spp, K) &&
+                       2ull * N <= binned_dense_points(up_w, up_h, spp, K, false));
 }
 
 bool binned_geometry(int up_w, int up_h, int spp, BinGeom* g) {

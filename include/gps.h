@@ -140,7 +140,7 @@ typedef struct gps_stats {
     uint64_t num_blocks;           /* culling blocks (0 when block culling is off) */
     int32_t splat_binned;          /* 1: the last pass used the binned splat */
     int32_t splat_fallback;        /* the point-parallel splat ran instead: 1 region lists overflowed,
-                                      2 too many samples per framebuffer word (GPS_SPLAT_AUTO) */
+                                      2 too many samples per framebuffer word, 3 too few points (GPS_SPLAT_AUTO) */
     uint32_t bin_entries;          /* (Gaussian, region) pairs of the last pass */
     uint32_t bin_jobs;             /* region jobs of the last pass */
     uint32_t bin_big;              /* Gaussians splatted with global atomics (too many regions or points) */
@@ -209,13 +209,13 @@ void gps_pass_destroy(gps_pass* pass);
  * spp) and the pass has at most 8 samples per framebuffer word (points * K <=
  * 8 * upscaled width * height, tested on the device after the point count;
  * denser passes splat point-parallel and report gps_stats.splat_fallback = 2).
- * Framebuffers of more than 2^22 words (upscaled width * height * spp; 2^20 in
- * a batch) take wider limits: 4 samples per point if the scene has a Gaussian
- * per 16 words and, in a single pass, at most 4 per word, and 6 samples per
- * word for every 2^22 words, up to 32 (32 in a batch).  A pass's first frame
- * with occlusion culling, which nothing culls, takes the 4-sample limit only
- * in scenes too small to be too dense (twice as many points as Gaussians).
- * All give the same framebuffer bit for bit.  No reference counterpart
+ * Framebuffers of more than 2^22 words (upscaled width * height * spp) take 6
+ * samples per word for every 2^22 words, up to 32.  From 6 * 2^20 words on
+ * points of 4 to 7 samples are binned too, when the scene has a Gaussian per 16
+ * words and at most 4 per word, and a pass at least 3e13 / words points (fewer:
+ * splat_fallback = 3); scenes that rarely reach or that exceed this are not
+ * tried.  In a batch views of more than 2^20 words take 32 samples per word, and
+ * points of 4 samples with a Gaussian per 16 words.  All give the same framebuffer bit for bit.  No reference counterpart
  * (the reference has only the point-parallel form,
  * gaussian_point_splatting.cu:383-432). */
 #define GPS_SPLAT_AUTO 0
@@ -268,7 +268,7 @@ gps_status gps_pass_set_ordered_splat(gps_pass* pass, int32_t mode);
  * gps_pass_create allocates for these settings.  Where GPS_SPLAT_AUTO can bin
  * frames of the settings both count the binned buffers: 16 B per Gaussian and
  * 8 B per listed point: room for 16 points per output pixel where a point has
- * at least 8 samples, in large framebuffers for 8 points per Gaussian or up to
+ * at least 8 samples, in large framebuffers for 8 to 16 points per Gaussian or up to
  * 40 per pixel, and for at most twice the point budget.  A pass that
  * cannot have this part is created without it and splats point-parallel.  A
  * frame of another supersampling factor than the pass's last reallocates

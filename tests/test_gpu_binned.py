@@ -94,21 +94,52 @@ def test_binned_batch_list_steps(gpu, n):
         assert_same(f"view {i} depth", x[1], y[1])
 
 
+def _auto_frames(gpu, arrays, w, h, spp, eyes, ss=2, **kw):
+    """The automatic choice's statistics per frame, its images checked against
+    the point-parallel splat's."""
+    st = gpu.RenderSettings(w, h, spp, ss, fully_disable_hierarchical_culling=True)
+    a, b = H.GpuRunner(arrays, st), H.GpuRunner(arrays, st)
+    b.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
+    out = []
+    for k, eye in enumerate(eyes):
+        flush(f"automatic {w}x{h} n {arrays.n} frame {k}")
+        f = gpu.frame_params(eye, (0, 0, 0), (0, 1, 0), 45.0, w, h, ss=ss, frame=3 + k, spp=spp,
+                             background=(0.2, 0.4, 0.6), **kw)
+        x, y = (r.render(f, [gpu.DBG_FRAMEBUFFER]) for r in (a, b))
+        _same(gpu, x, y, f"{w}x{h} n {arrays.n} frame {k}")
+        out.append((x.stats["splat_binned"], x.stats["splat_fallback"]))
+    return out
+
+
 def test_binned_auto_large_framebuffer(gpu):
-    """More than 2^22 framebuffer words: 4 samples a point are binned too, and
-    passes of up to 6 samples per word and 2^22 words."""
-    arrays = H.scene(0x5EED0821, 400_000, dict(H.C1, half_extent=8.0)).morton_sorted()
-    a, b = _frames(gpu, arrays, 1400, 780, 2, 1, (0.0, 3.0, -25.0), (gpu.Pass.SPLAT_AUTO, gpu.Pass.SPLAT_POINT_PARALLEL))
-    assert a.stats["splat_binned"] == 1 and a.stats["splat_fallback"] == 0, a.stats
-    _same(gpu, a, b, "large framebuffer")
+    """Points of 4 samples from 6 * 2^20 framebuffer words on: binned with at
+    least 3e13 / words points (4.6M here), else stood down on the device, frame
+    by frame; not tried in smaller framebuffers or scenes, nor where occluded
+    Gaussians are culled from a scene of fewer Gaussians than that."""
+    cfg = dict(H.C1, half_extent=8.0)
+    arrays = H.scene(0x5EED0821, 950_000, cfg).morton_sorted()
+    near, far = (0.0, 3.0, -25.0), (0.0, 3.0, -60.0)
+    assert _auto_frames(gpu, arrays, 1700, 956, 1, [near, far, near]) == [(1, 0), (1, 3), (1, 0)]
+    assert _auto_frames(gpu, arrays, 1400, 780, 1, [near]) == [(0, 0)]
+    assert _auto_frames(gpu, arrays, 1700, 956, 1, [near, near], occlusion=True) == [(0, 0)] * 2
+    assert _auto_frames(gpu, H.scene(0x5EED0821, 400_000, cfg), 1700, 956, 1, [near]) == [(0, 0)]
+
+
+def test_binned_auto_dense_large_framebuffer(gpu):
+    """Points of 9 samples: up to 8 samples per word, in framebuffers of more
+    than 2^22 words up to 6 for every 2^22 words (20 here)."""
+    arrays = H.scene(0x5EED0861, 2_700_000, dict(H.C1, half_extent=5.0, log_scale_mu=-4.2)).morton_sorted()
+    far, mid, near = ((0.0, 3.0, d) for d in (-40.0, -19.0, -9.5))
+    assert _auto_frames(gpu, arrays, 640, 360, 1, [far], ss=3) == [(1, 2)]  # 15 samples per word
+    assert _auto_frames(gpu, arrays, 1700, 956, 1, [mid, near], ss=3) == [(1, 0), (1, 2)]  # 9.8 and 27
 
 
 def test_first_culled_frame_is_point_parallel(gpu):
     """4 samples a point in a scene that may be too dense to bin: the first
     frame with occlusion culling, which nothing culls, takes no lists; later
     ones do.  The same images as point-parallel throughout."""
-    arrays = H.scene(0x5EED0831, 4_500_000, dict(H.C1, half_extent=30.0, log_scale_mu=-4.0)).morton_sorted()
-    w, h = 1400, 780
+    arrays = H.scene(0x5EED0831, 7_400_000, dict(H.C1, half_extent=30.0, log_scale_mu=-4.0))
+    w, h = 1700, 956
     st = gpu.RenderSettings(w, h, 1, 2, gaussians_per_block=256)
     a, b = H.GpuRunner(arrays, st), H.GpuRunner(arrays, st)
     b.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
