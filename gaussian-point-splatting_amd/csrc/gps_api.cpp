@@ -223,8 +223,8 @@ uint64_t bin_list_points(const gps_render_settings& st, int ss, uint64_t N) {
             const bool can = st.flexible_frame_size  // any smaller frame too
                                  ? K * spp >= GPS_BIN_AUTO_SAMPLES ||
                                        (K * spp >= GPS_BIN_AUTO_SAMPLES_FEW && up * spp >= GPS_BIN_FEW_FB)
-                                 : (binned_auto(st.width * ss, st.height * ss, spp, K, N, false, false) ||
-                                    binned_auto(st.width * ss, st.height * ss, spp, K, N, true, false)) &&
+                                 : (binned_auto(st.width * ss, st.height * ss, spp, K, N, false, 0) ||
+                                    binned_auto(st.width * ss, st.height * ss, spp, K, N, true, 0)) &&
                                        binned_geometry(st.width * ss, st.height * ss, spp, &g);
             if (!can) continue;
             const uint64_t dense = binned_dense_points(st.width * ss, st.height * ss, spp, K, false);
@@ -908,7 +908,7 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     // point-parallel form
     const bool binned = f.unbiased && p->list.points && p->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
                         (p->splat_mode == GPS_SPLAT_BINNED ||
-                         (!unculled && binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, f.occl, false))) &&
+                         (!unculled && binned_auto(f.up_w, f.up_h, f.spp, f.Ki, p->N, f.occl, 0))) &&
                         binned_geometry(f.up_w, f.up_h, f.spp, &bg_geom);
     stage_mark(p, 0, 0, 0, st);
     // The clear also resets the per-frame counters (pass results, culled

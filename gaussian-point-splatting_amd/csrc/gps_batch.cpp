@@ -388,7 +388,7 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
         // (unbiased frames only: the biased splat adds colours per sample).
         BinGeom g;
         if (bv.f.unbiased && b->splat_mode != GPS_SPLAT_POINT_PARALLEL &&
-            (b->splat_mode == GPS_SPLAT_BINNED || binned_auto(bv.f.up_w, bv.f.up_h, bv.f.spp, bv.f.Ki, b->N, false, true)) &&
+            (b->splat_mode == GPS_SPLAT_BINNED || binned_auto(bv.f.up_w, bv.f.up_h, bv.f.spp, bv.f.Ki, b->N, false, nviews)) &&
             binned_geometry(bv.f.up_w, bv.f.up_h, bv.f.spp, &g) && ensure_binned(b, may_alloc) &&
             regions + g.nregions <= b->bin_regions_cap) {
             bv.bg = g;

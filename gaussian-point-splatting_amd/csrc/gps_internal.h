@@ -243,7 +243,13 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 // A batch shares the lists' launches among its views and has no ordered form:
 // views of more than GPS_BIN_LARGE_FB_BATCH words take the wide limits (batch of
 // 16 views from 1.2M to 33M words, 4 to 13 samples per word: all point-parallel
-// 25.2 ms, views of up to 8 samples per word binned 14.7, all binned 8.7).
+// 25.2 ms, views of up to 8 samples per word binned 14.7, all binned 8.7).  Points
+// of 4 to 7 samples: from GPS_BIN_FEW_WORK_BATCH / (words * views) Gaussians on
+// (point-parallel over binned time of 3 / 12 views, clustered scenes from two
+// distances, then uniform; * below the limit: 1.2M words 200,000 Gaussians .86*
+// .89* 1.06* / .95* .97* 1.28*, 500,000 .88* .90* 1.17* / .99 1.03 1.57, 1M .92 .97
+// 1.32 / 1.03 1.12 1.63; 3.7M words 500,000 .94 1.02 1.40 / 1.04 1.15 1.76, 1M
+// 1.00 1.11 1.60 / 1.08 1.25 1.85).
 #define GPS_BIN_AUTO_SAMPLES 8
 #define GPS_BIN_DENSE_SAMPLES 8u
 #define GPS_BIN_LARGE_FB (1ull << 22)
@@ -251,6 +257,7 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 #define GPS_BIN_AUTO_SAMPLES_FEW 4
 #define GPS_BIN_FEW_FB (6ull << 20)
 #define GPS_BIN_FEW_WORK 30000000000000ull  // points * words
+#define GPS_BIN_FEW_WORK_BATCH 3000000000000ull  // Gaussians * words * views
 #define GPS_BIN_DENSE_LARGE 32u
 // The preprocess writes the records' bounds once more, 8 bytes each, for the
 // binned lists (which otherwise fetch a 64-byte record line for them: 168

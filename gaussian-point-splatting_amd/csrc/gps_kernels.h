@@ -131,10 +131,11 @@ struct BinnedArgs {
 };
 bool binned_geometry(int up_w, int up_h, int spp, BinGeom* g);
 // Whether the automatic choice may bin a frame of N Gaussians, and the points
-// above which such a frame is too dense to bin, tested on the device
+// above which such a frame is too dense to bin, tested on the device; `views`: of a
+// batch, 0 for a single frame
 // (GPS_BIN_AUTO_SAMPLES, GPS_BIN_DENSE_SAMPLES; a point writes K * spp samples
 // into up_w * up_h * spp words).
-bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool occl, bool batch);
+bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool occl, int views);
 uint32_t binned_dense_points(int up_w, int up_h, int spp, int K, bool batch);
 uint32_t binned_sparse_points(int up_w, int up_h, int spp, int K);  // too few (single frames)
 void launch_binned_splat(const BinnedArgs& a, hipStream_t st);

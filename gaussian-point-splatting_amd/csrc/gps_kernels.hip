@@ -3490,11 +3490,11 @@ uint32_t binned_sparse_points(int up_w, int up_h, int spp, int K) {
     return K * spp >= GPS_BIN_AUTO_SAMPLES ? 0u : (uint32_t)std::min<uint64_t>(GPS_BIN_FEW_WORK / words, 0xFFFFFFFFull);
 }
 
-bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool occl, bool batch) {
+bool binned_auto(int up_w, int up_h, int spp, int K, uint64_t N, bool occl, int views) {
     const uint64_t words = (uint64_t)up_w * (uint64_t)up_h * (uint64_t)spp;
     if (K * spp >= GPS_BIN_AUTO_SAMPLES) return true;
     if (K * spp < GPS_BIN_AUTO_SAMPLES_FEW || 16ull * N < words) return false;
-    if (batch) return words > GPS_BIN_LARGE_FB_BATCH;
+    if (views > 0) return words > GPS_BIN_LARGE_FB_BATCH && N * words * (uint64_t)views >= GPS_BIN_FEW_WORK_BATCH;
     return words >= GPS_BIN_FEW_FB && N <= 4ull * words &&
            (occl ? N >= binned_sparse_points(up_w, up_h, spp, K)
                  : 5ull * N >= binned_sparse_points(up_w, up_h, spp, K) &&

@@ -215,7 +215,8 @@ void gps_pass_destroy(gps_pass* pass);
  * words and at most 4 per word, and a pass at least 3e13 / words points (fewer:
  * splat_fallback = 3); scenes that rarely reach or that exceed this are not
  * tried.  In a batch views of more than 2^20 words take 32 samples per word, and
- * points of 4 samples with a Gaussian per 16 words.  All give the same framebuffer bit for bit.  No reference counterpart
+ * points of 4 to 7 samples where Gaussians * words * views is at least 3e12 and
+ * there is a Gaussian per 16 words.  All give the same framebuffer bit for bit.  No reference counterpart
  * (the reference has only the point-parallel form,
  * gaussian_point_splatting.cu:383-432). */
 #define GPS_SPLAT_AUTO 0

@@ -125,6 +125,34 @@ def test_binned_auto_large_framebuffer(gpu):
     assert _auto_frames(gpu, H.scene(0x5EED0821, 400_000, cfg), 1700, 956, 1, [near]) == [(0, 0)]
 
 
+@pytest.mark.parametrize("n,size,views,binned", [(900_000, (1280, 720), 1, 1), (400_000, (1280, 720), 1, 0),
+                                                 (400_000, (1280, 720), 3, 1), (200_000, (1280, 720), 9, 0),
+                                                 (900_000, (480, 270), 9, 0)])
+def test_binned_auto_batch(gpu, n, size, views, binned):
+    """Views of points of 4 samples: more than 2^20 words, a Gaussian per 16 of
+    them, Gaussians * words * views >= 3e12."""
+    w, h = size
+    arrays = H.scene(0x5EED0871, n, dict(H.C1, half_extent=8.0, log_scale_mu=-4.5))
+    scene, stream = gpu.Scene(arrays), gpu.Stream()
+    f = [gpu.frame_params((0.0, 3.0, -25.0 - i), (0, 0, 0), (0, 1, 0), 45.0, w, h, ss=2, frame=3, spp=1)
+         for i in range(views)]
+    out = [(gpu.DeviceArray((h, w, 3), np.float32, zero=True), gpu.DeviceArray((h, w), np.float32, zero=True)) for _ in f]
+    flush(f"automatic batch {size} n {n} views {views}")
+    got = []
+    for mode in (gpu.Pass.SPLAT_AUTO, gpu.Pass.SPLAT_POINT_PARALLEL):
+        b = gpu.Batch(scene, views, w, h, 1, 2)
+        b.set_splat_mode(mode)
+        b.render(f, [c for c, _ in out], [d for _, d in out], stream)
+        for i in range(views):
+            stats = b.view_stats(i, stream)
+            assert stats["splat_fallback"] == 0 and stats["splat_binned"] == (binned if mode == 0 else 0), (i, stats)
+        got.append([(c.download(), d.download()) for c, d in out])
+        b.close()
+    for i, (x, y) in enumerate(zip(*got)):
+        assert_same(f"view {i} colour", x[0], y[0])
+        assert_same(f"view {i} depth", x[1], y[1])
+
+
 def test_binned_auto_dense_large_framebuffer(gpu):
     """Points of 9 samples: up to 8 samples per word, in framebuffers of more
     than 2^22 words up to 6 for every 2^22 words (20 here)."""
