@@ -306,6 +306,7 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 #ifndef GPS_FOLD_TILES
 #define GPS_FOLD_TILES 1024u
 #endif
+static_assert(GPS_FOLD_TILES % 256 == 0, "the distribute workgroups' 256 threads take the same number of tiles each");
 inline bool fold_tiles(uint32_t ntiles) { return ntiles != 0u && ntiles <= GPS_FOLD_TILES; }
 #ifndef GPS_PRE_THREADS
 #define GPS_PRE_THREADS 256
