@@ -77,9 +77,10 @@ GPS_HD float det_sqrt_normal(float x) {
 // reciprocal root with one residual correction, g = x * y and
 // g + (x - g * g) * (y / 2), is the IEEE-rounded root there.  6 instructions
 // (24 cycles of a SIMD per wave) against det_sqrt_normal's 11 (48): a compare
-// with its select costs as much as four multiplications on gfx950.  Compared
-// with det_sqrt on the GPU for every float in [1, 4) (scaling by 4 commutes)
-// and for every value the sampling radius takes.  The host takes det_sqrt.
+// with its select costs as much as four multiplications on gfx950.  The GPU
+// test test_radius_root compares it with the IEEE root for every float in [1, 4)
+// (scaling by 4 commutes), a sample of 2^-100 .. 2^64 and every fifth float from
+// 2^-24 to 171, the radius' range.  The host takes det_sqrt.
 GPS_HD float det_sqrt_radius(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
     // x = 0: the infinite reciprocal root is cut off, so that g = 0

@@ -31,6 +31,35 @@ __global__ void selftest_math_kernel(int kind, const float* __restrict__ in, flo
     out[i] = r;
 }
 
+// The splat's sampling transform as the device compiles it (hardware root,
+// conversion and clamps), on words: floats are bit patterns.
+__global__ void selftest_sampling_kernel(int kind, const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                         uint64_t n) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    float a = 0.0f, b = 0.0f;
+    uint32_t r = 0u;
+    switch (kind) {
+        case 0: r = f2u_bits(det_sqrt_radius(u2f_bits(in[i]))); break;
+        case 1: r = (uint32_t)det_f2i_sat(u2f_bits(in[i])); break;
+        case 2: r = f2u_bits(det_neg2_logf_normal(u2f_bits(in[i]))); break;
+        case 3:
+        case 4:
+            det_sincosf_u32((float)in[i], &a, &b);
+            r = f2u_bits(kind == 3 ? a : b);
+            break;
+        case 5:
+        case 6: {
+            const float alpha = u2f_bits(in[3 * i + 2]);
+            const f32x2 xy = corrected_box_muller_v((float)in[3 * i], (float)in[3 * i + 1], corrected_inv_alpha(alpha),
+                                                    dilog(alpha));
+            r = f2u_bits(kind == 5 ? xy.x : xy.y);
+            break;
+        }
+    }
+    out[i] = r;
+}
+
 __global__ void selftest_rng_kernel(uint32_t n, uint32_t frame, int draws, uint32_t* __restrict__ out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -97,6 +126,15 @@ extern "C" gps_status gps_selftest_math(int32_t kind, const float* d_in, float* 
     if (!d_in || !d_out || kind < 0 || kind > 13) return GPS_ERR_INVALID_ARG;
     if (n == 0) return GPS_OK;
     hipLaunchKernelGGL(gps::selftest_math_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, kind, d_in, d_out, n);
+    return hipGetLastError() == hipSuccess ? GPS_OK : GPS_ERR_HIP;
+}
+
+extern "C" gps_status gps_selftest_sampling(int32_t kind, const uint32_t* d_in, uint32_t* d_out, uint64_t n,
+                                            void* stream) {
+    if (!d_in || !d_out || kind < 0 || kind > 6) return GPS_ERR_INVALID_ARG;
+    if (n == 0) return GPS_OK;
+    hipLaunchKernelGGL(gps::selftest_sampling_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, kind, d_in, d_out, n);
     return hipGetLastError() == hipSuccess ? GPS_OK : GPS_ERR_HIP;
 }

@@ -202,6 +202,7 @@ _sig("gps_pass_set_ordered_splat", C.c_int32, _vp, C.c_int32)
 _sig("gps_pass_timing_summary", C.c_int32, _vp, C.POINTER(C.c_double), C.POINTER(C.c_uint64),
      C.POINTER(C.c_uint64))
 _sig("gps_selftest_math", C.c_int32, C.c_int32, _vp, _vp, C.c_uint64, _vp)
+_sig("gps_selftest_sampling", C.c_int32, C.c_int32, _vp, _vp, C.c_uint64, _vp)
 _sig("gps_selftest_rng", C.c_int32, C.c_uint32, C.c_uint32, C.c_int32, _vp, _vp)
 _sig("gps_selftest_poisson", C.c_int32, C.c_uint32, _vp, _vp, _vp)
 _sig("gps_selftest_copy", C.c_int32, _vp, _vp, C.c_uint64, _vp)

@@ -665,8 +665,14 @@ void gps_server_destroy(gps_server* server);
  * 7 inv_dilog, 8 float->int round-to-nearest-even (saturating),
  * 9 Box-Muller x of (in[i], in[i+1]), 10 corrected Box-Muller y (alpha 0.7),
  * 11 FP8 E4M3 decode of code in[i], 12 the log's quotient x / (2 + x),
- * 13 the square root of the sampling transform (x = 0 or normal). */
+ * 13 the square root of the screen bounds (x = 0 or normal). */
 gps_status gps_selftest_math(int32_t kind, const float* d_in, float* d_out, uint64_t n, void* stream);
+/* The splat's sampling transform on the device, words in and out (floats as
+ * bit patterns).  kind: 0 the radius' square root, 1 float->int truncating and
+ * saturating, 2 -2 log x (x normal), 3 sine and 4 cosine of 2 pi in[i] / 2^32,
+ * 5 x and 6 y of the corrected Box-Muller transform of random words in[3i] and
+ * in[3i + 1] for opacity in[3i + 2]. */
+gps_status gps_selftest_sampling(int32_t kind, const uint32_t* d_in, uint32_t* d_out, uint64_t n, void* stream);
 /* Per item i: make_seed(i, frame) then `draws` pcg2d states (2+2*draws u32). */
 gps_status gps_selftest_rng(uint32_t n, uint32_t frame, int32_t draws, uint32_t* d_out, void* stream);
 /* Per item i: poisson(make_seed(i, 12345), lambda[i]). */

@@ -57,8 +57,8 @@ def test_device_log_quotient_exhaustive(gpu):
 
 
 def test_device_sqrt_range_exhaustive(gpu):
-    """The sampling transform's square root (hardware root and the +-1-ulp
-    fma correction, no tiny-input scaling) equals det_sqrt's IEEE-rounded
+    """The screen bounds' square root (hardware root and the +-1-ulp fma
+    correction, no tiny-input scaling) equals det_sqrt's IEEE-rounded
     root for every float in [1, 4) -- every mantissa at both exponent
     parities -- and for 0, a sample of floats from 2^-96 to 2^128, the 4096
     largest floats, infinity, and NaN for negative and NaN inputs."""
