@@ -94,6 +94,56 @@ def test_binned_batch_list_steps(gpu, n):
         assert_same(f"view {i} depth", x[1], y[1])
 
 
+@pytest.mark.parametrize("spp", [1, 4])
+def test_binned_list_overflow(gpu, spp):
+    """More listed points than a forced list holds (twice the budget): every
+    Gaussian lies on the corner of four regions, so each point is listed four
+    times.  The frame is splatted point-parallel from a cleared framebuffer,
+    and the next frame on the same pass is binned."""
+    arrays = H.scene(0x5EED0881, 4000, dict(H.C1, half_extent=0.05, log_scale_mu=-1.6, log_scale_sigma=0.1))
+    w = 256 if spp == 1 else 128
+    st = gpu.RenderSettings(w, w, spp, 1, max_number_of_points=1 << 20, fully_disable_hierarchical_culling=True)
+    a, b = H.GpuRunner(arrays, st), H.GpuRunner(arrays, st)
+    a.p.set_splat_mode(gpu.Pass.SPLAT_BINNED)
+    b.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
+    fallbacks = []
+    for k, z in enumerate((-4.0, -60.0, -4.0, -60.0)):
+        flush(f"list overflow spp {spp} frame {k}")
+        f = gpu.frame_params((0.0, 0.0, z), (0, 0, 0), (0, 1, 0), 45.0, w, w, ss=1, frame=1 + k, spp=spp,
+                             background=(0.2, 0.4, 0.6))
+        x, y = (r.render(f, [gpu.DBG_FRAMEBUFFER]) for r in (a, b))
+        _same(gpu, x, y, f"spp {spp} frame {k}")
+        assert x.stats["splat_binned"] == 1
+        fallbacks.append(x.stats["splat_fallback"])
+    assert fallbacks == [1, 0, 1, 0], fallbacks
+
+
+def test_binned_without_bounds(gpu):
+    """A scene of more than half as many Gaussians as points can be binned,
+    most of them out of view: no bounds are written, the lists read them from
+    the records.  Single passes and a batch."""
+    w, h = 320, 180
+    arrays = H.scene(0x5EED0891, 600_000, dict(H.C1, half_extent=60.0, log_scale_mu=-3.0)).morton_sorted()
+    st = gpu.RenderSettings(w, h, 2, 2)
+    f = gpu.frame_params((0.0, 1.0, -5.0), (0, 0, 0), (0, 1, 0), 45.0, w, h, ss=2, frame=3, spp=2, hierarchical=True,
+                         background=(0.2, 0.4, 0.6))
+    a, b = H.GpuRunner(arrays, st), H.GpuRunner(arrays, st)
+    b.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
+    flush("no bounds: single pass")
+    x, y = (r.render(f, [gpu.DBG_FRAMEBUFFER]) for r in (a, b))
+    assert 2 * arrays.n > 8 * w * h >= x.stats["num_points"][0] > 50_000, x.stats
+    assert x.stats["splat_binned"] == 1 and x.stats["splat_fallback"] == 0, x.stats
+    _same(gpu, x, y, "no bounds")
+    flush("no bounds: batch")
+    batch = gpu.Batch(a.scene, 1, w, h, 2, 2)
+    batch.render([f], [a.color], [a.depth], a.stream)
+    stats = batch.view_stats(0, a.stream)
+    assert stats["splat_binned"] == 1 and stats["splat_fallback"] == 0, stats
+    assert_same("batch colour", a.color.download(), y.color)
+    assert_same("batch depth", a.depth.download(), y.depth)
+    batch.close()
+
+
 def _auto_frames(gpu, arrays, w, h, spp, eyes, ss=2, **kw):
     """The automatic choice's statistics per frame, its images checked against
     the point-parallel splat's."""
