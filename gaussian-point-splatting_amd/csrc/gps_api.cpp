@@ -208,31 +208,31 @@ gps_status ensure_fb(gps_pass* p, int ss, uint64_t frame_words) {
 }
 
 // Points that a list needs for the automatic choice in frames of the settings'
-// size at supersampling `ss`, 0 where it bins none of them (a frame's points
-// have ss^2 or 1 samples per layer).  Gaussians that straddle regions are listed
-// in each, 1.15 to 1.3 times in all: room twice for GPS_BIN_DENSE_SAMPLES per
-// framebuffer word (points of few samples: at most for 16 per Gaussian), and
-// 1.25 times for the denser frames that large framebuffers take (at most 8 per
-// Gaussian, but two per Gaussian twice); never more than the point budget twice.
+// size at supersampling `ss`, 0 where it bins none of them.  A frame's points
+// have ss^2 samples per layer; one whose points are not reduced to that has
+// ss^2 times as many, and is stood down where they do not fit.  Gaussians that
+// straddle regions are listed in each, 1.15 to 1.3 times in all: room twice for
+// GPS_BIN_DENSE_SAMPLES per framebuffer word (points of few samples: at most for
+// 16 per Gaussian), and 1.25 times for the denser frames that large framebuffers
+// take (at most 8 per Gaussian, but two per Gaussian twice); never more than the
+// point budget twice.
 uint64_t bin_list_points(const gps_render_settings& st, int ss, uint64_t N) {
-    const uint64_t up = (uint64_t)st.width * ss * (uint64_t)st.height * ss;
+    const int uw = st.width * ss, uh = st.height * ss, K = ss * ss;
+    const uint64_t px = (uint64_t)st.width * (uint64_t)st.height;
     uint64_t need = 0;
-    for (const int K : {ss * ss, 1})
-        for (int spp = st.flexible_frame_size ? 1 : st.render_pass_count; spp <= std::min(st.render_pass_count, 4); ++spp) {
-            BinGeom g;
-            const bool can = st.flexible_frame_size  // any smaller frame too
-                                 ? K * spp >= GPS_BIN_AUTO_SAMPLES ||
-                                       (K * spp >= GPS_BIN_AUTO_SAMPLES_FEW && up * spp >= GPS_BIN_FEW_FB)
-                                 : (binned_auto(st.width * ss, st.height * ss, spp, K, N, false, 0) ||
-                                    binned_auto(st.width * ss, st.height * ss, spp, K, N, true, 0)) &&
-                                       binned_geometry(st.width * ss, st.height * ss, spp, &g);
-            if (!can) continue;
-            const uint64_t dense = binned_dense_points(st.width * ss, st.height * ss, spp, K, false);
-            uint64_t always = 2 * GPS_BIN_DENSE_SAMPLES * up / (uint64_t)K;
-            if (K * spp < GPS_BIN_AUTO_SAMPLES) always = std::min<uint64_t>(always, 16 * N + (1 << 20));
-            need = std::max<uint64_t>({need, always, std::min<uint64_t>(8 * N, dense * 5 / 4),
-                                       std::min<uint64_t>(2 * N, 2 * dense)});
-        }
+    for (int spp = st.flexible_frame_size ? 1 : st.render_pass_count; spp <= std::min(st.render_pass_count, 4); ++spp) {
+        BinGeom g;
+        const bool can = st.flexible_frame_size  // any smaller frame too
+                             ? K * spp >= GPS_BIN_AUTO_SAMPLES ||
+                                   (K * spp >= GPS_BIN_AUTO_SAMPLES_FEW && px * K * spp >= GPS_BIN_FEW_FB)
+                             : (binned_auto(uw, uh, spp, K, N, false, 0) || binned_auto(uw, uh, spp, K, N, true, 0)) &&
+                                   binned_geometry(uw, uh, spp, &g);
+        if (!can) continue;
+        uint64_t room = 2 * GPS_BIN_DENSE_SAMPLES * px;
+        if (K * spp < GPS_BIN_AUTO_SAMPLES) room = std::min<uint64_t>(room, 16 * N + (1 << 20));
+        const uint64_t dense = binned_dense_points(uw, uh, spp, K, false);
+        need = std::max<uint64_t>({need, room, std::min<uint64_t>(8 * N, dense * 5 / 4), std::min<uint64_t>(2 * N, 2 * dense)});
+    }
     const uint64_t budget = (uint64_t)std::max<int64_t>(st.max_number_of_points, 1 << 20);
     return std::min<uint64_t>({need, 2 * budget, 0xFFFFF000ull});
 }
