@@ -2313,11 +2313,11 @@ __global__ __launch_bounds__(GPS_BIN_THREADS) void bin_splat_kernel(
 
 // ------------------------------------------------------------------ binned splat, batches
 // The regions of all binned views of a batch are numbered consecutively
-// (view v owns [rbase(v), rbase(v) + nregions(v))), so the region scan, the
-// list scans and the job queue are the single-frame kernels over the whole
-// batch; counting and scattering take a grid row per view (grid.y = view)
-// with the view's own histogram in LDS, and a job finds its view by its
-// region.  Views whose bg.nregions is 0, or with more points than their
+// (view v owns [rbase(v), rbase(v) + nregions(v))), so the region scan and the
+// job queue are the single-frame kernels over the whole batch; the distributor
+// counts by the view of its tile, the scatter takes a grid row per view (grid.y
+// = view), each with the view's own histogram in LDS, and a job finds its view
+// by its region.  Views whose bg.nregions is 0, or with more points than their
 // dense_points, are left to the point-parallel batch splat (their regions stay
 // empty).
 
