@@ -224,7 +224,12 @@ static_assert((GPS_SPLAT_SLOTS & (GPS_SPLAT_SLOTS - 1)) == 0, "slots: a power of
 // that few passes pay for that test, the scene has as many Gaussians where
 // occluded ones are culled, a fifth as many where not (there also few enough not
 // to be too dense, for the bounds below), a Gaussian per 16 words, and at most 4
-// per word (the distributor counts per tile of the scene).  Point-parallel over
+// per word: the distributor counts for every tile of the scene, and a pass holds
+// 16 bytes per Gaussian more.  Above 4 little is left of the gain (fly-throughs,
+// point-parallel over automatic time without that limit: 3.0 per word 1.04, 4.8
+// 1.03, 6.2 at 6.5M words 1.00, 7.2 1.02, 12 over a 100M path 1.016 and 1.028 in
+// its first frames, 12.3 at 6.5M words, too dense in the second pass, .98; a 100M
+// pass would hold 1.9 GB more).  Point-parallel over
 // binned time at 4 samples a point, from clustered scenes seen from outside (c),
 // from a third (c3) and a twelfth (c12) of that distance, a uniform cube seen from
 // twice (u2) and once (u) the distance that fills the frame, from inside (ui), and
