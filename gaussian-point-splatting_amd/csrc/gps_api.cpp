@@ -710,6 +710,11 @@ uint64_t gps_pass_estimate_bytes(const gps_render_settings* st, const gps_scene*
 
 }  // extern "C"
 
+bool gps::stream_captured(void* stream) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return stream && (hipStreamIsCapturing((hipStream_t)stream, &s) != hipSuccess || s != hipStreamCaptureStatusNone);
+}
+
 uint64_t gps::pass_list_points(const gps_render_settings* st, const gps_scene* scene) {
     return bin_list_points(*st, st->supersampling_factor, scene->view.N);
 }
@@ -870,7 +875,9 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     hipStream_t st = (hipStream_t)stream;
     gps_status s = ensure_fb(p, ss, fb_words(fp->width * ss, fp->height * ss, spp));
     if (s != GPS_OK) return s;
-    ensure_bin_auto(p, ss, true);  // as the framebuffers: only when ss changed
+    // as the framebuffers, only when ss changed; small ones keep their size then,
+    // and a caller that captures the frame gets the list there is
+    if (p->bin_ss != ss && !stream_captured(stream)) ensure_bin_auto(p, ss, true);
 
     FrameConsts f;
     make_frame_consts(fp, spp, &f);

@@ -360,9 +360,7 @@ gps_status gps_batch_render(gps_batch* b, int32_t nviews, const gps_frame_params
     uint64_t list_points = 0;
     // A caller that captures this call gets no allocation: the list there is
     // serves, or the point-parallel splat.
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool may_alloc = !stream || (hipStreamIsCapturing(st, &capture) == hipSuccess &&
-                                       capture == hipStreamCaptureStatusNone);
+    const bool may_alloc = !stream_captured(stream);
     for (int v = 0; v < nviews; ++v) {
         const gps_frame_params& f = views[v];
         const int spp = f.samples_per_pixel > 0 ? f.samples_per_pixel : b->settings.max_spp;

@@ -344,6 +344,9 @@ gps_status pass_create(const gps_render_settings* st, gps_scene* scene, uint64_t
 uint64_t pass_list_points(const gps_render_settings* st, const gps_scene* scene);
 uint64_t pass_bytes(const gps_render_settings* st, const gps_scene* scene, uint64_t max_list);
 
+// Whether the caller captures `stream`: nothing is allocated then.
+bool stream_captured(void* stream);
+
 }  // namespace gps
 
 // Resident scene behind the gps_scene handle.

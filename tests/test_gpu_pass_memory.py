@@ -93,6 +93,45 @@ def test_supersampling_that_can_be_binned_later(gpu, small):
     assert lists[0] == lists[1] < lists[2], (sizes, fb)
 
 
+def _captured(gpu, r, frame):
+    """The frame captured by its caller: graph and executable."""
+    hip, st = gpu.lib, r.stream.handle
+    graph, exe = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(st, 1) == 0  # thread local
+    r.p.render(frame, r.color, r.depth, r.stream)
+    assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+    return graph, exe
+
+
+def test_captured_frame_of_another_supersampling(gpu, small):
+    """Framebuffers this small do not change with the factor: a frame that the
+    caller captures takes no list either, the next eager one does."""
+    w, h = 16, 12
+    st = gpu.RenderSettings(w, h, 1, 1)
+    r, other = H.GpuRunner(small, st), H.GpuRunner(small, st)
+    first, third = (_frame(gpu, w, h, ss, 1) for ss in (1, 3))
+    flush("captured supersampling: eager frames")
+    r.render(first)
+    other.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
+    want, again = other.render(third), other.render(first)
+    before = _device_bytes(gpu, r.p)
+    graph, exe = _captured(gpu, r, third)
+    assert _device_bytes(gpu, r.p) == before
+    for k in range(3):
+        flush(f"captured supersampling: replay {k}")
+        assert gpu.lib.hipGraphLaunch(exe, r.stream.handle) == 0
+        r.stream.synchronize()
+        assert_same(f"replay {k} colour", r.color.download(), want.color)
+        assert_same(f"replay {k} depth", r.depth.download(), want.depth)
+        assert_same(f"eager {k}", r.render(first).color, again.color)
+    got = r.render(third)
+    assert got.stats["splat_binned"] == 1, got.stats  # though too dense for the lists
+    assert _device_bytes(gpu, r.p) > before
+    assert_same("eager colour", got.color, want.color)
+    assert gpu.lib.hipGraphExecDestroy(exe) == 0 and gpu.lib.hipGraphDestroy(graph) == 0
+
+
 def test_forced_binning_allocates_once(gpu, small):
     scene = gpu.Scene(small)
     st = gpu.RenderSettings(640, 360, 1, 1, max_number_of_points=2_000_000)
