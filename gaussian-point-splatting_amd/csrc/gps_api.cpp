@@ -908,8 +908,9 @@ gps_status gps_pass_render(gps_pass* p, const gps_frame_params* fp, float* d_col
     // pass and next to nothing in the second.  Where the first may be too dense to
     // bin, points of few samples are not worth the lists in either (25M Gaussians
     // at 1080p, ss 2, us: lists, bounds and binned second pass 3076, without
-    // 2949).
-    const bool unculled = f.occl && !p->hiz_written && may_be_dense && f.Ki * f.spp < GPS_BIN_AUTO_SAMPLES;
+    // 2949).  A captured frame is replayed: all but once it is not the first.
+    const bool unculled = f.occl && !p->hiz_written && may_be_dense && f.Ki * f.spp < GPS_BIN_AUTO_SAMPLES &&
+                          !stream_captured(stream);
     BinGeom bg_geom;
     // the biased splat adds colours per sample and has only the
     // point-parallel form

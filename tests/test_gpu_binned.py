@@ -1,5 +1,7 @@
 """The binned splat at the edges of its lists, regions and jobs, bit for bit
 against the point-parallel splat (which the oracle's frames pin)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -228,3 +230,29 @@ def test_first_culled_frame_is_point_parallel(gpu):
         x, y = (r.render(f, [gpu.DBG_FRAMEBUFFER]) for r in (a, b))
         assert x.stats["splat_binned"] == (0 if k == 0 else 1), (k, x.stats)
         _same(gpu, x, y, f"frame {k}")
+
+
+def test_captured_first_culled_frame(gpu):
+    """... but not when the caller captures it: its replays are no first frames."""
+    arrays = H.scene(0x5EED0831, 7_400_000, dict(H.C1, half_extent=30.0, log_scale_mu=-4.0))
+    w, h = 1700, 956
+    st = gpu.RenderSettings(w, h, 1, 2, gaussians_per_block=256)
+    a, b = H.GpuRunner(arrays, st), H.GpuRunner(arrays, st)
+    b.p.set_splat_mode(gpu.Pass.SPLAT_POINT_PARALLEL)
+    f = gpu.frame_params((0.1, 3.0, -20.0), (0, 0, 0), (0, 1, 0), 45.0, w, h, ss=2, frame=1, occlusion=True,
+                         hierarchical=True, background=(0.2, 0.4, 0.6))
+    hip, stream = gpu.lib, a.stream.handle
+    graph, exe = C.c_void_p(), C.c_void_p()
+    flush("captured first culled frame")
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # thread local
+    a.p.render(f, a.color, a.depth, a.stream)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+    for k in range(3):
+        flush(f"captured first culled frame: replay {k}")
+        assert hip.hipGraphLaunch(exe, stream) == 0
+        a.stream.synchronize()
+        assert a.p.stats(a.stream)["splat_binned"] == 1
+        want = b.render(f)
+        assert np.array_equal(a.color.download(), want.color) and np.array_equal(a.depth.download(), want.depth), k
+    assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
