@@ -70,6 +70,30 @@ def test_estimate_follows_the_budget(gpu, small):
     assert by[3] - by[2] < 16 << 20  # the frame's own 16 points per pixel hold here
 
 
+@pytest.mark.parametrize("w,h,binnable,not_binnable", [
+    (3840, 2160, 3840 * 2160 // 4, 3840 * 2160 // 4 - 1),      # a Gaussian per 16 words
+    (1700, 956, 16 * 1700 * 956, 16 * 1700 * 956 + 1),         # 4 Gaussians per word
+    (1666, 944, None, 20_000_000),                             # 6 * 2^20 words
+    (1668, 944, 20_000_000, None),
+])
+def test_ends_of_the_rule_for_points_of_four_samples(gpu, w, h, binnable, not_binnable):
+    """The estimate counts a list exactly where such a frame may be binned
+    (the scenes hold no data)."""
+    st = gpu.RenderSettings(w, h, 1, 2, max_number_of_points=1 << 26, fully_disable_hierarchical_culling=True)
+    for n, can in ((binnable, True), (not_binnable, False)):
+        if n is None:
+            continue
+        handle = C.c_void_p()
+        assert gpu.lib.gps_scene_create_empty(n, 0, gpu.FORMAT_HALF_FP8, C.byref(handle)) == 0
+        settings = st.c()
+        bytes_ = int(gpu.lib.gps_pass_estimate_bytes(C.byref(settings), handle))
+        gpu.lib.gps_scene_destroy(handle)
+        fb = 2 * 8 * ((w * 2 + 63) // 64 * 64) * ((h * 2 + 63) // 64 * 64)
+        others = fb + 78 * n + 8 * w * h + (8 << 20)
+        print(f"{w}x{h} n {n}: {bytes_} bytes, {others} without lists", flush=True)
+        assert (bytes_ > others + 16 * n) if can else (bytes_ < others + 4 * n), (n, bytes_, others)
+
+
 def test_supersampling_that_can_be_binned_later(gpu, small):
     """A pass made for frames that cannot be binned takes its list with the
     framebuffers of the first frame that can."""
